@@ -215,6 +215,9 @@ static void fill_cw(CwArgs &a, const acx_grid *g)
         a.g3c = (1.0 - g->gamma_hi) * g->gamma_lo - 2.0 * a.g3s;
     }
     a.inv_g4 = 1.0 / g->gamma_hi;
+    a.k1a = (a.g3s - 11.0 / 60.0 + 1.0 / 60.0) * a.inv_g4;
+    a.k1w = (a.g3s - 11.0 / 60.0 + 1.0 / 10.0) * a.inv_g4;
+    a.k2 = a.g3s * a.inv_g4;
     a.nf = nonfinite_word_current();
 }
 

@@ -18,13 +18,14 @@
 //
 // Layout: a block covers BX x BY reconstruction columns, the outer ring being
 // the face-neighbour halo of the (BX-2) x (BY-2) output tile, and marches a
-// chunk of z-planes.  The block keeps the five planes m-2..m+2 of its
-// stencil region in an LDS ring (the next plane is loaded one iteration
-// ahead into registers and stored after the last read of the slot it
-// replaces).  x-neighbour face states and fluxes move by lane shuffles
-// inside a 32-lane row, y-neighbours through LDS, z-neighbours stay in
-// registers.  Selective mode (per-cell flags) replaces the full CWENO by
-// the linear 4th-order polynomial wherever the flag bit of a component is 0.
+// chunk of z-planes with the planes of its stencil region in an LDS ring (the
+// next plane is loaded one iteration ahead into registers and stored after
+// the last read of the slot it replaces).  x-neighbour face states move by
+// lane shuffles inside a 32-lane row, y-neighbours through LDS,
+// z-neighbours stay in registers.  k_cweno: the compensated FP32 stage, whose
+// selective mode (per-cell flags) replaces the full CWENO by the linear
+// 4th-order polynomial wherever the flag bit of a component is 0.
+// k_cweno64: the FP64 right-hand side and stages.
 #include <algorithm>
 
 #include "acx_device.h"
@@ -35,52 +36,41 @@ namespace acx {
 
 enum { EPI_RHS = 0, EPI_AXPY = 1, EPI_COMB = 2, EPI_F32C = 3 };
 
-// Face quantities of one component from its axis coefficients:
-// ACOUSTIC4 -> face-averaged values, WAVE2 -> h * face-averaged normal gradient.
-template <typename T, int SYS>
-__device__ __forceinline__ void face_q(T c0, const Axis3<T> &a, T (&fm)[3], T (&fp)[3])
+// Face-averaged values of one component from its axis coefficients.
+__device__ __forceinline__ void face_q(float c0, const Axis3<float> &a, float (&fm)[3], float (&fp)[3])
 {
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
-        if constexpr (SYS == ACX_ACOUSTIC4) {
-            const T even = c0 + a.c2[d] * T(1.0 / 6.0), odd = T(0.5) * a.c1[d] + a.c3[d] * T(1.0 / 20.0);
-            fm[d] = even - odd;
-            fp[d] = even + odd;
-        } else {
-            const T e = a.c1[d] + T(0.6) * a.c3[d];
-            fm[d] = e - a.c2[d];
-            fp[d] = e + a.c2[d];
-        }
+        const float even = c0 + a.c2[d] * float(1.0 / 6.0), odd = 0.5f * a.c1[d] + a.c3[d] * float(1.0 / 20.0);
+        fm[d] = even - odd;
+        fp[d] = even + odd;
     }
 }
 
-// Flux across a face normal to axis d from left (+face) and right (-face) states.
-template <typename T, int SYS, int NS>
-__device__ __forceinline__ void face_flux(int d, const T (&L)[NS], const T (&R)[NS], T K, T irho, T s, T (&F)[NS])
+// Flux across a face normal to axis d from left (+face) and right (-face)
+// states: 1/2 (F(Q_L) + F(Q_R) - s (Q_R - Q_L)), F_p = K u_n, F_un = p / rho0.
+__device__ __forceinline__ void face_flux(int d, const float (&L)[4], const float (&R)[4], float K, float irho, float s,
+                                          float (&F)[4])
 {
-    if constexpr (SYS == ACX_ACOUSTIC4) {
-        // 1/2 (F(Q_L) + F(Q_R) - s (Q_R - Q_L)), F_p = K u_n, F_un = p / rho0
 #pragma unroll
-        for (int v = 0; v < 4; ++v) F[v] = -s * (R[v] - L[v]);
-        F[0] += K * (L[1 + d] + R[1 + d]);
-        F[1 + d] += irho * (L[0] + R[0]);
+    for (int v = 0; v < 4; ++v) F[v] = -s * (R[v] - L[v]);
+    F[0] += K * (L[1 + d] + R[1 + d]);
+    F[1 + d] += irho * (L[0] + R[0]);
 #pragma unroll
-        for (int v = 0; v < 4; ++v) F[v] *= T(0.5);
-    } else {
-        F[0] = T(0.5) * (L[0] + R[0]);
-    }
+    for (int v = 0; v < 4; ++v) F[v] *= 0.5f;
 }
 
-// Shared-memory plan of one block (dynamic LDS):
+// FP32 compensated stage.  Shared-memory plan of one block (dynamic LDS):
 //   ring  [5][NS][BY+4][BX+4]  planes m-2 .. m+2 of the stencil region
 //   fym   [NS][BY][BX]         -y face state of each reconstruction column
 //   Fy    [NS][BY][BX]         flux through the +y face of each column
-template <typename T, int NS, int BX, int BY>
 struct CwLds {
+    static constexpr int BX = 32, BY = 16;   // reconstruction columns per block (output tile 30 x 14)
+    static constexpr int NS = 4;
     static constexpr int LX = BX + 4, LY = BY + 4;
     static constexpr int NR = 5;
     static constexpr size_t ring = (size_t)NR * NS * LY * LX;
-    static constexpr size_t bytes = (ring + 2ull * NS * BY * BX) * sizeof(T);
+    static constexpr size_t bytes = (ring + 2ull * NS * BY * BX) * sizeof(float);
 };
 
 // Waves per SIMD the register allocation aims for.  The selective patch
@@ -96,14 +86,13 @@ struct CwWaves {
 };
 
 // WALLS = false: every axis periodic (wrap-only index maps, no ghost signs).
-template <typename T, int SYS, int BX, int BY, int EPI, bool SEL, bool WALLS>
-__global__ void __launch_bounds__(BX *BY) __attribute__((amdgpu_waves_per_eu(CwWaves<SEL>::min_per_simd)))
+template <bool SEL, bool WALLS>
+__global__ void __launch_bounds__(CwLds::BX *CwLds::BY) __attribute__((amdgpu_waves_per_eu(CwWaves<SEL>::min_per_simd)))
 k_cweno(CwArgs p)
 {
-    constexpr int NV = SYS == ACX_ACOUSTIC4 ? 4 : 2;
-    constexpr int NS = SYS == ACX_ACOUSTIC4 ? 4 : 1;
-    constexpr int NT = BX * BY;
-    using L = CwLds<T, NS, BX, BY>;
+    using T = float;
+    using L = CwLds;
+    constexpr int NV = 4, NS = L::NS, BX = L::BX, BY = L::BY, NT = BX * BY;
     constexpr int LX = L::LX, LY = L::LY;
     static_assert(BX == 32, "x exchange uses 32-lane row shuffles");
     extern __shared__ __align__(16) unsigned char smem[];
@@ -113,7 +102,6 @@ k_cweno(CwArgs p)
 
     const T *__restrict__ Q = static_cast<const T *>(p.q);
     const T *__restrict__ D = static_cast<const T *>(p.d);
-    const T *__restrict__ U0 = static_cast<const T *>(p.u0);
     const T *__restrict__ LO = static_cast<const T *>(p.lo);
     T *__restrict__ OUT = static_cast<T *>(p.out);
     T *__restrict__ OUT2 = static_cast<T *>(p.out2);
@@ -160,7 +148,7 @@ k_cweno(CwArgs p)
                 rcol[r] = (uint32_t)(map_axis(gy0 - 2 + ly, ny, ky, rsy[r]) * nx + map_axis(gx0 - 2 + lx, nx, kx, rsx[r]));
             }
         }
-        const bool has_d = (EPI == EPI_F32C) && D != nullptr;
+        const bool has_d = D != nullptr;
         auto zoff = [&](int z, float &s) -> size_t {
             s = 1.f;
             return (size_t)map_axis(z, nz, kz, s) * plane;
@@ -213,7 +201,6 @@ k_cweno(CwArgs p)
         T zp_prev[NS], Fz_prev[NS], dxy_prev[NS];
 #pragma unroll
         for (int v = 0; v < NS; ++v) { zp_prev[v] = T(0); Fz_prev[v] = T(0); dxy_prev[v] = T(0); }
-        T vcen_prev = T(0);
         const int lx = tx + 2, ly = ty + 2;
 
         uint8_t fl_next = 0xff;
@@ -246,24 +233,12 @@ k_cweno(CwArgs p)
             const size_t cell = (size_t)(m - 1) * plane + ocol;
             Cell<T, NV> e0, e1, e2;
             if (fin) {
-                // COMB: U0 is loaded at the epilogue instead (8 fewer live VGPRs
-                // through the weights, where the registers spill)
-                if constexpr (EPI == EPI_F32C) {
-                    if (has_d) e0 = load_cell<T, NV>(D, cell);
-                    if (p.final_stage) {
-                        e1 = load_cell<T, NV>(LO, cell);
-                        e2 = load_cell<T, NV>(Q, cell);
-                    }
+                if (has_d) e0 = load_cell<T, NV>(D, cell);
+                if (p.final_stage) {
+                    e1 = load_cell<T, NV>(LO, cell);
+                    e2 = load_cell<T, NV>(Q, cell);
                 }
             }
-            T vcen = T(0);
-            if constexpr (SYS == ACX_WAVE2) {
-                float s;
-                const size_t idx = (zoff(m, s) + ocol) * NV + 1;
-                vcen = Q[idx];
-                if constexpr (EPI == EPI_F32C) { if (D) vcen += D[idx]; }
-            }
-
             const int sm2 = slot(m - 2), s0 = slot(m - 1), s1 = slot(m), s2 = slot(m + 1), sp2 = slot(m + 2);
             T fpx[NS], fmx[NS], fpy[NS], fmz[NS], fpz[NS];
 #pragma unroll
@@ -323,7 +298,7 @@ k_cweno(CwArgs p)
                     axis_linear(get(9), get(10), get(0), get(11), get(12), ax.c1[2], ax.c2[2], ax.c3[2]);
                 }
                 T m3[3], p3[3];
-                face_q<T, SYS>(get(0), ax, m3, p3);
+                face_q(get(0), ax, m3, p3);
                 fmx[v] = m3[0]; fpx[v] = p3[0];
                 s_fym[v][ty][tx] = m3[1];
                 fpy[v] = p3[1];
@@ -340,10 +315,10 @@ k_cweno(CwArgs p)
                 T Lf[NS], Rf[NS];
 #pragma unroll
                 for (int v = 0; v < NS; ++v) { Lf[v] = fpx[v]; Rf[v] = __shfl_down(fmx[v], 1, 32); }
-                face_flux<T, SYS, NS>(0, Lf, Rf, K, irho, sL, Fx);
+                face_flux(0, Lf, Rf, K, irho, sL, Fx);
 #pragma unroll
                 for (int v = 0; v < NS; ++v) { Lf[v] = fpy[v]; Rf[v] = ty + 1 < BY ? s_fym[v][ty + 1][tx] : T(0); }
-                face_flux<T, SYS, NS>(1, Lf, Rf, K, irho, sL, Fy);
+                face_flux(1, Lf, Rf, K, irho, sL, Fy);
             }
 #pragma unroll
             for (int v = 0; v < NS; ++v) s_Fy[v][ty][tx] = Fy[v];
@@ -361,53 +336,27 @@ k_cweno(CwArgs p)
                 T Fz[NS], Lf[NS], Rf[NS];
 #pragma unroll
                 for (int v = 0; v < NS; ++v) { Lf[v] = zp_prev[v]; Rf[v] = fmz[v]; }
-                face_flux<T, SYS, NS>(2, Lf, Rf, K, irho, sL, Fz);
+                face_flux(2, Lf, Rf, K, irho, sL, Fz);
                 if (fin) {
                     Cell<T, NV> r;
-                    if constexpr (SYS == ACX_ACOUSTIC4) {
-                        const T ih = T(p.inv_h);
+                    const T ih = T(p.inv_h);
 #pragma unroll
-                        for (int v = 0; v < 4; ++v) r.v[v] = -ih * (dxy_prev[v] + (Fz[v] - Fz_prev[v]));
-                    } else {
-                        r.v[0] = vcen_prev;
-                        r.v[1] = T(p.c2) * (dxy_prev[0] + (Fz[0] - Fz_prev[0]));
-                    }
+                    for (int v = 0; v < 4; ++v) r.v[v] = -ih * (dxy_prev[v] + (Fz[v] - Fz_prev[v]));
                     Cell<T, NV> o;
-                    if constexpr (EPI == EPI_RHS) {
-                        o = r;
-                    } else if constexpr (EPI == EPI_AXPY || EPI == EPI_COMB) {
-                        // Q of the own (in-domain) cell of plane m-1 is still in the ring
-                        Cell<T, NV> q;
-                        if constexpr (NS == NV) {
 #pragma unroll
-                            for (int v = 0; v < NV; ++v) q.v[v] = ring[s0][v][ly][lx];
-                        } else {
-                            q = load_cell<T, NV>(Q, cell);
+                    for (int v = 0; v < NV; ++v) o.v[v] = (has_d ? T(p.b) * e0.v[v] : T(0)) + T(p.c) * r.v[v];
+                    if (p.final_stage) {
+                        Cell<T, NV> nh, nl;
+#pragma unroll
+                        for (int v = 0; v < NV; ++v) {
+                            float t = e1.v[v] + o.v[v];
+                            float sm, er;
+                            two_sum(e2.v[v], t, sm, er);
+                            nh.v[v] = sm;
+                            nl.v[v] = er;
                         }
-                        if constexpr (EPI == EPI_AXPY) {
-#pragma unroll
-                            for (int v = 0; v < NV; ++v) o.v[v] = q.v[v] + T(p.c) * r.v[v];
-                        } else {
-                            e0 = load_cell<T, NV>(U0, cell);
-#pragma unroll
-                            for (int v = 0; v < NV; ++v) o.v[v] = T(p.a) * e0.v[v] + T(p.b) * q.v[v] + T(p.c) * r.v[v];
-                        }
-                    } else {
-#pragma unroll
-                        for (int v = 0; v < NV; ++v) o.v[v] = (has_d ? T(p.b) * e0.v[v] : T(0)) + T(p.c) * r.v[v];
-                        if (p.final_stage) {
-                            Cell<T, NV> nh, nl;
-#pragma unroll
-                            for (int v = 0; v < NV; ++v) {
-                                float t = (float)e1.v[v] + (float)o.v[v];
-                                float sm, er;
-                                two_sum((float)e2.v[v], t, sm, er);
-                                nh.v[v] = sm;
-                                nl.v[v] = er;
-                            }
-                            store_cell<T, NV>(OUT2, cell, nl);
-                            o = nh;
-                        }
+                        store_cell<T, NV>(OUT2, cell, nl);
+                        o = nh;
                     }
                     if (p.nf) finite_acc<T, NV>(nfbad, o);
                     store_cell<T, NV>(OUT, cell, o);
@@ -417,7 +366,6 @@ k_cweno(CwArgs p)
             }
 #pragma unroll
             for (int v = 0; v < NS; ++v) { zp_prev[v] = fpz[v]; dxy_prev[v] = dxy[v]; }
-            vcen_prev = vcen;
         }
         if constexpr (SEL) {
             __syncthreads();   // the next tile's prologue rewrites the ring
@@ -427,9 +375,319 @@ k_cweno(CwArgs p)
     watch_flush(p.nf, nfbad);
 }
 
+// FP64 stage kernel, bound by FP64 issue (cweno_faces64: about 265 of the 300
+// FP64 instructions per cell and component).  A thread reconstructs at most
+// two of the components: an ACOUSTIC4 block is 32 x 12 columns times two halves
+// (waves 0-5 p and u, waves 6-11 v and w), a WAVE2 block 32 x 16 columns on
+// the one component.  What decided the shape, measured on the 256^3 ACOUSTIC4
+// step (8.24 ms with cweno_weights + cweno_combine, four components per
+// thread on 32 x 16 columns): the new arithmetic in the old kernel 5.38 ms (256
+// VGPRs, 2 waves per SIMD, 24 spilled); two components per thread on 32 x 16
+// columns 8.07 ms (128 VGPRs for 4 waves per SIMD, 35 spilled: the scratch
+// traffic leaves the L1); on 32 x 12 columns 4.64 ms (3 waves per SIMD, 167
+// VGPRs, no spills), although the smaller tile recomputes more of its ring
+// (outputs are 78 % of the reconstructed columns instead of 82 %).  The WAVE2
+// RHS at 70 x 45 x 61 with walls: 31.8 -> 22.0 us.
+//
+// The LDS ring holds four planes, m-1 .. m+2 (each thread keeps its own
+// columns' m-1 and m-2 in registers); the plane m+3 is requested at the start
+// of iteration m and goes into the slot of plane m-1 after it.  x-neighbour
+// face states move by lane shuffles inside a 32-lane row; y-neighbour states
+// and, across the two halves of the block, the coupled states (p with v at
+// y faces, p with w at z faces; p with u at x faces are in one thread) go
+// through LDS.
+template <int SYS>
+struct Cw64 {
+    static constexpr int NS = SYS == ACX_ACOUSTIC4 ? 4 : 1;   // reconstructed components
+    static constexpr int NC = SYS == ACX_ACOUSTIC4 ? 2 : 1;   // of them per thread
+    static constexpr int NV = SYS == ACX_ACOUSTIC4 ? 4 : 2;   // components in memory
+    static constexpr int BX = 32, BY = SYS == ACX_ACOUSTIC4 ? 12 : 16, NCOL = BX * BY;
+    static constexpr int NT = NCOL * (NS / NC);
+    static constexpr int WPE = SYS == ACX_ACOUSTIC4 ? 3 : 4;  // waves per SIMD
+    static constexpr int LX = BX + 4, LY = BY + 4, NREG = LX * LY;
+    static constexpr int CS = NREG + 4;                       // doubles per component of a slot
+    static constexpr int NR = 4;
+    static constexpr int SLOT = NS * CS;
+    static constexpr int EX = NS * 2 * NCOL;                  // -y and +y face states
+    static constexpr int EZ = SYS == ACX_ACOUSTIC4 ? 2 * NCOL : 0;   // p and w sums at the lower z face
+    static constexpr size_t bytes = (size_t)(NR * SLOT + EX + EZ) * sizeof(double);
+    static constexpr int NLD = NREG * NV / 2;                 // 16-byte loads of one plane
+    static constexpr int PER = (NLD + NT - 1) / NT;
+};
+
+template <int SYS, int EPI, bool WALLS>
+__global__ void __launch_bounds__(Cw64<SYS>::NT) __attribute__((amdgpu_waves_per_eu(Cw64<SYS>::WPE)))
+k_cweno64(CwArgs p)
+{
+    using L = Cw64<SYS>;
+    constexpr int NC = L::NC, NV = L::NV, BX = L::BX, BY = L::BY, LX = L::LX, NCOL = L::NCOL, PER = L::PER;
+    constexpr bool AC = SYS == ACX_ACOUSTIC4;
+    extern __shared__ __align__(16) unsigned char smem[];
+    double *const ring = reinterpret_cast<double *>(smem);
+    double *const s_y = ring + L::NR * L::SLOT;   // [component][-y, +y][column]
+    double *const s_z = s_y + L::EX;              // [p, w][column]
+
+    const double *__restrict__ Q = static_cast<const double *>(p.q);
+    const double *__restrict__ U0 = static_cast<const double *>(p.u0);
+    double *__restrict__ OUT = static_cast<double *>(p.out);
+    const int nx = p.nx, ny = p.ny, nz = p.nz;
+    const size_t plane = (size_t)nx * ny;
+    const int kx = WALLS ? p.bc[0] : 0, ky = WALLS ? p.bc[1] : 0, kz = WALLS ? p.bc[2] : 0;
+
+    const int tid = threadIdx.x, colid = tid % NCOL, tx = colid % BX, ty = colid / BX;
+    const int half = AC ? __builtin_amdgcn_readfirstlane(tid / NCOL) : 0, v0 = half * NC;
+    const int tile = xcd_logical_tile(blockIdx.x, gridDim.x);
+    const int gx0 = (tile % p.ntx) * (BX - 2) - 1, gy0 = ((tile / p.ntx) % p.nty) * (BY - 2) - 1;
+    const int gx = gx0 + tx, gy = gy0 + ty;
+    const int zb = (tile / (p.ntx * p.nty)) * p.zc, ze = min(zb + p.zc, nz);
+    const bool interior = tx >= 1 && tx <= BX - 2 && ty >= 1 && ty <= BY - 2 && gx < nx && gy < ny;
+    float sx0 = 1.f, sy0 = 1.f;
+    const uint32_t ocol = (uint32_t)(map_axis(gy, ny, ky, sy0) * nx + map_axis(gx, nx, kx, sx0));
+
+    // this thread's 16-byte pieces (component pairs) of a plane's region
+    uint32_t rcol[PER];
+    float rs[PER][2];        // ghost signs of the pair from the x and y axes
+    int rdst[PER];           // ring index of its first component
+#pragma unroll
+    for (int r = 0; r < PER; ++r) {
+        const int idx = tid + r * L::NT, cell = idx / (NV / 2), part = idx % (NV / 2);
+        rcol[r] = 0;
+        rdst[r] = -1;
+        rs[r][0] = rs[r][1] = 1.f;
+        if (idx < L::NLD) {
+            const int lx = cell % LX, ly = cell / LX;
+            float sx = 1.f, sy = 1.f;
+            const int c = map_axis(gy0 - 2 + ly, ny, ky, sy) * nx + map_axis(gx0 - 2 + lx, nx, kx, sx);
+            rcol[r] = (uint32_t)c * (NV / 2) + part;
+            rdst[r] = (AC ? 2 * part * L::CS : 0) + cell;
+            if constexpr (WALLS) {
+                if (AC) {
+                    rs[r][0] = part == 0 ? 1.f : sy;   // p, v
+                    rs[r][1] = part == 0 ? sx : 1.f;   // u, w
+                } else {
+                    rs[r][0] = sx * sy;
+                }
+            }
+        }
+    }
+    auto load_plane = [&](int z, acx_dbl2 (&buf)[PER], float &sz) {
+        sz = 1.f;
+        const acx_dbl2 *P = reinterpret_cast<const acx_dbl2 *>(Q) + (size_t)map_axis(z, nz, kz, sz) * plane * (NV / 2);
+#pragma unroll
+        for (int r = 0; r < PER; ++r)
+            if (rdst[r] >= 0) buf[r] = P[rcol[r]];
+    };
+    auto store_plane = [&](int slot, const acx_dbl2 (&buf)[PER], float sz) {
+        double *d = ring + slot * L::SLOT;
+#pragma unroll
+        for (int r = 0; r < PER; ++r)
+            if (rdst[r] >= 0) {
+                double a = buf[r].x, b = buf[r].y;
+                if constexpr (WALLS) {
+                    a *= rs[r][0];
+                    b *= rs[r][1];
+                    if (!AC) a *= sz;
+                    else if (rdst[r] >= 2 * L::CS) b *= sz;   // w
+                }
+                d[rdst[r]] = a;
+                if constexpr (AC) d[rdst[r] + L::CS] = b;
+            }
+    };
+    const int cen = (ty + 2) * LX + tx + 2 + v0 * L::CS;   // own column, first own component
+
+    // prologue: planes zb-3 .. zb+1 through the ring; zb-3 only feeds the
+    // column values of iteration zb-1, so its slot is reused for zb+1
+    double um1[NC], um2[NC];
+    {
+        acx_dbl2 b0[PER], b1[PER], b2[PER];
+        float s0, s1, s2;
+        load_plane(zb - 3, b0, s0);
+        load_plane(zb - 2, b1, s1);
+        load_plane(zb - 1, b2, s2);
+        store_plane(3, b0, s0);
+        store_plane(0, b1, s1);
+        store_plane(1, b2, s2);
+        load_plane(zb, b1, s1);
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < NC; ++k) {
+            um2[k] = ring[3 * L::SLOT + cen + k * L::CS];
+            um1[k] = ring[cen + k * L::CS];
+        }
+        load_plane(zb + 1, b0, s0);
+        __syncthreads();
+        store_plane(2, b1, s1);
+        store_plane(3, b0, s0);
+        __syncthreads();
+    }
+
+    const double K = p.K, irho = p.invrho, sL = p.s;
+    double zp_prev[NC], Fz_prev[NC], dxy_prev[NC];   // of plane m-1: +z state, flux below, in-plane divergence
+#pragma unroll
+    for (int k = 0; k < NC; ++k) zp_prev[k] = Fz_prev[k] = dxy_prev[k] = 0.0;
+    double vcen = 0.0, vcen_prev = 0.0;
+    bool nfbad = false;
+    int slot = 0;   // of plane m-1
+    for (int m = zb - 1; m <= ze; ++m) {
+        acx_dbl2 nxt[PER];
+        float nsz = 1.f;
+        const bool pf = m + 3 <= ze + 2;
+        if (pf) load_plane(m + 3, nxt, nsz);
+        if constexpr (!AC) {
+            float s = 1.f;
+            vcen = Q[((size_t)map_axis(m, nz, kz, s) * plane + ocol) * NV + 1];
+        }
+        const double *R0 = ring + slot * L::SLOT + cen, *R1 = ring + ((slot + 1) & 3) * L::SLOT + cen;
+        const double *R2 = ring + ((slot + 2) & 3) * L::SLOT + cen, *R3 = ring + ((slot + 3) & 3) * L::SLOT + cen;
+        double fmx[NC], fpx[NC], F[NC];   // F: twice the flux at the face between planes m-1 and m
+#pragma unroll
+        for (int k = 0; k < NC; ++k) {
+            const int o = k * L::CS;
+            const double u0 = R1[o];
+            // stencil slot q (order of cweno_weights)
+            auto get = [&](int q) -> double {
+                switch (q) {
+                case 0: return u0;
+                case 1: return R1[o - 2];
+                case 2: return R1[o - 1];
+                case 3: return R1[o + 1];
+                case 4: return R1[o + 2];
+                case 5: return R1[o - 2 * LX];
+                case 6: return R1[o - LX];
+                case 7: return R1[o + LX];
+                case 8: return R1[o + 2 * LX];
+                case 9: return um2[k];
+                case 10: return um1[k];
+                case 11: return R2[o];
+                case 12: return R3[o];
+                case 13: return R1[o + LX + 1];   // xy: ++ +- -+ --
+                case 14: return R1[o - LX + 1];
+                case 15: return R1[o + LX - 1];
+                case 16: return R1[o - LX - 1];
+                case 17: return R2[o + LX];       // yz (y,z): ++ +- -+ --
+                case 18: return R0[o + LX];
+                case 19: return R2[o - LX];
+                case 20: return R0[o - LX];
+                case 21: return R2[o + 1];        // zx (z,x): ++ +- -+ --
+                case 22: return R2[o - 1];
+                case 23: return R0[o + 1];
+                case 24: return R0[o - 1];
+                case 25: return R2[o + LX + 1];   // corners (x,y,z): +++ -++ +-+ ++- --+ -+- +-- ---
+                case 26: return R2[o + LX - 1];
+                case 27: return R2[o - LX + 1];
+                case 28: return R0[o + LX + 1];
+                case 29: return R2[o - LX - 1];
+                case 30: return R0[o + LX - 1];
+                case 31: return R0[o - LX + 1];
+                default: return R0[o - LX - 1];
+                }
+            };
+            double fm[3], fp[3];
+            cweno_faces64<SYS>(get, p, fm, fp);
+            fmx[k] = fm[0]; fpx[k] = fp[0];
+            F[k] = AC ? -sL * (fm[2] - zp_prev[k]) : fm[2] + zp_prev[k];
+            if constexpr (AC) {
+                if (k == half) s_z[half * NCOL + colid] = fm[2] + zp_prev[k];   // p or w
+            }
+            zp_prev[k] = fp[2];
+            s_y[((v0 + k) * 2 + 0) * NCOL + colid] = fm[1];
+            s_y[((v0 + k) * 2 + 1) * NCOL + colid] = fp[1];
+            um2[k] = um1[k];
+            um1[k] = u0;
+            asm volatile("" ::: "memory");   // one component's stencil live at a time
+        }
+
+        // x: twice the flux at the +x face, minus the one at the -x face
+        double d[NC];
+        {
+            double G[NC];
+#pragma unroll
+            for (int k = 0; k < NC; ++k) {
+                const double R = __shfl_down(fmx[k], 1, 32);
+                if constexpr (AC) {
+                    G[k] = -sL * (R - fpx[k]);
+                    fmx[k] = R + fpx[k];
+                } else {
+                    G[k] = R + fpx[k];
+                }
+            }
+            if constexpr (AC) {
+                if (half == 0) {
+                    G[0] += K * fmx[1];
+                    G[1] += irho * fmx[0];
+                }
+            }
+#pragma unroll
+            for (int k = 0; k < NC; ++k) d[k] = G[k] - __shfl_up(G[k], 1, 32);
+        }
+        __syncthreads();   // B1: exchanged states visible; every read of plane m-1 is done
+
+        if (pf) store_plane(slot, nxt, nsz);   // into the slot of plane m-1
+        // y: both faces from the neighbours' states
+        {
+            const int up = ty + 1 < BY ? colid + BX : colid, dn = ty > 0 ? colid - BX : colid;
+#pragma unroll
+            for (int k = 0; k < NC; ++k) {
+                const double *e = s_y + (v0 + k) * 2 * NCOL;
+                const double R = e[up], Lm = e[NCOL + dn], lo = e[colid], hi = e[NCOL + colid];
+                if constexpr (AC) d[k] -= sL * ((R - hi) - (lo - Lm));
+                else d[k] += (R + hi) - (lo + Lm);
+            }
+            if constexpr (AC) {
+                // p takes K (v_L + v_R), v takes (p_L + p_R) / rho0: component 0 of either half
+                const double *e = s_y + (half ? 0 : 2) * 2 * NCOL;
+                d[0] += (half ? irho : K) * ((e[up] + e[NCOL + colid]) - (e[colid] + e[NCOL + dn]));
+            }
+        }
+        // z: the coupled part
+        if constexpr (AC) {
+            const double o = s_z[(1 - half) * NCOL + colid];
+            if (half == 0) F[0] += K * o;
+            else F[1] += irho * o;
+        }
+        if (m >= zb + 1 && interior) {
+            const size_t cell = (size_t)(m - 1) * plane + ocol;
+            double *oc = OUT + cell * NV;
+            acx_dbl2 r, q;
+            if constexpr (AC) {
+                const double ih = -0.5 * p.inv_h;
+                r.x = ih * (dxy_prev[0] + (F[0] - Fz_prev[0]));
+                r.y = ih * (dxy_prev[1] + (F[1] - Fz_prev[1]));
+                q.x = um2[0];   // the column's plane m-1
+                q.y = um2[1];
+            } else {
+                r.x = vcen_prev;
+                r.y = 0.5 * p.c2 * (dxy_prev[0] + (F[0] - Fz_prev[0]));
+                q.x = um2[0];
+                q.y = vcen_prev;
+            }
+            acx_dbl2 o;
+            if constexpr (EPI == EPI_RHS) {
+                o = r;
+            } else if constexpr (EPI == EPI_AXPY) {
+                o = q + p.c * r;
+            } else {
+                const acx_dbl2 u = *reinterpret_cast<const acx_dbl2 *>(U0 + cell * NV + v0);
+                o = p.a * u + p.b * q + p.c * r;
+            }
+            nfbad |= !__builtin_isfinite(o.x) || !__builtin_isfinite(o.y);
+            *reinterpret_cast<acx_dbl2 *>(oc + v0) = o;
+        }
+#pragma unroll
+        for (int k = 0; k < NC; ++k) {
+            dxy_prev[k] = d[k];
+            Fz_prev[k] = F[k];
+        }
+        vcen_prev = vcen;
+        slot = (slot + 1) & 3;
+        __syncthreads();   // B2: plane m+3 visible; the exchanged states are read
+    }
+    watch_flush(p.nf, nfbad);
+}
+
 // ---------------------------------------------------------------------------
 
-constexpr int CW_BX = 32, CW_BY = 16;   // reconstruction columns per block (output tile 30 x 14)
+constexpr int CW_BX = CwLds::BX, CW_BY = CwLds::BY;
 
 // One block per column of up to TM_ZT CWENO tiles along z: a tile is marked
 // when a cell of it, or a face neighbour of one (a cell of the one-cell ring
@@ -522,8 +780,8 @@ int launch_cweno_tilemask(const CwArgs &a, const uint8_t *flags, uint8_t *mask, 
     return hip_check(hipGetLastError(), "tile list launch");
 }
 
-template <typename T, int SYS, int EPI, bool SEL, bool WALLS>
-static int launch_cw_tw(const CwArgs &a, hipStream_t s)
+template <bool SEL, bool WALLS>
+static int launch_cw32_w(const CwArgs &a, hipStream_t s)
 {
     constexpr int BX = CW_BX, BY = CW_BY;
     CwArgs b = a;
@@ -531,15 +789,13 @@ static int launch_cw_tw(const CwArgs &a, hipStream_t s)
     b.nty = (a.ny + BY - 3) / (BY - 2);
     if (b.zc <= 0) {
         // round model with a start of 4 planes (the recomputed ring planes and
-        // the prologue).  Measured (FP64, gamma = 0.85): 64 planes at 256^3
-        // (+3.7 % over 32; 96 leaves a one-workgroup last round), 96 at 384^3
-        // (+2-4 % over 64; 128 -12 %).
+        // the prologue)
         static int per_cu = 0;
         if (!per_cu) {
             int n = 0;
             if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                    &n, reinterpret_cast<const void *>(&k_cweno<T, SYS, BX, BY, EPI, SEL, WALLS>), BX * BY,
-                    CwLds<T, SYS == ACX_ACOUSTIC4 ? 4 : 1, BX, BY>::bytes) != hipSuccess || n <= 0)
+                    &n, reinterpret_cast<const void *>(&k_cweno<SEL, WALLS>), BX * BY,
+                    CwLds::bytes) != hipSuccess || n <= 0)
                 n = 1;
             per_cu = n;
         }
@@ -553,18 +809,17 @@ static int launch_cw_tw(const CwArgs &a, hipStream_t s)
         if (!per_cu_sel) {
             int n = 0;
             if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                    &n, reinterpret_cast<const void *>(&k_cweno<T, SYS, BX, BY, EPI, SEL, WALLS>), BX * BY,
-                    CwLds<T, SYS == ACX_ACOUSTIC4 ? 4 : 1, BX, BY>::bytes) != hipSuccess || n <= 0)
+                    &n, reinterpret_cast<const void *>(&k_cweno<SEL, WALLS>), BX * BY,
+                    CwLds::bytes) != hipSuccess || n <= 0)
                 n = 1;
             per_cu_sel = n;
         }
         blocks = std::min(blocks, (size_t)device_cus() * per_cu_sel);
     }
-    constexpr int NS = SYS == ACX_ACOUSTIC4 ? 4 : 1;
-    constexpr size_t lds = CwLds<T, NS, BX, BY>::bytes;
+    constexpr size_t lds = CwLds::bytes;
     static bool attr_set = false;
     if (!attr_set) {
-        int rc = hip_check(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_cweno<T, SYS, BX, BY, EPI, SEL, WALLS>),
+        int rc = hip_check(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_cweno<SEL, WALLS>),
                                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds),
                            "k_cweno LDS attribute");
         if (rc) return rc;
@@ -572,16 +827,54 @@ static int launch_cw_tw(const CwArgs &a, hipStream_t s)
     }
     dim3 blk(BX, BY, 1);
     dim3 grd((unsigned)blocks, 1, 1);
-    hipLaunchKernelGGL((k_cweno<T, SYS, BX, BY, EPI, SEL, WALLS>), grd, blk, lds, s, b);
+    hipLaunchKernelGGL((k_cweno<SEL, WALLS>), grd, blk, lds, s, b);
     return hip_check(hipGetLastError(), "k_cweno launch");
 }
 
-template <typename T, int SYS, int EPI, bool SEL>
-static int launch_cw_t(const CwArgs &a, hipStream_t s)
+template <int SYS, int EPI, bool WALLS>
+static int launch_cw64(const CwArgs &a, hipStream_t s)
+{
+    using L = Cw64<SYS>;
+    const void *fn = reinterpret_cast<const void *>(&k_cweno64<SYS, EPI, WALLS>);
+    static bool attr_set = false;
+    if (!attr_set) {
+        int rc = hip_check(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)L::bytes),
+                           "k_cweno64 LDS attribute");
+        if (rc) return rc;
+        attr_set = true;
+    }
+    CwArgs b = a;
+    b.ntx = (a.nx + L::BX - 3) / (L::BX - 2);
+    b.nty = (a.ny + L::BY - 3) / (L::BY - 2);
+    if (b.zc <= 0) {
+        static int per_cu = 0;
+        if (!per_cu) {
+            int n = 0;
+            if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, fn, L::NT, L::bytes) != hipSuccess || n <= 0) n = 1;
+            per_cu = n;
+        }
+        b.zc = auto_zc(b.ntx, b.nty, a.nz, device_cus() * per_cu, 4);
+    }
+    b.ntz = (a.nz + b.zc - 1) / b.zc;
+    const size_t blocks = (size_t)b.ntx * b.nty * b.ntz;
+    hipLaunchKernelGGL((k_cweno64<SYS, EPI, WALLS>), dim3((unsigned)blocks), dim3(L::NT), L::bytes, s, b);
+    return hip_check(hipGetLastError(), "k_cweno64 launch");
+}
+
+template <int SYS, int EPI>
+static int launch_cw64_e(const CwArgs &a, hipStream_t s)
 {
     if (a.bc[0] != ACX_PERIODIC || a.bc[1] != ACX_PERIODIC || a.bc[2] != ACX_PERIODIC)
-        return launch_cw_tw<T, SYS, EPI, SEL, true>(a, s);
-    return launch_cw_tw<T, SYS, EPI, SEL, false>(a, s);
+        return launch_cw64<SYS, EPI, true>(a, s);
+    return launch_cw64<SYS, EPI, false>(a, s);
+}
+
+template <bool SEL>
+static int launch_cw32(const CwArgs &a, hipStream_t s)
+{
+    if (a.bc[0] != ACX_PERIODIC || a.bc[1] != ACX_PERIODIC || a.bc[2] != ACX_PERIODIC)
+        return launch_cw32_w<SEL, true>(a, s);
+    return launch_cw32_w<SEL, false>(a, s);
 }
 
 int launch_cweno(const CwArgs &a, int sys, int epi, bool fp32, bool selective, hipStream_t s)
@@ -589,21 +882,20 @@ int launch_cweno(const CwArgs &a, int sys, int epi, bool fp32, bool selective, h
     if (fp32) {
         if (epi != EPI_F32C || sys != ACX_ACOUSTIC4)
             return set_error(ACX_EUNSUPPORTED, "fp32 cweno kernel: compensated ACOUSTIC4 stage only");
-        return selective ? launch_cw_t<float, ACX_ACOUSTIC4, EPI_F32C, true>(a, s)
-                         : launch_cw_t<float, ACX_ACOUSTIC4, EPI_F32C, false>(a, s);
+        return selective ? launch_cw32<true>(a, s) : launch_cw32<false>(a, s);
     }
     if (selective) return set_error(ACX_EUNSUPPORTED, "fp64 cweno kernel: selective mode not built");
     if (sys == ACX_ACOUSTIC4) {
         switch (epi) {
-        case EPI_RHS: return launch_cw_t<double, ACX_ACOUSTIC4, EPI_RHS, false>(a, s);
-        case EPI_AXPY: return launch_cw_t<double, ACX_ACOUSTIC4, EPI_AXPY, false>(a, s);
-        case EPI_COMB: return launch_cw_t<double, ACX_ACOUSTIC4, EPI_COMB, false>(a, s);
+        case EPI_RHS: return launch_cw64_e<ACX_ACOUSTIC4, EPI_RHS>(a, s);
+        case EPI_AXPY: return launch_cw64_e<ACX_ACOUSTIC4, EPI_AXPY>(a, s);
+        case EPI_COMB: return launch_cw64_e<ACX_ACOUSTIC4, EPI_COMB>(a, s);
         }
     } else {
         switch (epi) {
-        case EPI_RHS: return launch_cw_t<double, ACX_WAVE2, EPI_RHS, false>(a, s);
-        case EPI_AXPY: return launch_cw_t<double, ACX_WAVE2, EPI_AXPY, false>(a, s);
-        case EPI_COMB: return launch_cw_t<double, ACX_WAVE2, EPI_COMB, false>(a, s);
+        case EPI_RHS: return launch_cw64_e<ACX_WAVE2, EPI_RHS>(a, s);
+        case EPI_AXPY: return launch_cw64_e<ACX_WAVE2, EPI_AXPY>(a, s);
+        case EPI_COMB: return launch_cw64_e<ACX_WAVE2, EPI_COMB>(a, s);
         }
     }
     return set_error(ACX_EUNSUPPORTED, "cweno kernel: unsupported epilogue");

@@ -27,6 +27,15 @@ __device__ __forceinline__ double rcp64(double t)
     return fma(r, e, r);
 }
 
+// 1/t in FP64 to the last place or so: the estimate r = (1 - e)/t with
+// |e| <= 2^-24.4 refined by r (1 + e + e^2), which leaves e^3.
+__device__ __forceinline__ double rcp64_full(double t)
+{
+    const double r = __builtin_amdgcn_rcp(t);
+    const double e = fma(-t, r, 1.0);
+    return fma(r, fma(e, e, e), r);
+}
+
 template <typename T>
 __device__ __forceinline__ T pos_pow4_inv(T g, T t)
 {
@@ -225,6 +234,137 @@ __device__ __forceinline__ void cweno_axes_lds(Get get, const CwArgs &p, Axis3<T
     asm volatile("" ::: "memory");
     cweno_combine<T>(get(0), get(1), get(2), get(3), get(4), get(5), get(6), get(7), get(8), get(9), get(10),
                      get(11), get(12), wt, w3, p, o);
+}
+
+// FP64 CWENO4 of one cell and component straight to its six face quantities
+// (ACOUSTIC4: face-averaged values; WAVE2: h times the face-averaged normal
+// gradients), the same scheme as cweno_weights + cweno_combine in far fewer
+// operations.  The stage kernel is bound by FP64 issue, so the operation
+// count is what it costs: about 240 FP64 instructions per cell and component,
+// 3 of them reciprocals, against 515 with 9.  get(q): stencil slots of
+// cweno_weights.  The memory clobbers keep one group of LDS values live at a
+// time.
+//
+// Per axis, from the first differences e1 .. e4 of m2, m1, u0, p1, p2:
+//   A, B, C = e4-e3, e3-e2, e2-e1 (second), a, c = A-B, B-C (third),
+//   S = e2+e3, T = a+c, F = a-c (fourth)
+// and the indicators are formed times 4 (with 4 eps; the weights are ratios):
+//   central       4(cx^2 + 13/3 uxx^2)     = S^2 + 13/3 B^2
+//   one-sided +   4(dx1^2 + 13/3 dxx1^2)   = (2 e3 - A)^2 + 13/3 A^2
+//   one-sided -                              (2 e2 + C)^2 + 13/3 C^2
+//   4th order     4(ux^2 + 13/3 uxx^2 + ux uxxx/5 + 39.06 uxxx^2)
+//                                          = S^2 + 13/3 B^2 + T (1.1125 T - S/3)
+// For a pair of axes with the diagonals pp pm mp mm and the central
+// differences Sa, Sb: al, be = (pp-pm) - Sb, (mp-mm) - Sb and
+// ph, ps = (pp-mp) - Sa, (pm-mm) - Sa are twice the mixed derivatives of the
+// four sided stencils; M = (al-be)^2 = (ph-ps)^2 is 16 u_ab^2, and the mixed
+// third derivatives are (al+be)/4, (ph+ps)/4, whose squares follow from the
+// others: (al+be)^2 = 2(al^2+be^2) - M.
+// With normalised weights n4 (R4), n1, n2 (sided +, -) along an axis, and
+// gamma_R4 + sum gamma_R3 = 1, the combination of reconstruction.c:223-257 is
+//   2 c1  = S - n1 a - n2 c + n4 (g3s - 11/60)/g4 T
+//   2 c2  = B + n1 a - n2 c - n4 g3s/g4 F
+//   12 c3 = n4/g4 T
+// The eight reciprocals 1/IS come from two, each of a product of four IS
+// (in range whenever IS^4 is), each refined to full precision.
+template <int SYS, typename Get>
+__device__ __forceinline__ void cweno_faces64(Get get, const CwArgs &p, double (&fm)[3], double (&fp)[3])
+{
+    const double k13 = 13.0 / 3.0, k7 = 7.0 / 6.0, eps = 4.0e-12;
+    const double u0 = get(0);
+    double S[3], B[3], a[3], c[3];
+    double C[3], P[3], M[3], is4;
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        const double m2 = get(1 + 4 * d), m1 = get(2 + 4 * d), p1 = get(3 + 4 * d), p2 = get(4 + 4 * d);
+        const double e1 = m1 - m2, e2 = u0 - m1, e3 = p1 - u0, e4 = p2 - p1;
+        const double A = e4 - e3, Cc = e2 - e1;
+        B[d] = e3 - e2;
+        S[d] = e2 + e3;
+        a[d] = A - B[d];
+        c[d] = B[d] - Cc;
+        const double T = a[d] + c[d];
+        const double D1 = fma(2.0, e3, -A), D2 = fma(2.0, e2, Cc);
+        C[d] = fma(S[d], S[d], fma(k13 * B[d], B[d], 0.5 * eps));   // a sum of two carries eps
+        P[d] = fma(D1, D1, (k13 * A) * A);
+        M[d] = fma(D2, D2, (k13 * Cc) * Cc);
+        const double t = fma(S[d], -1.0 / 3.0, 1.1125 * T);
+        is4 = d == 0 ? T * t : fma(T, t, is4);
+    }
+    const double Cyz = C[1] + C[2], Czx = C[2] + C[0], Cxy = C[0] + C[1];
+    double t0 = Cyz + (C[0] - 0.5 * eps);
+    is4 += t0;
+    asm volatile("" ::: "memory");
+    // twice the mixed derivatives of one pair of axes
+    auto pair = [&](int q, double Sa, double Sb, double &al, double &be, double &ph, double &ps, double &m) {
+        const double pp = get(q), pm = get(q + 1), mp = get(q + 2), mm = get(q + 3);
+        al = (pp - pm) - Sb;
+        be = (mp - mm) - Sb;
+        ph = (pp - mp) - Sa;
+        const double x = al - be;
+        ps = ph - x;
+        m = x * x;
+    };
+    double q[6], Mxy, Myz, Mzx;
+    {
+        double al, be, ph, ps;
+        pair(13, S[0], S[1], al, be, ph, ps, Mxy);   // (x, y): x+, x-, y+, y-
+        q[0] = al * al; q[1] = be * be; q[2] = ph * ph; q[3] = ps * ps;
+        asm volatile("" ::: "memory");
+        pair(17, S[1], S[2], al, be, ph, ps, Myz);   // (y, z): y+, y-, z+, z-
+        q[2] = fma(al, al, q[2]); q[3] = fma(be, be, q[3]); q[4] = ph * ph; q[5] = ps * ps;
+        asm volatile("" ::: "memory");
+        pair(21, S[2], S[0], al, be, ph, ps, Mzx);   // (z, x): z+, z-, x+, x-
+        q[4] = fma(al, al, q[4]); q[5] = fma(be, be, q[5]); q[0] = fma(ph, ph, q[0]); q[1] = fma(ps, ps, q[1]);
+    }
+    asm volatile("" ::: "memory");
+    const double Ms = (Mxy + Myz) + Mzx;
+    const double Q = ((q[0] + q[1]) + (q[2] + q[3])) + (q[4] + q[5]);
+    t0 = fma(0.25 * k7, Ms, t0);
+    is4 = fma(2.35, Q, is4);
+    is4 = fma(0.25 * k7 - 2.35, Ms, is4);
+    {
+        const double z = ((get(25) - get(26)) - (get(27) - get(29))) - ((get(28) - get(30)) - (get(31) - get(32)));
+        is4 = fma((61.0 / 768.0) * z, z, is4);
+    }
+    const double t1 = fma(k7, fma(0.25, Myz, q[0]), P[0] + Cyz), t2 = fma(k7, fma(0.25, Myz, q[1]), M[0] + Cyz);
+    const double t3 = fma(k7, fma(0.25, Mzx, q[2]), P[1] + Czx), t4 = fma(k7, fma(0.25, Mzx, q[3]), M[1] + Czx);
+    const double t5 = fma(k7, fma(0.25, Mxy, q[4]), P[2] + Cxy), t6 = fma(k7, fma(0.25, Mxy, q[5]), M[2] + Cxy);
+
+    // gamma / IS^4, p = 4 (reconstruction.c:205-218)
+    auto inv4 = [](double &w, double &x, double &y, double &z) {
+        const double wx = w * x, yz = y * z;
+        const double r = rcp64_full(wx * yz);
+        const double rwx = r * yz, ryz = r * wx;
+        const double iw = rwx * x, ix = rwx * w, iy = ryz * z, iz = ryz * y;
+        w = iw; x = ix; y = iy; z = iz;
+    };
+    double r4 = is4, r0 = t0, r1 = t1, r2 = t2, r3 = t3, r5 = t4, r6 = t5, r7 = t6;
+    inv4(r4, r0, r1, r2);
+    inv4(r3, r5, r6, r7);
+    auto pow4 = [](double r) { const double r2 = r * r; return r2 * r2; };
+    double w4 = p.g4 * pow4(r4);
+    double n[6] = {pow4(r1), pow4(r2), pow4(r3), pow4(r5), pow4(r6), pow4(r7)};
+    const double sided = ((n[0] + n[1]) + (n[2] + n[3])) + (n[4] + n[5]);
+    const double it = rcp64_full(fma(p.g3s, sided, fma(p.g3c, pow4(r0), w4)));
+    const double is = p.g3s * it;
+    w4 *= it;
+    const double ke = p.k2 * w4, ko = (SYS == ACX_ACOUSTIC4 ? p.k1a : p.k1w) * w4;
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        const double h1 = n[2 * d] * a[d], h2 = n[2 * d + 1] * c[d];
+        const double T = a[d] + c[d], F = a[d] - c[d];
+        const double E = fma(-ke, F, fma(is, h1 - h2, B[d]));
+        const double O = fma(ko, T, fma(-is, h1 + h2, S[d]));
+        if constexpr (SYS == ACX_ACOUSTIC4) {
+            const double even = fma(1.0 / 12.0, E, u0);
+            fm[d] = fma(-0.25, O, even);
+            fp[d] = fma(0.25, O, even);
+        } else {
+            fm[d] = 0.5 * (O - E);
+            fp[d] = 0.5 * (O + E);
+        }
+    }
 }
 
 } // namespace acx

@@ -42,6 +42,9 @@ struct CwArgs {
     double a, b, c;
     double K, invrho, s, inv_h, c2;
     double g4, g3c, g3s, inv_g4;   // linear weights: gamma_R4, gamma_R3[0], gamma_R3[1..6], 1/gamma_R4
+    // FP64 combination (cweno_faces64): (g3s - 11/60)/g4 plus the share of c3
+    // in the odd part (ACOUSTIC4 1/60, WAVE2 1/10, over g4), and g3s/g4
+    double k1a, k1w, k2;
     unsigned *nf;                  // non-finite watch word (host-mapped; null: no watch)
 };
 
