@@ -113,11 +113,8 @@ static int launch_linear_dma_w2(const LinArgs &a, hipStream_t s)
 
 // ---------------------------------------------------------------------------
 
-// Automatic z-chunk (auto_zc, acx_api.hip): measured for these kernels (ACOUSTIC4,
-// 256^3 and 384^3), the round model ranks the z-chunks as the timings do for
-// the FP64 halo-ring kernel (one workgroup per CU: 128 planes at 256^3, +4 %
-// over 64; 64 at 384^3) and the FP32 lead-plane kernel (two per CU: 64 at
-// 256^3, 128 at 384^3, +3 % over 64).
+// Automatic z-chunk: the round model of auto_zc (acx_api.hip) with a start of
+// 10 planes.
 template <typename T, int SYS, int EPI, int PF, int WPE, int BX, int BY, bool WALLS = false, bool NT = false>
 static int launch_linear_v(const LinArgs &a, hipStream_t s)
 {
