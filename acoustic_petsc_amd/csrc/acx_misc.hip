@@ -1,6 +1,7 @@
 // acx_misc.hip -- FP64 reductions, the CTCS leapfrog sibling and host-side
 // synthetic fields.
 #include <math.h>
+#include <mutex>
 #include <stdlib.h>
 #include <string.h>
 #include <vector>
@@ -9,15 +10,24 @@
 
 namespace acx {
 
-// ---- deterministic two-pass FP64 reductions ------------------------------
-// pass 1: each block reduces a grid-stride slice to (sum, max) with wavefront
-// shuffles; pass 2: one block reduces the partials in a fixed order.
+// ---- deterministic FP64 reductions ---------------------------------------
+// Each block reduces a grid-stride slice to (sum, max) with wavefront
+// shuffles and leaves them in host-mapped memory; the host adds up the
+// partials in a fixed order once the stream has been waited for.  (The last
+// block to finish doing it on the device, with the fences that takes in every
+// block, made the kernel twice as long; a second launch costs 10 us.)
+// Bound by memory: four loads in flight per thread, nontemporal (9 % faster on
+// a state larger than the caches, the same on smaller ones), 4 blocks per CU.
+// A call on the 537 MB state of 256^3 ACOUSTIC4: all components 210 -> 96
+// us, one component 231 -> 98 us (8-byte loads at the cell's stride; before,
+// every value with a 64-bit remainder each), energy 140 -> 96 us.
 constexpr int RED_THREADS = 256;
-constexpr int RED_BLOCKS = 1024;
+constexpr int RED_BLOCKS = 1024;   // most partials of one reduction
+constexpr int RED_UNROLL = 4;
 
 // max that keeps a NaN (fmax drops it): a NaN anywhere makes the result NaN,
 // as PETSc's VecNorm(NORM_INFINITY) reports it
-__device__ __forceinline__ double nmax(double a, double b) { return (a > b || a != a) ? a : b; }
+__host__ __device__ __forceinline__ double nmax(double a, double b) { return (a > b || a != a) ? a : b; }
 
 __device__ __forceinline__ void wave_reduce(double &s, double &m)
 {
@@ -84,94 +94,184 @@ __global__ void __launch_bounds__(CP_THREADS) k_copy1(const double *__restrict__
     }
 }
 
-// mode 0: x = X[i] (component filter); mode 1: x = (hi + lo) - B, also sums B^2
+// Blocks for n items, RED_UNROLL per thread and sweep.
+static int red_blocks(size_t n)
+{
+    const size_t per = (size_t)RED_THREADS * RED_UNROLL, b = (n + per - 1) / per;
+    return b < 1 ? 1 : b > RED_BLOCKS ? RED_BLOCKS : (int)b;
+}
+
+// f(i) over i = 0 .. n-1, RED_UNROLL loads of a thread in flight: get(i)
+// loads item i, use(item) accumulates it (items in ascending order per thread).
+template <typename Get, typename Use>
+__device__ __forceinline__ void red_sweep(size_t n, Get get, Use use)
+{
+    constexpr size_t span = (size_t)RED_THREADS * RED_UNROLL;
+    size_t base = blockIdx.x * span + threadIdx.x;
+    const size_t step = gridDim.x * span;
+    for (; base + (RED_UNROLL - 1) * RED_THREADS < n; base += step) {
+        decltype(get(base)) v[RED_UNROLL];
+#pragma unroll
+        for (int u = 0; u < RED_UNROLL; ++u) v[u] = get(base + (size_t)u * RED_THREADS);
+#pragma unroll
+        for (int u = 0; u < RED_UNROLL; ++u) use(v[u]);
+    }
+    for (; base < n; base += RED_THREADS) use(get(base));   // the last, partial sweep
+}
+
+// Sum of squares and largest magnitude: of n2 pairs of values (PAIRS: the
+// array is 16-byte aligned and every component counts), or of the n values
+// X[0], X[stride], ...
+template <bool PAIRS>
 __global__ void __launch_bounds__(RED_THREADS)
-k_reduce_pass1(const double *__restrict__ X, size_t n, int nvar, int comp, double *__restrict__ part)
+k_norms(const double *__restrict__ X, size_t n, int stride, double *__restrict__ part)
 {
     double s = 0.0, m = 0.0;
-    for (size_t i = blockIdx.x * (size_t)RED_THREADS + threadIdx.x; i < n; i += (size_t)gridDim.x * RED_THREADS) {
-        if (comp >= 0 && (int)(i % nvar) != comp) continue;
-        double v = X[i];
-        s += v * v;
-        m = nmax(m, fabs(v));
+    if constexpr (PAIRS) {
+        const acx_dbl2 *X2 = reinterpret_cast<const acx_dbl2 *>(X);
+        double t = 0.0, k = 0.0;
+        red_sweep(n / 2, [&](size_t i) { return __builtin_nontemporal_load(X2 + i); }, [&](acx_dbl2 v) {
+            s = fma(v.x, v.x, s);
+            t = fma(v.y, v.y, t);
+            m = nmax(m, fabs(v.x));
+            k = nmax(k, fabs(v.y));
+        });
+        if ((n & 1) && blockIdx.x == 0 && threadIdx.x == 0) {
+            const double v = X[n - 1];
+            s = fma(v, v, s);
+            m = nmax(m, fabs(v));
+        }
+        s += t;
+        m = nmax(m, k);
+    } else {
+        red_sweep(n, [&](size_t i) { return __builtin_nontemporal_load(X + i * stride); }, [&](double v) {
+            s = fma(v, v, s);
+            m = nmax(m, fabs(v));
+        });
     }
     block_reduce(s, m);
     if (threadIdx.x == 0) { part[2 * blockIdx.x] = s; part[2 * blockIdx.x + 1] = m; }
 }
 
 __global__ void __launch_bounds__(RED_THREADS)
-k_diff_pass1(const float *__restrict__ HI, const float *__restrict__ LO, const double *__restrict__ B, size_t n,
-             double *__restrict__ part)
+k_diff(const float *__restrict__ HI, const float *__restrict__ LO, const double *__restrict__ B, size_t n,
+       double *__restrict__ part)
 {
+    struct Item { float hi, lo; double b; };
     double s = 0.0, m = 0.0, sb = 0.0, mb = 0.0;
-    for (size_t i = blockIdx.x * (size_t)RED_THREADS + threadIdx.x; i < n; i += (size_t)gridDim.x * RED_THREADS) {
-        double a = (double)HI[i] + (LO ? (double)LO[i] : 0.0);
-        double d = a - B[i];
+    red_sweep(n, [&](size_t i) { return Item{HI[i], LO ? LO[i] : 0.f, B[i]}; }, [&](const Item &v) {
+        const double d = ((double)v.hi + (double)v.lo) - v.b;
         s += d * d;
         m = nmax(m, fabs(d));
-        sb += B[i] * B[i];
-    }
+        sb += v.b * v.b;
+    });
     block_reduce(s, m);
     __syncthreads();
     block_reduce(sb, mb);
     if (threadIdx.x == 0) { part[3 * blockIdx.x] = s; part[3 * blockIdx.x + 1] = m; part[3 * blockIdx.x + 2] = sb; }
 }
 
+// Twice the acoustic energy density summed over the cells, as 2 ncell pairs of
+// values: (p, u) where the pair index is even, (v, w) where it is odd; a
+// thread's pairs are all of one kind.
 __global__ void __launch_bounds__(RED_THREADS)
-k_energy_pass1(const double *__restrict__ U, size_t ncell, double invK, double rho0, double *__restrict__ part)
+k_energy(const double *__restrict__ U, size_t ncell, double invK, double rho0, double *__restrict__ part)
 {
-    double s = 0.0, m = 0.0;
-    for (size_t i = blockIdx.x * (size_t)RED_THREADS + threadIdx.x; i < ncell; i += (size_t)gridDim.x * RED_THREADS) {
-        const double2 *p = reinterpret_cast<const double2 *>(U + 4 * i);
-        double2 a = p[0], b = p[1];
-        double e = a.x * a.x * invK + rho0 * (a.y * a.y + b.x * b.x + b.y * b.y);
-        s += e;
-        m = nmax(m, e);
-    }
+    static_assert(RED_THREADS % 2 == 0, "pair parity per thread");
+    const acx_dbl2 *X2 = reinterpret_cast<const acx_dbl2 *>(U);
+    const double wx = threadIdx.x & 1 ? rho0 : invK;
+    double s = 0.0, t = 0.0, m = 0.0;
+    red_sweep(2 * ncell, [&](size_t i) { return __builtin_nontemporal_load(X2 + i); }, [&](acx_dbl2 v) {
+        s = fma(v.x, v.x, s);
+        t = fma(v.y, v.y, t);
+    });
+    s = wx * s + rho0 * t;
     block_reduce(s, m);
     if (threadIdx.x == 0) { part[2 * blockIdx.x] = s; part[2 * blockIdx.x + 1] = m; }
 }
 
-__global__ void __launch_bounds__(RED_THREADS)
-k_reduce_pass2(const double *__restrict__ part, int nblk, int stride, double *__restrict__ out)
+// The partials of one call (up to three per block) in host-mapped memory.
+// Each device keeps RED_SLOTS of them, made on first use and lent to one call
+// at a time, so calls on different streams and threads never share one; a
+// call that finds none free makes its own.  A call on a 24^3 state, with the
+// second launch, the pool allocation and the copy gone: 67 -> 21 us.
+constexpr int RED_SLOTS = 16;
+constexpr size_t RED_PART = 3 * (size_t)RED_BLOCKS;
+
+struct RedPool {
+    double *host = nullptr, *dev = nullptr;
+    unsigned used = 0;
+};
+static RedPool g_red[64];
+static std::mutex g_red_mu;
+
+struct RedScratch {
+    int device = -1, slot = -1;
+    double *host = nullptr, *part = nullptr;   // host and device address of the partials
+};
+
+static int red_make(double **host, double **dev, size_t slots)
 {
-    // fixed-order accumulation of the block partials (columns 0: sum, 1: max, 2: sum)
-    double s = 0.0, m = 0.0, s2 = 0.0, dummy = 0.0;
-    for (int i = threadIdx.x; i < nblk; i += RED_THREADS) {
-        s += part[stride * i];
-        m = nmax(m, part[stride * i + 1]);
-        if (stride > 2) s2 += part[stride * i + 2];
+    // an allocation is allowed here while another thread captures a stream
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    int rc = hip_check(hipHostMalloc((void **)host, slots * RED_PART * sizeof(double),
+                                     hipHostMallocMapped | hipHostMallocCoherent), "reduce scratch");
+    if (!rc && (rc = hip_check(hipHostGetDevicePointer((void **)dev, *host, 0), "reduce scratch"))) {
+        (void)hipHostFree(*host);
+        *host = nullptr;
     }
-    block_reduce(s, m);
-    __syncthreads();
-    block_reduce(s2, dummy);
-    if (threadIdx.x == 0) { out[0] = s; out[1] = m; out[2] = s2; }
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    return rc;
 }
 
-// Partials (3 per block) + result of one reduction.
-constexpr size_t RED_SCRATCH = 3 * RED_BLOCKS + 4;
-
-// The partials of one call, taken from the stream-ordered pool of `s` and
-// returned to it when the call ends, so calls on different streams never
-// share them.
-static int red_alloc(double **part, hipStream_t s)
+static int red_take(RedScratch &r, hipStream_t s)
 {
-    return hip_check(hipMallocAsync((void **)part, RED_SCRATCH * sizeof(double), s), "reduce scratch");
-}
-
-static int finish(double *part, int stride, double *host_out, int nout, hipStream_t s)
-{
-    double *res = part + 3 * RED_BLOCKS;
-    hipLaunchKernelGGL(k_reduce_pass2, dim3(1), dim3(RED_THREADS), 0, s, part, RED_BLOCKS, stride, res);
-    int rc = hip_check(hipGetLastError(), "reduce pass 2");
-    double tmp[3];
-    if (!rc) rc = hip_check(hipMemcpyAsync(tmp, res, 3 * sizeof(double), hipMemcpyDeviceToHost, s), "reduce copy");
-    const int rf = hip_check(hipFreeAsync(part, s), "reduce scratch free");
-    if (!rc) rc = rf;
-    if (!rc) rc = hip_check(hipStreamSynchronize(s), "reduce sync");
+    // a reduction waits for its stream, which a capture does not allow
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &cap) == hipSuccess && cap != hipStreamCaptureStatusNone)
+        return hip_check(hipErrorStreamCaptureUnsupported, "reduce");
+    int rc = hip_check(hipGetDevice(&r.device), "reduce scratch: device");
     if (rc) return rc;
-    memcpy(host_out, tmp, nout * sizeof(double));
-    return ACX_OK;
+    if (r.device >= 0 && r.device < 64) {
+        std::lock_guard<std::mutex> lk(g_red_mu);
+        RedPool &p = g_red[r.device];
+        if (!p.host && (rc = red_make(&p.host, &p.dev, RED_SLOTS))) return rc;
+        for (int k = 0; k < RED_SLOTS; ++k)
+            if (!(p.used >> k & 1u)) {
+                p.used |= 1u << k;
+                r.slot = k;
+                r.host = p.host + k * RED_PART;
+                r.part = p.dev + k * RED_PART;
+                return ACX_OK;
+            }
+    }
+    return red_make(&r.host, &r.part, 1);
+}
+
+// The launch's error, the wait and the sums over the blocks (out: sum, max,
+// third column); the scratch goes back unless the wait failed (its kernel
+// might still run).
+static int red_finish(RedScratch &r, int nblk, int cols, double (&out)[3], hipStream_t s, const char *what)
+{
+    const int rc = hip_check(hipGetLastError(), what);
+    const int rs = hip_check(hipStreamSynchronize(s), "reduce sync");
+    if (rs) return rc ? rc : rs;
+    out[0] = out[1] = out[2] = 0.0;
+    if (!rc)
+        for (int b = 0; b < nblk; ++b) {
+            const double *p = r.host + (size_t)cols * b;
+            out[0] += p[0];
+            out[1] = nmax(out[1], p[1]);
+            if (cols > 2) out[2] += p[2];
+        }
+    if (r.slot >= 0) {
+        std::lock_guard<std::mutex> lk(g_red_mu);
+        g_red[r.device].used &= ~(1u << r.slot);
+    } else {
+        (void)hipHostFree(r.host);
+    }
+    return rc;
 }
 
 // ---- CTCS leapfrog (3d/ctcs/point_source/wave.c:138-215) -----------------
@@ -498,16 +598,19 @@ int acx_norms_f64(const double *X, size_t ncells, int nvar, int comp, double *ou
 {
     if (!X || !out || nvar < 1 || comp >= nvar) return set_error(ACX_EINVAL, "norms: bad arguments");
     hipStream_t s = (hipStream_t)stream;
-    double *part = nullptr;
-    int rc = red_alloc(&part, s);
+    RedScratch sc;
+    int rc = red_take(sc, s);
     if (rc) return rc;
-    hipLaunchKernelGGL(k_reduce_pass1, dim3(RED_BLOCKS), dim3(RED_THREADS), 0, s, X, ncells * nvar, nvar, comp, part);
-    if ((rc = hip_check(hipGetLastError(), "norms pass 1"))) {
-        (void)hipFreeAsync(part, s);
-        return rc;
-    }
+    const size_t n = comp < 0 ? ncells * nvar : ncells;
+    const bool pairs = comp < 0 && ((uintptr_t)X & 15) == 0;
+    const int nblk = red_blocks(pairs ? n / 2 : n);
+    if (pairs)
+        hipLaunchKernelGGL(k_norms<true>, dim3(nblk), dim3(RED_THREADS), 0, s, X, n, 1, sc.part);
+    else
+        hipLaunchKernelGGL(k_norms<false>, dim3(nblk), dim3(RED_THREADS), 0, s, comp < 0 ? X : X + comp, n,
+                           comp < 0 ? 1 : nvar, sc.part);
     double r[3];
-    if ((rc = finish(part, 2, r, 3, s))) return rc;
+    if ((rc = red_finish(sc, nblk, 2, r, s, "norms launch"))) return rc;
     out[0] = r[0];
     out[1] = r[1];
     return ACX_OK;
@@ -540,16 +643,13 @@ int acx_diff_f32c_f64(const float *HI, const float *LO, const double *B, size_t 
 {
     if (!HI || !B || !out) return set_error(ACX_EINVAL, "diff: bad arguments");
     hipStream_t s = (hipStream_t)stream;
-    double *part = nullptr;
-    int rc = red_alloc(&part, s);
+    RedScratch sc;
+    int rc = red_take(sc, s);
     if (rc) return rc;
-    hipLaunchKernelGGL(k_diff_pass1, dim3(RED_BLOCKS), dim3(RED_THREADS), 0, s, HI, LO, B, n, part);
-    if ((rc = hip_check(hipGetLastError(), "diff pass 1"))) {
-        (void)hipFreeAsync(part, s);
-        return rc;
-    }
+    const int nblk = red_blocks(n);
+    hipLaunchKernelGGL(k_diff, dim3(nblk), dim3(RED_THREADS), 0, s, HI, LO, B, n, sc.part);
     double r[3];
-    if ((rc = finish(part, 3, r, 3, s))) return rc;
+    if ((rc = red_finish(sc, nblk, 3, r, s, "diff launch"))) return rc;
     out[0] = r[2] > 0 ? sqrt(r[0] / r[2]) : sqrt(r[0]);
     out[1] = r[1];
     return ACX_OK;
@@ -559,18 +659,15 @@ int acx_energy_f64(const acx_grid *g, const double *U, double *out, void *stream
 {
     if (!g || !U || !out || g->system != ACX_ACOUSTIC4) return set_error(ACX_EINVAL, "energy: ACOUSTIC4 state required");
     hipStream_t s = (hipStream_t)stream;
-    double *part = nullptr;
-    int rc = red_alloc(&part, s);
+    RedScratch sc;
+    int rc = red_take(sc, s);
     if (rc) return rc;
     const size_t nc = (size_t)g->n[0] * g->n[1] * g->n[2];
     const double K = g->rho0 * g->c0 * g->c0;
-    hipLaunchKernelGGL(k_energy_pass1, dim3(RED_BLOCKS), dim3(RED_THREADS), 0, s, U, nc, 1.0 / K, g->rho0, part);
-    if ((rc = hip_check(hipGetLastError(), "energy pass 1"))) {
-        (void)hipFreeAsync(part, s);
-        return rc;
-    }
+    const int nblk = red_blocks(2 * nc);
+    hipLaunchKernelGGL(k_energy, dim3(nblk), dim3(RED_THREADS), 0, s, U, nc, 1.0 / K, g->rho0, sc.part);
     double r[3];
-    if ((rc = finish(part, 2, r, 3, s))) return rc;
+    if ((rc = red_finish(sc, nblk, 2, r, s, "energy launch"))) return rc;
     out[0] = 0.5 * r[0] * g->h * g->h * (g->n[2] == 1 ? 1.0 : g->h);   // cell area on a 2D grid
     return ACX_OK;
 }

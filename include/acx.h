@@ -106,8 +106,8 @@ int acx_ssp_rks3_step_f32c(const acx_grid *g, const float *HI, const float *LO, 
 /* out[0] = sum of squares of component `comp` (all components if comp < 0),
  * out[1] = max abs; host pointer out[2].  VecNorm (error_norms.c:87-89).
  * A NaN anywhere makes both results NaN (as PETSc's VecNorm).  The partial
- * sums live in a buffer taken per call on `stream` (stream-ordered), so
- * calls on different streams do not share scratch. */
+ * sums live in scratch lent to one call at a time, so calls on different
+ * streams and threads do not share it. */
 int acx_norms_f64(const double *X, size_t ncells, int nvar, int comp, double *out, void *stream);
 /* Y = X for n doubles, stream-ordered (VecCopy, used by the SSP stages of
  * PETSc's TSSSP, which the reference selects at 3d/weno4/plane_wave/
