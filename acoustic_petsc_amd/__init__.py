@@ -125,6 +125,7 @@ def lib():
             "acx_vec_copy_f64": [vp, vp, _C.c_size_t, vp],
             "acx_energy_f64": [gp, vp, _C.POINTER(dbl), vp],
             "acx_ctcs_update_f64": [_C.POINTER(_Ctcs), vp, vp, vp, vp, i32, _C.POINTER(dbl), vp],
+            "acx_ctcs_steps_f64": [_C.POINTER(_Ctcs), vp, vp, vp, vp, i32, i32, vp, vp],
             "acx_field_gaussians": [gp, _C.c_uint64, i32, dbl, dbl, dbl, dbl, vp],
             "acx_field_plane_wave": [gp, _C.POINTER(i32), dbl, dbl, vp],
         }
@@ -365,19 +366,17 @@ def ctcs_run(p, nt, stream=None):
     """UpdatePressure loop of wave.c:109-121 on the GPU; returns the receiver trace."""
     torch = _torch()
     n = (p.n[2], p.n[1], p.n[0])
-    Pold = torch.zeros(n, dtype=torch.float64, device="cuda")
-    P = torch.zeros_like(Pold)
-    Pnew = torch.zeros_like(Pold)
-    C = torch.full_like(Pold, p.c0)
-    cs = p.c_struct()
-    trace = []
-    r = (_C.c_double * 1)()
-    for it in range(nt):
-        _check(lib().acx_ctcs_update_f64(_C.byref(cs), _ptr(Pold, torch.float64), _ptr(P, torch.float64),
-                                         _ptr(Pnew, torch.float64), _ptr(C, torch.float64), it, r, _stream(stream)))
-        trace.append(r[0])
-        Pold, P, Pnew = P, Pnew, Pold   # Pold = P; P = Pnew (VecCopy pair, wave.c:115-116)
-    return trace
+    st = stream if stream is not None else torch.cuda.current_stream()
+    with torch.cuda.stream(st):
+        Pold = torch.zeros(n, dtype=torch.float64, device="cuda")
+        P = torch.zeros_like(Pold)
+        Pnew = torch.zeros_like(Pold)
+        C = torch.full_like(Pold, p.c0)
+        trace = torch.zeros(nt, dtype=torch.float64, device="cuda")
+        f64 = torch.float64
+        _check(lib().acx_ctcs_steps_f64(_C.byref(p.c_struct()), _ptr(Pold, f64), _ptr(P, f64), _ptr(Pnew, f64),
+                                        _ptr(C, f64), 0, nt, _ptr(trace, f64), _stream(st)))
+        return trace.tolist()
 
 
 # ---- synthetic fields (host) ---------------------------------------------

@@ -276,16 +276,19 @@ static int red_finish(RedScratch &r, int nblk, int cols, double (&out)[3], hipSt
 
 // ---- CTCS leapfrog (3d/ctcs/point_source/wave.c:138-215) -----------------
 
-__device__ __forceinline__ double ctcs_source(double t, double f0)
+// The source's share of one update at its cell (wave.c:234-240), formed once
+// per launch on the host: every kernel form adds the same value.
+static double ctcs_source_step(const acx_ctcs &c, int it)
 {
-    const double t0 = 4.0 / f0;   // wave.c:234-240
-    return -2.0 * (t - t0) * f0 * f0 * exp(-1.0 * f0 * f0 * (t - t0) * (t - t0));
+    const double t = it * c.dt, f0 = c.f0, t0 = 4.0 / f0;
+    const double s = -2.0 * (t - t0) * f0 * f0 * exp(-1.0 * f0 * f0 * (t - t0) * (t - t0));
+    return s / (c.dx * c.dy * c.dz) * c.dt * c.dt;
 }
 
 template <int ST>
 __global__ void __launch_bounds__(256)
 k_ctcs(const double *__restrict__ Pold, const double *__restrict__ P, double *__restrict__ Pnew,
-       const double *__restrict__ C, acx_ctcs c, int it, double *__restrict__ rcv)
+       const double *__restrict__ C, acx_ctcs c, double src, double *__restrict__ rcv)
 {
     const int nx = c.n[0], ny = c.n[1], nz = c.n[2];
     const int i = blockIdx.x * blockDim.x + threadIdx.x, j = blockIdx.y, k = blockIdx.z;
@@ -312,7 +315,7 @@ k_ctcs(const double *__restrict__ Pold, const double *__restrict__ P, double *__
     const size_t o = ((size_t)k * ny + j) * nx + i;
     const double cc = C[o], dt = c.dt;
     double pn = 2.0 * p0 - Pold[o] + cc * cc * dt * dt * (pxx + pyy + pzz);
-    if (i == c.src[0] && j == c.src[1] && k == c.src[2]) pn += ctcs_source(it * dt, c.f0) / (c.dx * c.dy * c.dz) * dt * dt;
+    if (i == c.src[0] && j == c.src[1] && k == c.src[2]) pn += src;
     if (rcv && i == c.rcv[0] && j == c.rcv[1] && k == c.rcv[2]) rcv[0] = p0;
     Pnew[o] = pn;
 }
@@ -329,7 +332,7 @@ constexpr int CT_BX = 32, CT_BY = 8;
 template <int ST>
 __global__ void __launch_bounds__(CT_BX *CT_BY)
 k_ctcs_z(const double *__restrict__ Pold, const double *__restrict__ P, double *__restrict__ Pnew,
-         const double *__restrict__ C, acx_ctcs c, int it, int zc, double *__restrict__ rcv)
+         const double *__restrict__ C, acx_ctcs c, double src, int zc, double *__restrict__ rcv)
 {
     constexpr int LX = CT_BX + 2 * ST, LY = CT_BY + 2 * ST, NH = 2 * ST * (CT_BX + CT_BY);
     static_assert(NH <= CT_BX * CT_BY, "every halo cell of a plane needs a thread of its own");
@@ -395,8 +398,7 @@ k_ctcs_z(const double *__restrict__ Pold, const double *__restrict__ P, double *
                        1.0 / 12.0 * q[0]) * invdz2;
             }
             double pn = 2.0 * p0 - po + cc * cc * dt * dt * (pxx + pyy + pzz);
-            if (i == c.src[0] && j == c.src[1] && z == c.src[2])
-                pn += ctcs_source(it * dt, c.f0) / (c.dx * c.dy * c.dz) * dt * dt;
+            if (i == c.src[0] && j == c.src[1] && z == c.src[2]) pn += src;
             if (rcv && i == c.rcv[0] && j == c.rcv[1] && z == c.rcv[2]) rcv[0] = p0;
             Pnew[o] = pn;
         }
@@ -438,7 +440,7 @@ struct CtDma {
 template <int ST>
 __global__ void __launch_bounds__(CtDma::BX *CtDma::BY) __attribute__((amdgpu_waves_per_eu(4)))
 k_ctcs_dma(const double *__restrict__ Pold, const double *__restrict__ P, double *__restrict__ Pnew,
-           const double *__restrict__ C, acx_ctcs c, int it, int zc, double *__restrict__ rcv)
+           const double *__restrict__ C, acx_ctcs c, double src, int zc, double *__restrict__ rcv)
 {
     using D = CtDma;
     __shared__ __attribute__((aligned(16))) unsigned char ring[D::NSLOT * D::SLOT];
@@ -555,13 +557,127 @@ k_ctcs_dma(const double *__restrict__ Pold, const double *__restrict__ P, double
                        1.0 / 12.0 * q[0]) * invdz2;
             }
             double pn = 2.0 * p0 - po + cc * cc * dt * dt * (pxx + pyy + pzz);
-            if (i == c.src[0] && j == c.src[1] && z == c.src[2])
-                pn += ctcs_source(it * dt, c.f0) / (c.dx * c.dy * c.dz) * dt * dt;
+            if (i == c.src[0] && j == c.src[1] && z == c.src[2]) pn += src;
             if (rcv && i == c.rcv[0] && j == c.rcv[1] && z == c.rcv[2]) rcv[0] = p0;
             Pnew[(size_t)z * plane + col] = pn;
         }
     }
     // every load issued has been waited for by the last iteration (vmcnt 0)
+}
+
+// The same update for 3D grids that live in the caches between steps (even x
+// extent, 16-byte aligned arrays): one thread per pair of x-neighbours, 13
+// 16-byte loads all in flight at once instead of a march along z.
+// Arithmetic as in k_ctcs, term by term.  Up to about 2.5e6 cells (four arrays
+// of 80 MB together) the march is bound by the latency of its planes, not by
+// bytes.  us per update, march and this kernel: 48^3 6.8 / 3.3, 64^3 7.1 /
+// 3.9, 100^3 11.7 / 7.8, 128^3 15.6 / 14.4, 160^3 24.2 / 26.2, 256^3 108 / 132.
+constexpr int CD_THREADS = 256;
+constexpr size_t CD_CELLS = 2500000;
+
+template <int ST>
+__global__ void __launch_bounds__(CD_THREADS)
+k_ctcs_pair(const double *__restrict__ Pold, const double *__restrict__ P, double *__restrict__ Pnew,
+            const double *__restrict__ C, acx_ctcs c, double src, int bpp, double *__restrict__ rcv)
+{
+    const int np = c.n[0] / 2, ny = c.n[1], nz = c.n[2];
+    const int b = xcd_logical_tile(blockIdx.x, gridDim.x), k = b / bpp;
+    const unsigned e = (unsigned)(b - k * bpp) * CD_THREADS + threadIdx.x;   // pair of the plane
+    if (e >= (unsigned)np * (unsigned)ny) return;
+    const int j = (int)(e / (unsigned)np), i2 = (int)(e - (unsigned)j * (unsigned)np);
+    auto W = [](int a, int n) { return a < 0 ? a + n : (a >= n ? a - n : a); };
+    const acx_dbl2 *P2 = reinterpret_cast<const acx_dbl2 *>(P);
+    auto at = [&](int a, int bb, int d) {
+        return P2[((size_t)W(k + d, nz) * ny + W(j + bb, ny)) * np + W(i2 + a, np)];
+    };
+    const size_t o = ((size_t)k * ny + j) * np + i2;
+    const acx_dbl2 p0 = P2[o], xm = at(-1, 0, 0), xp = at(1, 0, 0);
+    const acx_dbl2 ym1 = at(0, -1, 0), yp1 = at(0, 1, 0), zm1 = at(0, 0, -1), zp1 = at(0, 0, 1);
+    acx_dbl2 ym2 = p0, yp2 = p0, zm2 = p0, zp2 = p0;
+    if (ST == 2) {
+        ym2 = at(0, -2, 0);
+        yp2 = at(0, 2, 0);
+        zm2 = at(0, 0, -2);
+        zp2 = at(0, 0, 2);
+    }
+    const acx_dbl2 po = reinterpret_cast<const acx_dbl2 *>(Pold)[o], cc = reinterpret_cast<const acx_dbl2 *>(C)[o];
+    const double x[6] = {xm.x, xm.y, p0.x, p0.y, xp.x, xp.y};
+    const double invdx2 = 1.0 / (c.dx * c.dx), invdy2 = 1.0 / (c.dy * c.dy), invdz2 = 1.0 / (c.dz * c.dz);
+    const double dt = c.dt;
+    acx_dbl2 r;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const double q = x[2 + h];
+        double pxx, pyy, pzz;
+        if (ST == 1) {
+            pxx = (x[3 + h] - 2.0 * q + x[1 + h]) * invdx2;
+            pyy = (yp1[h] - 2.0 * q + ym1[h]) * invdy2;
+            pzz = (zp1[h] - 2.0 * q + zm1[h]) * invdz2;
+        } else {
+            pxx = (-1.0 / 12 * x[4 + h] + 4.0 / 3.0 * x[3 + h] - 5.0 / 2.0 * q + 4.0 / 3.0 * x[1 + h] -
+                   1.0 / 12.0 * x[h]) * invdx2;
+            pyy = (-1.0 / 12 * yp2[h] + 4.0 / 3.0 * yp1[h] - 5.0 / 2.0 * q + 4.0 / 3.0 * ym1[h] - 1.0 / 12.0 * ym2[h]) *
+                  invdy2;
+            pzz = (-1.0 / 12 * zp2[h] + 4.0 / 3.0 * zp1[h] - 5.0 / 2.0 * q + 4.0 / 3.0 * zm1[h] - 1.0 / 12.0 * zm2[h]) *
+                  invdz2;
+        }
+        double pn = 2.0 * q - po[h] + cc[h] * cc[h] * dt * dt * (pxx + pyy + pzz);
+        const int i = 2 * i2 + h;
+        if (i == c.src[0] && j == c.src[1] && k == c.src[2]) pn += src;
+        if (rcv && i == c.rcv[0] && j == c.rcv[1] && k == c.rcv[2]) rcv[0] = q;
+        r[h] = pn;
+    }
+    reinterpret_cast<acx_dbl2 *>(Pnew)[o] = r;
+}
+
+static int check_ctcs(const acx_ctcs *c, const double *POLD, const double *P, const double *PNEW, const double *C)
+{
+    if (!c || !POLD || !P || !PNEW || !C || PNEW == P) return set_error(ACX_EINVAL, "ctcs: bad arguments");
+    for (int d = 0; d < 3; ++d)
+        if (c->n[d] < 5 && c->n[d] != 1) return set_error(ACX_EINVAL, "ctcs: at least 5 cells per axis (or 1)");
+    if (c->stencil != 1 && c->stencil != 2) return set_error(ACX_EINVAL, "stencil width can be either 1 or 2");
+    return ACX_OK;
+}
+
+// One leapfrog update; rcv (device, may be null) receives P at the receiver.
+static int launch_ctcs(const acx_ctcs *c, const double *POLD, const double *P, double *PNEW, const double *C, int it,
+                       double *rcv, hipStream_t s)
+{
+    const double src = ctcs_source_step(*c, it);
+    const bool vol = c->n[0] >= 5 && c->n[1] >= 5 && c->n[2] >= 5;
+    const bool pairs = vol && c->n[0] % 2 == 0 && (size_t)c->n[0] * c->n[1] < 0xffffffffu &&
+                       ((((uintptr_t)POLD) | ((uintptr_t)P) | ((uintptr_t)C) | ((uintptr_t)PNEW)) & 15) == 0;
+    if (pairs && (size_t)c->n[0] * c->n[1] * c->n[2] <= CD_CELLS) {
+        const size_t bpp = ((size_t)c->n[0] / 2 * c->n[1] + CD_THREADS - 1) / CD_THREADS;
+        dim3 blk(CD_THREADS), grd((unsigned)(bpp * c->n[2]));
+        if (c->stencil == 1) hipLaunchKernelGGL(k_ctcs_pair<1>, grd, blk, 0, s, POLD, P, PNEW, C, *c, src, (int)bpp, rcv);
+        else hipLaunchKernelGGL(k_ctcs_pair<2>, grd, blk, 0, s, POLD, P, PNEW, C, *c, src, (int)bpp, rcv);
+    } else if (pairs) {
+        // 3D, LDS-DMA march: z-chunk from the round model, two blocks per CU
+        // (measured at 256^3: 144 -> 152 G cell-updates/s, bit-identical to
+        // the register-queue march below)
+        const int ntx = (c->n[0] + CtDma::BX - 1) / CtDma::BX, nty = (c->n[1] + CtDma::BY - 1) / CtDma::BY;
+        const int zc = auto_zc(ntx, nty, c->n[2], device_cus() * 2, 4);
+        const size_t nb = (size_t)ntx * nty * ((c->n[2] + zc - 1) / zc);
+        dim3 blk(CtDma::BX, CtDma::BY), grd((unsigned)nb);
+        if (c->stencil == 1) hipLaunchKernelGGL(k_ctcs_dma<1>, grd, blk, 0, s, POLD, P, PNEW, C, *c, src, zc, rcv);
+        else hipLaunchKernelGGL(k_ctcs_dma<2>, grd, blk, 0, s, POLD, P, PNEW, C, *c, src, zc, rcv);
+    } else if (vol) {
+        // 3D: z-march; 32 planes per block, halved (down to 4) below 1024 blocks
+        const size_t cols = (size_t)((c->n[0] + CT_BX - 1) / CT_BX) * ((c->n[1] + CT_BY - 1) / CT_BY);
+        int zc = 32;
+        while (zc > 4 && cols * ((c->n[2] + zc - 1) / zc) < 1024) zc /= 2;
+        const size_t nb = cols * ((c->n[2] + zc - 1) / zc);
+        dim3 blk(CT_BX, CT_BY), grd((unsigned)nb);
+        if (c->stencil == 1) hipLaunchKernelGGL(k_ctcs_z<1>, grd, blk, 0, s, POLD, P, PNEW, C, *c, src, zc, rcv);
+        else hipLaunchKernelGGL(k_ctcs_z<2>, grd, blk, 0, s, POLD, P, PNEW, C, *c, src, zc, rcv);
+    } else {
+        // 2D / 1D programs (axes of one cell): one thread per cell
+        dim3 blk(256), grd((c->n[0] + 255) / 256, c->n[1], c->n[2]);
+        if (c->stencil == 1) hipLaunchKernelGGL(k_ctcs<1>, grd, blk, 0, s, POLD, P, PNEW, C, *c, src, rcv);
+        else hipLaunchKernelGGL(k_ctcs<2>, grd, blk, 0, s, POLD, P, PNEW, C, *c, src, rcv);
+    }
+    return hip_check(hipGetLastError(), "ctcs launch");
 }
 
 // ---- host fields ---------------------------------------------------------
@@ -675,10 +791,8 @@ int acx_energy_f64(const acx_grid *g, const double *U, double *out, void *stream
 int acx_ctcs_update_f64(const acx_ctcs *c, const double *POLD, const double *P, double *PNEW, const double *C,
                         int it, double *rcv_out, void *stream)
 {
-    if (!c || !POLD || !P || !PNEW || !C || PNEW == P) return set_error(ACX_EINVAL, "ctcs: bad arguments");
-    for (int d = 0; d < 3; ++d)
-        if (c->n[d] < 5 && c->n[d] != 1) return set_error(ACX_EINVAL, "ctcs: at least 5 cells per axis (or 1)");
-    if (c->stencil != 1 && c->stencil != 2) return set_error(ACX_EINVAL, "stencil width can be either 1 or 2");
+    int rc = check_ctcs(c, POLD, P, PNEW, C);
+    if (rc) return rc;
     hipStream_t s = (hipStream_t)stream;
     // the receiver sample goes through a one-value buffer of this call (none
     // when the caller does not ask for it)
@@ -687,39 +801,28 @@ int acx_ctcs_update_f64(const acx_ctcs *c, const double *POLD, const double *P, 
         const int ra = hip_check(hipMallocAsync((void **)&rcv, sizeof(double), s), "ctcs receiver buffer");
         if (ra) return ra;
     }
-    const bool aligned = ((((uintptr_t)POLD) | ((uintptr_t)P) | ((uintptr_t)C)) & 15) == 0;
-    if (c->n[0] >= 5 && c->n[1] >= 5 && c->n[2] >= 5 && c->n[0] % 2 == 0 && aligned &&
-        (size_t)c->n[0] * c->n[1] < 0xffffffffu) {
-        // 3D, LDS-DMA march: z-chunk from the round model, two blocks per CU
-        // (measured at 256^3: 144 -> 152 G cell-updates/s, bit-identical to
-        // the register-queue march below)
-        const int ntx = (c->n[0] + CtDma::BX - 1) / CtDma::BX, nty = (c->n[1] + CtDma::BY - 1) / CtDma::BY;
-        const int zc = auto_zc(ntx, nty, c->n[2], device_cus() * 2, 4);
-        const size_t nb = (size_t)ntx * nty * ((c->n[2] + zc - 1) / zc);
-        dim3 blk(CtDma::BX, CtDma::BY), grd((unsigned)nb);
-        if (c->stencil == 1) hipLaunchKernelGGL(k_ctcs_dma<1>, grd, blk, 0, s, POLD, P, PNEW, C, *c, it, zc, rcv);
-        else hipLaunchKernelGGL(k_ctcs_dma<2>, grd, blk, 0, s, POLD, P, PNEW, C, *c, it, zc, rcv);
-    } else if (c->n[0] >= 5 && c->n[1] >= 5 && c->n[2] >= 5) {
-        // 3D: z-march; 32 planes per block, halved (down to 4) below 1024 blocks
-        const size_t cols = (size_t)((c->n[0] + CT_BX - 1) / CT_BX) * ((c->n[1] + CT_BY - 1) / CT_BY);
-        int zc = 32;
-        while (zc > 4 && cols * ((c->n[2] + zc - 1) / zc) < 1024) zc /= 2;
-        const size_t nb = cols * ((c->n[2] + zc - 1) / zc);
-        dim3 blk(CT_BX, CT_BY), grd((unsigned)nb);
-        if (c->stencil == 1) hipLaunchKernelGGL(k_ctcs_z<1>, grd, blk, 0, s, POLD, P, PNEW, C, *c, it, zc, rcv);
-        else hipLaunchKernelGGL(k_ctcs_z<2>, grd, blk, 0, s, POLD, P, PNEW, C, *c, it, zc, rcv);
-    } else {
-        // 2D / 1D programs (axes of one cell): one thread per cell
-        dim3 blk(256), grd((c->n[0] + 255) / 256, c->n[1], c->n[2]);
-        if (c->stencil == 1) hipLaunchKernelGGL(k_ctcs<1>, grd, blk, 0, s, POLD, P, PNEW, C, *c, it, rcv);
-        else hipLaunchKernelGGL(k_ctcs<2>, grd, blk, 0, s, POLD, P, PNEW, C, *c, it, rcv);
-    }
-    int rc = hip_check(hipGetLastError(), "ctcs launch");
+    rc = launch_ctcs(c, POLD, P, PNEW, C, it, rcv, s);
     if (rcv_out) {
         if (!rc) rc = hip_check(hipMemcpyAsync(rcv_out, rcv, sizeof(double), hipMemcpyDeviceToHost, s), "ctcs rcv copy");
         const int rf = hip_check(hipFreeAsync(rcv, s), "ctcs receiver buffer free");
         if (!rc) rc = rf;
         if (!rc) rc = hip_check(hipStreamSynchronize(s), "ctcs sync");
+    }
+    return rc;
+}
+
+int acx_ctcs_steps_f64(const acx_ctcs *c, double *POLD, double *P, double *PNEW, const double *C, int it, int nt,
+                       double *trace, void *stream)
+{
+    if (nt < 0) return set_error(ACX_EINVAL, "ctcs: nt must be >= 0");
+    int rc = check_ctcs(c, POLD, P, PNEW, C);
+    if (!rc && (POLD == P || POLD == PNEW)) rc = set_error(ACX_EINVAL, "ctcs: the three time levels must be distinct");
+    for (int k = 0; k < nt && !rc; ++k) {
+        rc = launch_ctcs(c, POLD, P, PNEW, C, it + k, trace ? trace + k : nullptr, (hipStream_t)stream);
+        double *t = POLD;
+        POLD = P;
+        P = PNEW;
+        PNEW = t;
     }
     return rc;
 }

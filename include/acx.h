@@ -148,6 +148,16 @@ typedef struct acx_ctcs {
 int acx_ctcs_update_f64(const acx_ctcs *c, const double *POLD, const double *P, double *PNEW,
                         const double *C, int it, double *rcv_out, void *stream);
 
+/* nt updates it, it+1, ... with the time levels rotating through the three
+ * arrays (the first reads POLD and P and writes PNEW, the next reads P and
+ * PNEW and writes POLD, ...): the loop of 3d/ctcs/point_source/wave.c:109-121
+ * without waiting for the receiver in each step.  trace (device, nt doubles,
+ * may be NULL) gets P at the receiver before each update; entries stay as
+ * they were when rcv is -1.  Stream-ordered; equals nt calls of
+ * acx_ctcs_update_f64 bit for bit. */
+int acx_ctcs_steps_f64(const acx_ctcs *c, double *POLD, double *P, double *PNEW, const double *C, int it, int nt,
+                       double *trace, void *stream);
+
 /* ---- host-side helpers (no GPU needed) -------------------------------- */
 
 /* Seeded synthetic fields on the host (splitmix64), exact cell averages:

@@ -118,3 +118,62 @@ def test_2d_1d_programs(acx, orc, torch_gpu, n):
     rate = np.log2(errs[0] / errs[1])
     print(f"[case] ctcs {n}: errors {errs[0]:.3e} {errs[1]:.3e} rate {rate:.2f}", flush=True)
     assert 1.8 < rate < 2.2
+
+
+# ---- kernel forms of the 3D update against each other -----------------------------
+
+@pytest.mark.parametrize("n", [(6, 5, 5), (8, 7, 6), (50, 33, 9), (100, 21, 13), (176, 120, 119), (176, 120, 120)])
+@pytest.mark.parametrize("stencil", [1, 2])
+def test_update_forms_agree_bit_for_bit(n, stencil, acx, torch_gpu):
+    """Aligned arrays with an even x extent take the pair kernel (up to 2.5e6
+    cells) or the LDS-DMA march; 8 bytes off alignment the register march."""
+    torch = torch_gpu
+    gen = torch.Generator("cuda").manual_seed(11)
+    N = n[0] * n[1] * n[2]
+
+    def arrays(off):
+        return [torch.empty(N + off, dtype=torch.float64, device="cuda")[off:] for _ in range(4)]
+
+    A, B = arrays(0), arrays(1)
+    for a, b in zip(A, B):
+        a.copy_(torch.randn(N, dtype=torch.float64, device="cuda", generator=gen))
+        b.copy_(a)
+    p = acx.Ctcs(n=n, dx=0.5, dy=0.4, dz=0.6, dt=1e-3, stencil=stencil, src=(1, 2, 3), rcv=(n[0] - 1, n[1] - 1, 2))
+    print(f"[case] ctcs forms n={n} stencil={stencil}", flush=True)
+    import ctypes
+    for arr in (A, B):
+        r = (ctypes.c_double * 1)()
+        ptr = [ctypes.c_void_p(t.data_ptr()) for t in arr]
+        acx._check(acx.lib().acx_ctcs_update_f64(ctypes.byref(p.c_struct()), *ptr, 3, r, acx._stream()))
+        assert r[0] == arr[1].view(n[2], n[1], n[0])[2, n[1] - 1, n[0] - 1].item()
+    assert torch.equal(A[2], B[2])
+
+
+@pytest.mark.parametrize("n", [(24, 20, 18), (25, 20, 18), (30, 22, 1)])
+def test_steps_equal_single_updates(n, acx, torch_gpu):
+    torch = torch_gpu
+    import ctypes
+    N = n[0] * n[1] * n[2]
+    gen = torch.Generator("cuda").manual_seed(12)
+    P = [torch.randn(N, dtype=torch.float64, device="cuda", generator=gen) for _ in range(3)]
+    Q = [t.clone() for t in P]
+    C = torch.rand(N, dtype=torch.float64, device="cuda", generator=gen) + 1.0
+    p = acx.Ctcs(n=n, dt=1e-2, src=(3, 4, 0), rcv=(5, 6, 0)).c_struct()
+    ptr = lambda t: ctypes.c_void_p(t.data_ptr())  # noqa: E731
+    nt = 7
+    trace = torch.zeros(nt, dtype=torch.float64, device="cuda")
+    print(f"[case] ctcs steps n={n}", flush=True)
+    acx._check(acx.lib().acx_ctcs_steps_f64(ctypes.byref(p), *(ptr(t) for t in P), ptr(C), 2, nt, ptr(trace), acx._stream()))
+    want = []
+    a, b, c = Q
+    for k in range(nt):
+        r = (ctypes.c_double * 1)()
+        acx._check(acx.lib().acx_ctcs_update_f64(ctypes.byref(p), ptr(a), ptr(b), ptr(c), ptr(C), 2 + k, r, acx._stream()))
+        want.append(r[0])
+        a, b, c = b, c, a
+    assert trace.tolist() == want
+    assert all(torch.equal(x, y) for x, y in zip(P, Q))
+    # refused: aliased time levels, a negative count
+    L = acx.lib()
+    assert L.acx_ctcs_steps_f64(ctypes.byref(p), ptr(P[0]), ptr(P[0]), ptr(P[2]), ptr(C), 0, 1, None, acx._stream()) == 1
+    assert L.acx_ctcs_steps_f64(ctypes.byref(p), ptr(P[0]), ptr(P[1]), ptr(P[2]), ptr(C), 0, -1, None, acx._stream()) == 1
