@@ -39,7 +39,7 @@ int env_int(const char *name, int dflt)
 // a 32^3 WAVE2 step 34 -> 21 us (8 planes: 8 workgroups; 1 plane: 64), the
 // FP32 step at 384^3 2.57 -> 2.50 ms (77 planes instead of 128); the same
 // chunk as before at 256^3.
-int auto_zc(int ntx, int nty, int nz, int slots, int start)
+int auto_zc(int ntx, int nty, int nz, int slots, int start, double *cost_out)
 {
     int best = nz, prev = 0;
     double best_cost = -1.0;
@@ -55,6 +55,7 @@ int auto_zc(int ntx, int nty, int nz, int slots, int start)
             best = z;
         }
     }
+    if (cost_out) *cost_out = best_cost;
     return best;
 }
 
@@ -185,6 +186,8 @@ static void fill_lin(LinArgs &a, const acx_grid *g)
     a.s = g->c0;
     a.inv48h = 1.0 / (48.0 * g->h);
     a.lapc = g->c0 * g->c0 / (48.0 * g->h * g->h);
+    a.K_s = a.K / a.s;
+    a.invrho_s = a.invrho / a.s;
     a.nf = nonfinite_word_current();
 }
 

@@ -28,19 +28,14 @@ constexpr int ENS_MAXP = 256;
 
 struct EnsConfig { int by, zc; };
 constexpr int ENS_NCONFIG = 8;
-static const EnsConfig kConfigs[ENS_NCONFIG] = {{8, 16}, {8, 32}, {8, 64}, {16, 16}, {16, 32}, {16, 64},
-                                                {8, 128}, {16, 128}};
+static const EnsConfig kConfigs[ENS_NCONFIG] = {{8, 16}, {8, 32}, {8, 64}, {12, 16}, {12, 32}, {12, 64},
+                                                {8, 128}, {12, 128}};
 
-// EPI: EPI_F32C for stages 1-3, EPI_F32CF for the stage that ends the step.
-// Registers capped for 4 waves per SIMD: the final stage with the non-finite
-// watch otherwise takes 133 VGPRs on the 8-row tiles, 3 waves per SIMD, and
-// loses 7 % of the ensemble rate (measured on MI355X).
-template <int BY, int EPI>
-__global__ void __launch_bounds__(ENS_BX *BY) __attribute__((amdgpu_waves_per_eu(4)))
+template <int BY, int STAGE>
+__global__ void __launch_bounds__(ENS_BX *BY) __attribute__((amdgpu_waves_per_eu(BY / 4)))
 k_ensemble(const EnsProblem *__restrict__ probs, int nprob, int total, unsigned *__restrict__ counter, LinArgs base)
 {
-    using Tile = LinTile<float, ACX_ACOUSTIC4, ENS_BX, BY>;
-    __shared__ float lds[2][Tile::NS][BY + 6][ENS_BX + 6];
+    __shared__ typename Tile32<ACX_ACOUSTIC4, BY>::template Shared<STAGE> lds;
     __shared__ int s_item;
     __shared__ int s_first[ENS_MAXP];   // first work item of every problem (ascending)
     const int tid = threadIdx.y * ENS_BX + threadIdx.x;
@@ -75,8 +70,7 @@ k_ensemble(const EnsProblem *__restrict__ probs, int nprob, int total, unsigned 
         a.out2 = base.out2 ? static_cast<float *>(base.out2) + o : nullptr;
         const int x0 = (local % pr.ntx) * ENS_BX, y0 = ((local / pr.ntx) % pr.nty) * BY;
         const int zb = (local / (pr.ntx * pr.nty)) * a.zc;
-        // loads one plane ahead, periodic, results streamed past L2
-        linear_tile<float, ACX_ACOUSTIC4, ENS_BX, BY, EPI, 1, false, true>(a, x0, y0, zb, lds);
+        linear_tile32<ACX_ACOUSTIC4, BY, STAGE, false>(a, x0, y0, zb, lds);
         __syncthreads();   // LDS is reused by the next item
     }
 }
@@ -98,7 +92,7 @@ struct acx_ensemble {
     float *hi[2], *lo[2], *d0, *d1;
     int cur;                           // index of the current (hi, lo)
     int config;
-    int persistent_blocks[2];          // per rows-per-tile variant (8, 16)
+    int persistent_blocks[2];          // per rows-per-tile variant (8, 12)
     hipGraphExec_t graph;
     double graph_dt;
     int graph_config, graph_cur;
@@ -138,12 +132,8 @@ static int ens_launch(acx_ensemble *e, const LinArgs &a, hipStream_t s)
 {
     hipLaunchKernelGGL(k_clear, dim3(1), dim3(1), 0, s, e->d_counter);
     const int nb = e->persistent_blocks[BY == 8 ? 0 : 1];
-    if (a.final_stage)
-        hipLaunchKernelGGL((k_ensemble<BY, EPI_F32CF>), dim3(nb), dim3(ENS_BX, BY), 0, s, e->d_probs, e->nprob,
-                           ens_total(e), e->d_counter, a);
-    else
-        hipLaunchKernelGGL((k_ensemble<BY, EPI_F32C>), dim3(nb), dim3(ENS_BX, BY), 0, s, e->d_probs, e->nprob,
-                           ens_total(e), e->d_counter, a);
+    auto k = a.final_stage ? k_ensemble<BY, F32_LAST> : a.d ? k_ensemble<BY, F32_MID> : k_ensemble<BY, F32_FIRST>;
+    hipLaunchKernelGGL(k, dim3(nb), dim3(ENS_BX, BY), 0, s, e->d_probs, e->nprob, ens_total(e), e->d_counter, a);
     return hip_check(hipGetLastError(), "ensemble launch");
 }
 
@@ -165,9 +155,10 @@ static int ens_stage(acx_ensemble *e, const float *D, float *OUT, float *OUT2, d
     a.invrho = 1.0;
     a.s = 1.0;
     a.inv48h = 1.0 / (48.0 * e->h);
+    a.K_s = a.invrho_s = 1.0;
     a.nf = final_stage ? nonfinite_word_current() : nullptr;   // the step's output is watched
     // bc = periodic (0) from memset
-    return kConfigs[e->config].by == 8 ? ens_launch<8>(e, a, s) : ens_launch<16>(e, a, s);
+    return kConfigs[e->config].by == 8 ? ens_launch<8>(e, a, s) : ens_launch<12>(e, a, s);
 }
 
 static int ens_step(acx_ensemble *e, double dt, hipStream_t s)
@@ -216,18 +207,18 @@ int acx_ensemble_create(int nprob, const int32_t *n, double h, acx_ensemble **ou
         hipMemset(e->hi[0], 0, bytes);
         hipMemset(e->lo[0], 0, bytes);
         e->cur = 0;
-        int dev = 0, cus = 0, b8 = 0, b16 = 0, f8 = 0, f16 = 0;
+        int dev = 0, cus = 0, b8 = 0, b12 = 0, f8 = 0, f12 = 0;
         hipGetDevice(&dev);
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-        // persistent grid: blocks that fit at once, the fewer of the two epilogue kinds
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&b8, k_ensemble<8, EPI_F32C>, ENS_BX * 8, 0);
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&b16, k_ensemble<16, EPI_F32C>, ENS_BX * 16, 0);
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&f8, k_ensemble<8, EPI_F32CF>, ENS_BX * 8, 0);
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&f16, k_ensemble<16, EPI_F32CF>, ENS_BX * 16, 0);
+        // persistent grid: blocks that fit at once, the fewer of the stage kinds (the first has the fewest registers)
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&b8, k_ensemble<8, F32_MID>, ENS_BX * 8, 0);
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&b12, k_ensemble<12, F32_MID>, ENS_BX * 12, 0);
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&f8, k_ensemble<8, F32_LAST>, ENS_BX * 8, 0);
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&f12, k_ensemble<12, F32_LAST>, ENS_BX * 12, 0);
         b8 = f8 < b8 ? f8 : b8;
-        b16 = f16 < b16 ? f16 : b16;
+        b12 = f12 < b12 ? f12 : b12;
         e->persistent_blocks[0] = cus * (b8 > 0 ? b8 : 1);
-        e->persistent_blocks[1] = cus * (b16 > 0 ? b16 : 1);
+        e->persistent_blocks[1] = cus * (b12 > 0 ? b12 : 1);
         rc = ens_layout(e);
     }
     if (rc) {

@@ -22,6 +22,7 @@ struct LinArgs {
     int final_stage;
     double a, b, c;    // epilogue coefficients
     double K, invrho, s, inv48h, lapc;
+    double K_s, invrho_s;   // K / s, 1 / (rho0 s)
     unsigned *nf;      // non-finite watch word (host-mapped; null: no watch)
 };
 
@@ -63,8 +64,9 @@ constexpr size_t sel_buffer_bytes(size_t tiles) { return sel_list_offset(tiles) 
 int launch_cweno_tilemask(const CwArgs &a, const uint8_t *flags, uint8_t *mask, hipStream_t s);
 
 int set_error(int code, const char *fmt, ...);
-// z-chunk of a 2.5D march from the round model (acx_api.hip); CUs of the current device
-int auto_zc(int ntx, int nty, int nz, int slots, int start);
+// z-chunk of a 2.5D march from the round model (acx_api.hip) and its cost in
+// planes; CUs of the current device
+int auto_zc(int ntx, int nty, int nz, int slots, int start, double *cost = nullptr);
 int device_cus();
 // integer tuning knob from the environment (dflt when unset or empty)
 int env_int(const char *name, int dflt);

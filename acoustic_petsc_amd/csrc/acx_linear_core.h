@@ -2,12 +2,13 @@
 // acx_linear.hip for the method); shared by the per-grid kernel and the
 // persistent ensemble kernel.
 #pragma once
+#include <type_traits>
 #include "acx_device.h"
 #include "acx_internal.h"
 
 namespace acx {
 
-template <typename T, int SYS, int BX, int BY>
+template <int SYS, int BX, int BY>
 struct LinTile {
     static constexpr int NV = SYS == ACX_ACOUSTIC4 ? 4 : 2;   // components in memory
     static constexpr int NS = SYS == ACX_ACOUSTIC4 ? 4 : 1;   // components in the stencil
@@ -16,35 +17,93 @@ struct LinTile {
 };
 
 // Epilogue kinds
-// EPI_F32CF: the compensated FP32 stage that ends the step (writes the new
-// HI and LO; p.final_stage is implied), instantiated on its own so that the
-// lead-plane march can keep HI of the last four planes in registers for the
-// epilogue's exact sum instead of loading it again three planes later.
-enum { EPI_RHS = 0, EPI_AXPY = 1, EPI_COMB = 2, EPI_F32C = 3, EPI_F32CF = 4 };
+enum { EPI_RHS = 0, EPI_AXPY = 1, EPI_COMB = 2, EPI_F32C = 3 };
 
-// One tile: columns [x0, x0+BX) x [y0, y0+BY), planes [zb, ze) of the grid
-// described by p (shared by the per-grid kernel and the ensemble kernel).
-// WALLS = false: every axis periodic (no ghost signs, wrap-only index maps).
-// NT: results stored nontemporally (streamed past L2).
-template <typename T, int SYS, int BX, int BY, int EPI, int PF = 2, bool WALLS = true, bool NT = false>
-__device__ __forceinline__ void linear_tile(const LinArgs &p, int x0, int y0, int zb,
-                                            T (&lds)[2][LinTile<T, SYS, BX, BY>::NS][BY + 6][BX + 6])
+// FP32 compensated stages.  One tile: columns [x0, x0+64) x [y0, y0+BY),
+// planes [zb, ze) of the grid described by p (shared by the per-grid kernel and
+// the ensemble kernel).  WALLS = false: every axis periodic (no ghost signs,
+// wrap-only index maps).  STAGE: F32_FIRST no increment D yet; F32_MID reads
+// HI and D, writes the next increment; F32_LAST also reads LO and writes the
+// new (HI, LO).
+//
+// Lead-plane march: at iteration j the plane j is staged in LDS (own column
+// and halo loaded for the same plane index as the neighbouring blocks load
+// those rows as their interior, so shared rows meet in L2), its in-plane
+// (x, y) part of the RHS is formed and kept, and plane j-3, whose
+// z-neighbourhood j-6 .. j is now complete in registers, is finished and
+// stored.
+//
+// The stage moves 32 to 80 bytes per cell and was bound by issue and by waits
+// before it was bound by those bytes: per cell 175 FP32 and 67 move
+// instructions.  Now about 135 and none:
+// - the loop is unrolled by the 8 planes of the register ring, so no plane
+//   ever moves between registers, and a load lands in the register that
+//   keeps its plane;
+// - the sums s_k = q(+k) + q(-k) over the axes are taken before the weights
+//   (the differences of A7 likewise), in units of s/(48 h);
+// - a cell is one 16-byte LDS entry (12 16-byte reads);
+// - results are stored through a buffer descriptor per wavefront row, whose
+//   bound drops the columns past the grid: without a branch around the store
+//   the compiler can count it, and waits for a plane's loads alone instead of
+//   for every load and store before them;
+// - D of the last four planes waits in LDS for the epilogue, which leaves room
+//   for 3 wavefronts per SIMD without spills.
+// Measured at 384^3, us per stage (first, second and third, last) against the
+// register-queue march it replaces: 475 -> 345, 590 -> 520, 857 -> 840 of
+// 279, 418, 697 at the copy's rate; the step 2.51 -> 2.23 ms, at 256^3 0.72 ->
+// 0.66 ms.  Its error against 64-bit steps is lower too (one step of
+// ACOUSTIC4 7.7e-9 -> 7.4e-9, of WAVE2 7.9e-7 -> 7.3e-7).
+enum { F32_FIRST = 0, F32_MID = 1, F32_LAST = 2 };
+
+template <int SYS, int BY>
+struct Tile32 {
+    static constexpr int BX = 64;
+    static constexpr int NV = SYS == ACX_ACOUSTIC4 ? 4 : 2;   // components in memory
+    static constexpr int NS = SYS == ACX_ACOUSTIC4 ? 4 : 1;   // components in the stencil
+    static constexpr int LX = BX + 6, LY = BY + 6;
+    static constexpr int NHALO = 6 * BX + 6 * BY;              // star stencil: no plane corners
+    struct alignas(4 * NS) Entry { float v[NS]; };
+    // the two planes being read and staged, and D of the last four planes of
+    // every column (its own thread's only)
+    struct Lds { Entry q[2][LY][LX]; };
+    struct LdsD : Lds { Cell<float, NV> d[4][BY][BX]; };
+    template <int STAGE> using Shared = typename std::conditional<STAGE == F32_FIRST, Lds, LdsD>::type;
+};
+
+typedef unsigned acx_u32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned acx_u32x2 __attribute__((ext_vector_type(2)));
+
+// Nontemporal store of this lane's cell of a wavefront row: row points at the
+// row's first cell (wave-uniform), bytes bounds the cells that exist.
+template <int NV>
+__device__ __forceinline__ void store_row_nt(float *row, unsigned bytes, const Cell<float, NV> &c)
 {
-    using Tile = LinTile<T, SYS, BX, BY>;
-    constexpr int NV = Tile::NV, NS = Tile::NS;
+    const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(row, 0, (int)bytes, 0x00020000);
+    const int off = (int)__lane_id() * NV * 4;
+    if constexpr (NV == 4)
+        __builtin_amdgcn_raw_buffer_store_b128(
+            acx_u32x4{__float_as_uint(c.v[0]), __float_as_uint(c.v[1]), __float_as_uint(c.v[2]), __float_as_uint(c.v[3])},
+            r, off, 0, 2);
+    else
+        __builtin_amdgcn_raw_buffer_store_b64(acx_u32x2{__float_as_uint(c.v[0]), __float_as_uint(c.v[1])}, r, off, 0, 2);
+}
+
+template <int SYS, int BY, int STAGE, bool WALLS>
+__device__ __forceinline__ void linear_tile32(const LinArgs &p, int x0, int y0, int zb,
+                                              typename Tile32<SYS, BY>::template Shared<STAGE> &lds)
+{
+    using Tile = Tile32<SYS, BY>;
+    constexpr int NV = Tile::NV, NS = Tile::NS, BX = Tile::BX;
+    constexpr bool AC = SYS == ACX_ACOUSTIC4, HAS_D = STAGE != F32_FIRST, LAST = STAGE == F32_LAST;
+    using C = Cell<float, NV>;
     static_assert(BX * BY >= Tile::NHALO, "every halo cell of a plane needs a thread of its own");
 
-    const T *__restrict__ Q = static_cast<const T *>(p.q);
-    const T *__restrict__ D = static_cast<const T *>(p.d);       // F32C: increment added to Q
-    const T *__restrict__ U0 = static_cast<const T *>(p.u0);
-    const T *__restrict__ LO = static_cast<const T *>(p.lo);
-    T *__restrict__ OUT = static_cast<T *>(p.out);
-    T *__restrict__ OUT2 = static_cast<T *>(p.out2);
-
+    const float *__restrict__ Q = static_cast<const float *>(p.q);
+    const float *__restrict__ D = static_cast<const float *>(p.d);
+    const float *__restrict__ LO = static_cast<const float *>(p.lo);
     const int nx = p.nx, ny = p.ny, nz = p.nz;
-    const int tx = threadIdx.x, ty = threadIdx.y, tid = ty * BX + tx;
+    const int tx = threadIdx.x, ty = __builtin_amdgcn_readfirstlane((int)threadIdx.y), tid = ty * BX + tx;
     const int ze = min(zb + p.zc, nz);
-    const bool active = (x0 + tx < nx) && (y0 + ty < ny);
     const size_t plane = (size_t)nx * ny;
     const int bcx = WALLS ? p.bc[0] : 0, bcy = WALLS ? p.bc[1] : 0, bcz = WALLS ? p.bc[2] : 0;
 
@@ -54,298 +113,286 @@ __device__ __forceinline__ void linear_tile(const LinArgs &p, int x0, int y0, in
     const int my = map_axis(y0 + ty, ny, bcy, sgy);
     const size_t col = (size_t)my * nx + mx;
 
-    // halo cell owned by this thread (x halo for rows 0..BY-1, y halo for cols 0..BX-1)
+    // halo cell of this thread (x halo for rows 0..BY-1, y halo for cols
+    // 0..BX-1); threads without one load their own column again
     int hx = -1, hy = -1;
-    size_t hcol = 0;
+    size_t hcol = col;
     float hsx = 1.f, hsy = 1.f;
     if (tid < Tile::NHALO) {
         int t = tid;
         if (t < 6 * BY) {            // x halo: 3 left, 3 right per row
-            int row = t / 6, k = t % 6;
+            const int row = t / 6, k = t % 6;
             hy = row + 3;
             hx = k < 3 ? k : BX + k;  // 0,1,2 | BX+3..BX+5
         } else {
             t -= 6 * BY;
-            int colx = t % BX, k = t / BX;
+            const int colx = t % BX, k = t / BX;
             hx = colx + 3;
             hy = k < 3 ? k : BY + k;
         }
-        int gx = map_axis(x0 + hx - 3, nx, bcx, hsx);
-        int gy = map_axis(y0 + hy - 3, ny, bcy, hsy);
+        const int gx = map_axis(x0 + hx - 3, nx, bcx, hsx);
+        const int gy = map_axis(y0 + hy - 3, ny, bcy, hsy);
         hcol = (size_t)gy * nx + gx;
     }
 
-    auto zmap = [&](int z, float &s) -> size_t {
-        s = 1.f;
-        return (size_t)map_axis(z, nz, bcz, s) * plane;
+    // Byte offsets inside a plane: 32 bits in the all-periodic instantiation
+    // (taken when a plane is below 4 GB), so a load's address is a scalar
+    // base and one register.
+    using Off = typename std::conditional<WALLS, size_t, uint32_t>::type;
+    const Off colb = (Off)(col * NV * 4), hcolb = (Off)(hcol * NV * 4);
+    auto load = [](const float *plane_base, Off o) {
+        return load_cell<float, NV>(reinterpret_cast<const float *>(reinterpret_cast<const char *>(plane_base) + o), 0);
+    };
+    // the plane loaded next, its offset and its ghost sign
+    int zi = 0;
+    size_t zoff = 0;
+    float zs = 1.f;
+    auto seek = [&](int z) {
+        zs = 1.f;
+        zi = map_axis(z, nz, bcz, zs);
+        zoff = (size_t)zi * plane * NV;
+    };
+    auto step = [&](int z) {   // from plane z - 1 to z
+        if constexpr (WALLS) {
+            seek(z);
+        } else {
+            ++zi;
+            zoff = zi == nz ? 0 : zoff + plane * NV;
+            zi = zi == nz ? 0 : zi;
+        }
+    };
+    // this wavefront's row of the results
+    const unsigned row_bytes = y0 + ty < ny ? (unsigned)min(BX, nx - x0) * NV * 4u : 0u;
+    const size_t row0 = (size_t)(y0 + ty) * nx + x0;
+
+    // Rings in registers, slot (plane - zb - 3) & 7; what is live at a time is
+    // less than a ring.
+    C q[8];                 // the column's planes j-6 .. j (HI + D, signed)
+    C hi[8];                // HI of plane j+1 as loaded (F32_LAST: of planes j-3 .. j+1)
+    C d;                    // D of plane j+1 (those of planes j-3 .. j wait in LDS, slot & 3)
+    float xy[8][NS];        // in-plane parts of the RHS of planes j-3 .. j
+    C hq, hd;               // halo cell of plane j+1
+    C lo;                   // F32_LAST: LO of the plane to be finished next
+
+    auto load_column = [&](C &qq, C &dd) {
+        qq = load(Q + zoff, colb);
+        if constexpr (HAS_D) dd = load(D + zoff, colb);
+    };
+    auto load_halo = [&]() {
+        hq = load(Q + zoff, hcolb);
+        if constexpr (HAS_D) hd = load(D + zoff, hcolb);
+    };
+    auto value = [&](const C &a, const C &b, float sx, float sy, float sz) -> C {
+        C c = a;
+        if constexpr (HAS_D) {
+#pragma unroll
+            for (int v = 0; v < NV; ++v) c.v[v] += b.v[v];
+        }
+        if constexpr (WALLS) apply_bc_sign<float, NV>(c, sx, sy, sz);
+        return c;
+    };
+    auto stage = [&](int buf, const C &own) {
+        typename Tile::Entry e;
+#pragma unroll
+        for (int v = 0; v < NS; ++v) e.v[v] = own.v[v];
+        lds.q[buf][ty + 3][tx + 3] = e;
+        if (hx >= 0) {
+            const C h = value(hq, hd, hsx, hsy, zs);
+#pragma unroll
+            for (int v = 0; v < NS; ++v) e.v[v] = h.v[v];
+            lds.q[buf][hy][hx] = e;
+        }
+    };
+    // In-plane part without the centre's share.  The nearest neighbours, which
+    // carry the largest weight, enter as differences from the centre q0 (exact
+    // for smooth data): B7 = s3 - 6 s2 + 15 (s1 - 2 q0) + 10 q0 per axis, L7 =
+    // -s3 + 2 s2 + 49 (s1 - 2 q0) - 2 q0.
+    const float ks = float(p.K_s), rs = float(p.invrho_s);
+    auto in_plane = [&](int buf, const C &q0, float (&o)[NS]) {
+        float a[3];   // A7 sums: u along x plus v along y, p along x, p along y
+        auto ring = [&](int k, float wB, float wA, bool first) {
+            const typename Tile::Entry xp = lds.q[buf][ty + 3][tx + 3 + k], xm = lds.q[buf][ty + 3][tx + 3 - k];
+            const typename Tile::Entry yp = lds.q[buf][ty + 3 + k][tx + 3], ym = lds.q[buf][ty + 3 - k][tx + 3];
+            float s[NS];
+#pragma unroll
+            for (int v = 0; v < NS; ++v)
+                s[v] = k == 1 ? ((xp.v[v] - q0.v[v]) + (xm.v[v] - q0.v[v])) + ((yp.v[v] - q0.v[v]) + (ym.v[v] - q0.v[v]))
+                              : (xp.v[v] + xm.v[v]) + (yp.v[v] + ym.v[v]);
+#pragma unroll
+            for (int v = 0; v < NS; ++v) o[v] = first ? (AC ? s[v] : -s[v]) : fmaf(wB, s[v], o[v]);
+            if constexpr (AC) {
+                const float t[3] = {(xp.v[1] - xm.v[1]) + (yp.v[2] - ym.v[2]), xp.v[0] - xm.v[0], yp.v[0] - ym.v[0]};
+#pragma unroll
+                for (int c = 0; c < 3; ++c) a[c] = first ? t[c] : fmaf(wA, t[c], a[c]);
+            }
+        };
+        // one ring of neighbours in registers at a time
+        ring(3, 1.f, 1.f, true);
+        asm volatile("" ::: "memory");
+        ring(1, AC ? 15.f : 49.f, 37.f, false);
+        asm volatile("" ::: "memory");
+        ring(2, AC ? -6.f : 2.f, -8.f, false);
+        if constexpr (AC) {
+            o[0] = fmaf(-ks, a[0], o[0]);
+            o[1] = fmaf(-rs, a[1], o[1]);
+            o[2] = fmaf(-rs, a[2], o[2]);
+        }
     };
 
-    // Lead-plane march.  At iteration j the plane j is staged in LDS (own
-    // column and halo loaded for the same plane index as the neighbouring
-    // blocks load those rows as their interior, so shared rows meet in L2),
-    // its in-plane (x, y) part of the RHS is formed and queued, and plane
-    // c = j - 3, whose z-neighbourhood c-3..c+3 is now complete in registers,
-    // is finished and stored.
-    //
-    // Loads run PF iterations ahead.  A slot holds the raw loaded words (the
-    // ghost sign and the FP32 increment are applied when the slot is
-    // consumed, so nothing waits on a load at issue time), and the loop is
-    // unrolled PF times so every slot keeps fixed registers while in flight.
-    constexpr int NP = SYS == ACX_ACOUSTIC4 ? 4 : 1;
-    const T inv48h = T(p.inv48h), Kc = T(p.K), irho = T(p.invrho), sLLF = T(p.s);
-    const T lap = T(p.lapc);   // WAVE2: c^2 / (48 h^2)
-    const int jbeg = zb - 3, jend = ze + 2;
-    constexpr bool F32C = EPI == EPI_F32C || EPI == EPI_F32CF;
-    const bool has_d = F32C && D != nullptr;
-    const bool fin_stage = EPI == EPI_F32CF || (EPI == EPI_F32C && p.final_stage);
+    // prologue: planes zb-3 .. zb+2, the in-plane parts of the last three
+    {
+        C dd[6];
+        float sz[6];
+        size_t zo[6];
+        seek(zb - 3);
+#pragma unroll
+        for (int k = 0; k < 6; ++k) {
+            load_column(q[2 + k], dd[k]);
+            sz[k] = zs;
+            zo[k] = zoff;
+            step(zb - 2 + k);
+        }
+        const size_t znext = zoff;
+        const float snext = zs;
+#pragma unroll
+        for (int k = 0; k < 6; ++k) {
+            if (k >= 3) {
+                if constexpr (HAS_D) lds.d[(2 + k) & 3][ty][tx] = dd[k];
+                hi[2 + k] = q[2 + k];
+            }
+            q[2 + k] = value(q[2 + k], dd[k], sgx, sgy, sz[k]);
+        }
+#pragma unroll
+        for (int k = 3; k < 6; ++k) {
+            asm volatile("" ::: "memory");   // no later load earlier: the prologue's registers set the kernel's
+            zoff = zo[k];
+            zs = sz[k];
+            load_halo();
+            stage(k & 1, q[2 + k]);
+            __syncthreads();
+            in_plane(k & 1, q[2 + k], xy[2 + k]);
+        }
+        asm volatile("" ::: "memory");
+        zoff = znext;
+        zs = snext;
+        load_column(hi[0], d);
+        load_halo();
+        if constexpr (LAST) lo = load_cell_nt<float, NV>(LO, (size_t)zb * plane + col);
+    }
 
-    struct Slot {
-        Cell<T, NV> q, d, hq, hd, e0, e1, e2;
-        float zs;
-    };
-    Slot sl[PF];
+    // epilogue factors: the RHS in units of s/(48 h) (WAVE2: c^2/(48 h^2))
+    // in two floats: rounded to one, a factor shifts every step the same way
+    const double ccd = AC ? p.c * p.inv48h * p.s : p.c * p.lapc;
+    const float cc = float(ccd), ccl = float(ccd - cc), cb = float(p.b), c1 = float(p.c), c1l = float(p.c - c1);
+    const bool active = tx < nx - x0 && y0 + ty < ny;
+    bool nfbad = false;   // non-finite watch of this thread's outputs
 
-    auto issue = [&](Slot &S, int j) {
-        if (j > jend) return;
-        const size_t off = zmap(j, S.zs);
-        S.q = load_cell<T, NV>(Q, off + col);
-        if (has_d) S.d = load_cell<T, NV>(D, off + col);
-        if (hx >= 0 && j >= zb && j < ze) {
-            S.hq = load_cell<T, NV>(Q, off + hcol);
-            if (has_d) S.hd = load_cell<T, NV>(D, off + hcol);
+    // iteration of plane j = zb + 3 + u (mod 8): finishes plane c = j - 3
+    auto body = [&](auto uu, int j) {
+        constexpr int u = decltype(uu)::value, uc = (u + 5) & 7;
+        q[u] = value(hi[u], d, sgx, sgy, zs);
+        if constexpr (HAS_D) lds.d[u & 3][ty][tx] = d;
+        const bool more = j < ze;   // planes ze .. ze+2 serve the z-stencils only
+        if (more) stage(u & 1, q[u]);
+        step(j + 1);
+        load_column(hi[(u + 1) & 7], d);
+        load_halo();
+        if (more) {
+            __syncthreads();
+            in_plane(u & 1, q[u], xy[u]);
+        } else {
+#pragma unroll
+            for (int v = 0; v < NS; ++v) xy[u][v] = 0.f;   // unused; ends the life of plane j-8's
         }
         const int c = j - 3;
-        if (c >= zb && c < ze && active) {
-            const size_t cidx = (size_t)c * plane + col;
-            if constexpr (EPI == EPI_COMB) S.e0 = load_cell<T, NV>(U0, cidx);
-            if constexpr (F32C) {
-                if (fin_stage) {
-                    // LO is read once: streamed past L2 with the nontemporal stores
-                    if constexpr (NT) S.e1 = load_cell_nt<T, NV>(LO, cidx);
-                    else S.e1 = load_cell<T, NV>(LO, cidx);
-                    // HI of plane c, exact (EPI_F32CF: from the register queue)
-                    if constexpr (EPI == EPI_F32C) S.e2 = load_cell<T, NV>(Q, cidx);
-                }
+        const C &zm3 = q[(u + 2) & 7], &zm2 = q[(u + 3) & 7], &zm1 = q[(u + 4) & 7], &q0 = q[uc];
+        const C &zp1 = q[(u + 6) & 7], &zp2 = q[(u + 7) & 7], &zp3 = q[u];
+        C o, dc;
+        if constexpr (HAS_D) dc = lds.d[uc & 3][ty][tx];
+        if constexpr (AC) {
+            float r[4];
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const float s1 = (zp1.v[v] - q0.v[v]) + (zm1.v[v] - q0.v[v]);
+                const float s2 = zp2.v[v] + zm2.v[v], s3 = zp3.v[v] + zm3.v[v];
+                r[v] = xy[uc][v] + fmaf(15.f, s1, fmaf(30.f, q0.v[v], fmaf(-6.f, s2, s3)));
             }
+            auto A = [&](int v) {
+                const float t1 = zp1.v[v] - zm1.v[v], t2 = zp2.v[v] - zm2.v[v], t3 = zp3.v[v] - zm3.v[v];
+                return fmaf(-8.f, t2, fmaf(37.f, t1, t3));
+            };
+            r[0] = fmaf(-ks, A(3), r[0]);
+            r[3] = fmaf(-rs, A(0), r[3]);
+#pragma unroll
+            for (int v = 0; v < 4; ++v) o.v[v] = fmaf(cc, r[v], HAS_D ? fmaf(ccl, r[v], cb * dc.v[v]) : ccl * r[v]);
+        } else {
+            const float s1 = (zp1.v[0] - q0.v[0]) + (zm1.v[0] - q0.v[0]);
+            const float s2 = zp2.v[0] + zm2.v[0], s3 = zp3.v[0] + zm3.v[0];
+            const float r = xy[uc][0] + fmaf(49.f, s1, fmaf(-6.f, q0.v[0], fmaf(2.f, s2, -s3)));
+            const float v = q0.v[1];   // du/dt = v (rhs_function.c:330)
+            o.v[0] = fmaf(c1, v, HAS_D ? fmaf(c1l, v, cb * dc.v[0]) : c1l * v);
+            o.v[1] = fmaf(cc, r, HAS_D ? fmaf(ccl, r, cb * dc.v[1]) : ccl * r);
+        }
+        const size_t out = ((size_t)c * plane + row0) * NV;
+        if constexpr (LAST) {
+            // HI' + LO' = HI + (LO + increment), exact
+            C nh, nl;
+#pragma unroll
+            for (int v = 0; v < NV; ++v) two_sum(hi[uc].v[v], lo.v[v] + o.v[v], nh.v[v], nl.v[v]);
+            store_row_nt<NV>(static_cast<float *>(p.out2) + out, row_bytes, nl);
+            o = nh;
+            lo = load_cell_nt<float, NV>(LO, (size_t)min(c + 1, ze - 1) * plane + col);
+        }
+        store_row_nt<NV>(static_cast<float *>(p.out) + out, row_bytes, o);
+        if constexpr (LAST) {
+            C w = o;
+#pragma unroll
+            for (int v = 0; v < NV; ++v) w.v[v] = active ? o.v[v] : 0.f;
+            finite_acc<float, NV>(nfbad, w);
         }
     };
-
-    Cell<T, NV> qz[7];   // column values of planes j-6 .. j after the push
-    T xyq[4][NP];        // in-plane RHS parts of planes j-3 .. j
-    // F32C: the increment D of planes j-3 .. j, kept from the stencil loads for
-    // the epilogue of plane j-3 (a second load of it three planes later missed L2)
-    Cell<T, NV> dq[F32C ? 4 : 1];
-    // EPI_F32CF: HI of planes j-3 .. j as loaded (before adding D)
-    Cell<T, NV> hq[EPI == EPI_F32CF ? 4 : 1];
-#pragma unroll
-    for (int k = 0; k < (F32C ? 4 : 1); ++k)
-#pragma unroll
-        for (int v = 0; v < NV; ++v) dq[k].v[v] = T(0);
-#pragma unroll
-    for (int k = 0; k < (EPI == EPI_F32CF ? 4 : 1); ++k)
-#pragma unroll
-        for (int v = 0; v < NV; ++v) hq[k].v[v] = T(0);
-#pragma unroll
-    for (int k = 0; k < 7; ++k)
-#pragma unroll
-        for (int v = 0; v < NV; ++v) qz[k].v[v] = T(0);
-#pragma unroll
-    for (int k = 0; k < 4; ++k)
-#pragma unroll
-        for (int v = 0; v < NP; ++v) xyq[k][v] = T(0);
-
-#pragma unroll
-    for (int u = 0; u < PF; ++u) issue(sl[u], jbeg + u);
-
-    bool nfbad = false;   // non-finite watch of this thread's outputs
-    int buf = 0;
-    for (int jb = jbeg; jb <= jend; jb += PF) {
-#pragma unroll
-        for (int u = 0; u < PF; ++u) {
-            const int j = jb + u;
-            if (j > jend) break;
-            Slot &S = sl[u];
-            const bool stage_xy = (j >= zb) && (j < ze);
-            const int c = j - 3;
-            const bool finish = (c >= zb) && (c < ze) && active;
-
-            // consume the slot of plane j
-            Cell<T, NV> cur = S.q;
-            if constexpr (EPI == EPI_F32CF) {
-#pragma unroll
-                for (int k = 0; k < 3; ++k) hq[k] = hq[k + 1];
-                hq[3] = S.q;
-            }
-            if (has_d) {
-#pragma unroll
-                for (int v = 0; v < NV; ++v) cur.v[v] += S.d.v[v];
-                if constexpr (F32C) {
-#pragma unroll
-                    for (int k = 0; k < 3; ++k) dq[k] = dq[k + 1];
-                    dq[3] = S.d;
-                }
-            }
-            if constexpr (WALLS) apply_bc_sign<T, NV>(cur, sgx, sgy, S.zs);
-
-            T nxy[NP];
-#pragma unroll
-            for (int v = 0; v < NP; ++v) nxy[v] = T(0);
-            if (stage_xy) {
-#pragma unroll
-                for (int v = 0; v < NS; ++v) lds[buf][v][ty + 3][tx + 3] = cur.v[v];
-                if (hx >= 0) {
-                    Cell<T, NV> hcur = S.hq;
-                    if (has_d) {
-#pragma unroll
-                        for (int v = 0; v < NV; ++v) hcur.v[v] += S.hd.v[v];
-                    }
-                    if constexpr (WALLS) apply_bc_sign<T, NV>(hcur, hsx, hsy, S.zs);
-#pragma unroll
-                    for (int v = 0; v < NS; ++v) lds[buf][v][hy][hx] = hcur.v[v];
-                }
-                __syncthreads();
-                if constexpr (SYS == ACX_ACOUSTIC4) {
-                    T accB[4], dAx = T(0), dAy = T(0), dAvel = T(0);
-#pragma unroll
-                    for (int v = 0; v < 4; ++v) {
-                        const T *row = &lds[buf][v][ty + 3][tx + 3];
-                        const T q0 = cur.v[v];
-                        const T xm3 = row[-3], xm2 = row[-2], xm1 = row[-1], xp1 = row[1], xp2 = row[2], xp3 = row[3];
-                        const T ym3 = lds[buf][v][ty][tx + 3], ym2 = lds[buf][v][ty + 1][tx + 3];
-                        const T ym1 = lds[buf][v][ty + 2][tx + 3];
-                        const T yp1 = lds[buf][v][ty + 4][tx + 3], yp2 = lds[buf][v][ty + 5][tx + 3];
-                        const T yp3 = lds[buf][v][ty + 6][tx + 3];
-                        accB[v] = stencil_B7(xm3, xm2, xm1, q0, xp1, xp2, xp3) + stencil_B7(ym3, ym2, ym1, q0, yp1, yp2, yp3);
-                        if (v == 0) {
-                            dAx = stencil_A7(xm3, xm2, xm1, xp1, xp2, xp3);
-                            dAy = stencil_A7(ym3, ym2, ym1, yp1, yp2, yp3);
-                        } else if (v == 1) {
-                            dAvel += stencil_A7(xm3, xm2, xm1, xp1, xp2, xp3);
-                        } else if (v == 2) {
-                            dAvel += stencil_A7(ym3, ym2, ym1, yp1, yp2, yp3);
-                        }
-                    }
-                    nxy[0] = sLLF * accB[0] - Kc * dAvel;
-                    nxy[1] = sLLF * accB[1] - irho * dAx;
-                    nxy[2] = sLLF * accB[2] - irho * dAy;
-                    nxy[3] = sLLF * accB[3];
-                } else {
-                    const T *row = &lds[buf][0][ty + 3][tx + 3];
-                    const T q0 = cur.v[0];
-                    nxy[0] = stencil_L7(row[-3], row[-2], row[-1], q0, row[1], row[2], row[3]) +
-                             stencil_L7(lds[buf][0][ty][tx + 3], lds[buf][0][ty + 1][tx + 3], lds[buf][0][ty + 2][tx + 3],
-                                        q0, lds[buf][0][ty + 4][tx + 3], lds[buf][0][ty + 5][tx + 3],
-                                        lds[buf][0][ty + 6][tx + 3]);
-                }
-                buf ^= 1;
-            }
-
-            // push plane j
-#pragma unroll
-            for (int k = 0; k < 6; ++k) qz[k] = qz[k + 1];
-            qz[6] = cur;
-#pragma unroll
-            for (int k = 0; k < 3; ++k)
-#pragma unroll
-                for (int v = 0; v < NP; ++v) xyq[k][v] = xyq[k + 1][v];
-#pragma unroll
-            for (int v = 0; v < NP; ++v) xyq[3][v] = nxy[v];
-
-            if (finish) {
-                // z part of plane c from qz[0..6] = planes c-3..c+3
-                const size_t cidx = (size_t)c * plane + col;
-                Cell<T, NV> r;
-                if constexpr (SYS == ACX_ACOUSTIC4) {
-                    T bz[4];
-#pragma unroll
-                    for (int v = 0; v < 4; ++v)
-                        bz[v] = stencil_B7(qz[0].v[v], qz[1].v[v], qz[2].v[v], qz[3].v[v], qz[4].v[v], qz[5].v[v],
-                                           qz[6].v[v]);
-                    const T azp = stencil_A7(qz[0].v[0], qz[1].v[0], qz[2].v[0], qz[4].v[0], qz[5].v[0], qz[6].v[0]);
-                    const T azw = stencil_A7(qz[0].v[3], qz[1].v[3], qz[2].v[3], qz[4].v[3], qz[5].v[3], qz[6].v[3]);
-                    r.v[0] = inv48h * (xyq[0][0] + sLLF * bz[0] - Kc * azw);
-                    r.v[1] = inv48h * (xyq[0][1] + sLLF * bz[1]);
-                    r.v[2] = inv48h * (xyq[0][2] + sLLF * bz[2]);
-                    r.v[3] = inv48h * (xyq[0][3] + sLLF * bz[3] - irho * azp);
-                } else {
-                    r.v[0] = qz[3].v[1];     // du/dt = v (rhs_function.c:330)
-                    r.v[1] = lap * (xyq[0][0] + stencil_L7(qz[0].v[0], qz[1].v[0], qz[2].v[0], qz[3].v[0], qz[4].v[0],
-                                                           qz[5].v[0], qz[6].v[0]));
-                }
-                Cell<T, NV> o;
-                if constexpr (EPI == EPI_RHS) {
-                    o = r;
-                } else if constexpr (EPI == EPI_AXPY) {
-                    const T cc = T(p.c);
-#pragma unroll
-                    for (int v = 0; v < NV; ++v) o.v[v] = qz[3].v[v] + cc * r.v[v];
-                } else if constexpr (EPI == EPI_COMB) {
-                    const T aa = T(p.a), bb = T(p.b), cc = T(p.c);
-#pragma unroll
-                    for (int v = 0; v < NV; ++v) o.v[v] = aa * S.e0.v[v] + bb * qz[3].v[v] + cc * r.v[v];
-                } else {
-                    // compensated FP32: increments relative to the step's base (HI + LO)
-                    const T bb = T(p.b), cc = T(p.c);
-#pragma unroll
-                    for (int v = 0; v < NV; ++v) o.v[v] = (has_d ? bb * dq[0].v[v] : T(0)) + cc * r.v[v];
-                    if (fin_stage) {
-                        Cell<T, NV> nh, nl;
-#pragma unroll
-                        for (int v = 0; v < NV; ++v) {
-                            const float hi = (float)(EPI == EPI_F32CF ? hq[0].v[v] : S.e2.v[v]);
-                            const float t = (float)S.e1.v[v] + (float)o.v[v];
-                            float sm, er;
-                            two_sum(hi, t, sm, er);
-                            nh.v[v] = sm;
-                            nl.v[v] = er;
-                        }
-                        if constexpr (NT) store_cell_nt<T, NV>(OUT2, cidx, nl);
-                        else store_cell<T, NV>(OUT2, cidx, nl);
-                        o = nh;
-                    }
-                }
-                if (p.nf) finite_acc<T, NV>(nfbad, o);
-                if constexpr (NT) store_cell_nt<T, NV>(OUT, cidx, o);
-                else store_cell<T, NV>(OUT, cidx, o);
-            }
-            issue(S, j + PF);   // refill this slot for plane j + PF
-        }
+    const int jend = ze + 2;
+    for (int j = zb + 3;; j += 8) {
+        body(std::integral_constant<int, 0>{}, j);
+        if (j + 1 > jend) break;
+        body(std::integral_constant<int, 1>{}, j + 1);
+        if (j + 2 > jend) break;
+        body(std::integral_constant<int, 2>{}, j + 2);
+        if (j + 3 > jend) break;
+        body(std::integral_constant<int, 3>{}, j + 3);
+        if (j + 4 > jend) break;
+        body(std::integral_constant<int, 4>{}, j + 4);
+        if (j + 5 > jend) break;
+        body(std::integral_constant<int, 5>{}, j + 5);
+        if (j + 6 > jend) break;
+        body(std::integral_constant<int, 6>{}, j + 6);
+        if (j + 7 > jend) break;
+        body(std::integral_constant<int, 7>{}, j + 7);
+        if (j + 8 > jend) break;
     }
     watch_flush(p.nf, nfbad);
 }
 
-// Centre-plane march of the same tile: the own column's z-queue holds planes
-// z-3 .. z+3 before plane z is computed, and plane z (with its x/y halo) is
-// staged in LDS and finished in the same iteration.  Fewer live registers
-// than the lead-plane march (no queue of in-plane parts), at the price of
-// halo loads one plane ahead of the neighbours' interior loads.  The column
-// (4 planes ahead) and halo (1 plane ahead) loads keep their raw words until
-// the end of the iteration, so their latency overlaps the iteration's work.
-// NT: epilogue operands and results stream past L2 (nontemporal), leaving L2
-// to the stage input that neighbouring tiles re-read as halo.
-//
-// NB = 2: the plane is staged in a double buffer and its halo is loaded one
-// plane ahead.  NB = 5 (halo ring): the halo of plane z+4 is loaded together
-// with the column's plane z+4, i.e. at the iteration in which the
+// Centre-plane march (FP64): the own column's z-queue holds planes z-3 .. z+3
+// before plane z is computed, and plane z (with its x/y halo) is staged in LDS
+// and finished in the same iteration.  The halo of plane z+4 is loaded
+// together with the column's plane z+4, i.e. at the iteration in which the
 // neighbouring tiles load those cells as their interior, so the shared rows
 // are still in L2; it waits in its slot of a 5-plane LDS ring until plane z+4
-// is computed.
-template <typename T, int SYS, int BX, int BY, int EPI, bool LATE_EPI, bool WALLS, bool NT, int NB>
+// is computed.  Epilogue operands and results stream past L2 (nontemporal),
+// leaving L2 to the stage input that neighbouring tiles re-read as halo.
+template <int SYS, int BX, int BY, int EPI, bool WALLS>
 __device__ __forceinline__ void linear_tile_centre(const LinArgs &p, int x0, int y0, int zb,
-                                                   T (&lds)[NB][LinTile<T, SYS, BX, BY>::NS][BY + 6][BX + 6])
+                                                   double (&lds)[5][LinTile<SYS, BX, BY>::NS][BY + 6][BX + 6])
 {
-    static_assert(NB == 2 || NB == 5, "double buffer or 5-plane halo ring");
-    constexpr bool HRING = NB == 5;
-    using Tile = LinTile<T, SYS, BX, BY>;
+    using Tile = LinTile<SYS, BX, BY>;
     constexpr int NV = Tile::NV, NS = Tile::NS;
+    using C = Cell<double, NV>;
     static_assert(BX * BY >= Tile::NHALO, "every halo cell of a plane needs a thread of its own");
 
-    const T *__restrict__ Q = static_cast<const T *>(p.q);
-    const T *__restrict__ D = static_cast<const T *>(p.d);
-    const T *__restrict__ U0 = static_cast<const T *>(p.u0);
-    const T *__restrict__ LO = static_cast<const T *>(p.lo);
-    T *__restrict__ OUT = static_cast<T *>(p.out);
-    T *__restrict__ OUT2 = static_cast<T *>(p.out2);
+    const double *__restrict__ Q = static_cast<const double *>(p.q);
+    const double *__restrict__ U0 = static_cast<const double *>(p.u0);
+    double *__restrict__ OUT = static_cast<double *>(p.out);
 
     const int nx = p.nx, ny = p.ny, nz = p.nz;
     const int tx = threadIdx.x, ty = threadIdx.y, tid = ty * BX + tx;
@@ -353,9 +400,6 @@ __device__ __forceinline__ void linear_tile_centre(const LinArgs &p, int x0, int
     const bool active = (x0 + tx < nx) && (y0 + ty < ny);
     const size_t plane = (size_t)nx * ny;
     const int bcx = WALLS ? p.bc[0] : 0, bcy = WALLS ? p.bc[1] : 0, bcz = WALLS ? p.bc[2] : 0;
-    constexpr bool F32C = EPI == EPI_F32C || EPI == EPI_F32CF;
-    const bool has_d = F32C && D != nullptr;
-    const bool fin_stage = EPI == EPI_F32CF || (EPI == EPI_F32C && p.final_stage);
 
     float sgx = 1.f, sgy = 1.f;
     const int mx = map_axis(x0 + tx, nx, bcx, sgx);
@@ -381,56 +425,40 @@ __device__ __forceinline__ void linear_tile_centre(const LinArgs &p, int x0, int
         int gy = map_axis(y0 + hy - 3, ny, bcy, hsy);
         hcol = (size_t)gy * nx + gx;
     }
-    auto zmap = [&](int z, float &s) -> size_t {
-        s = 1.f;
-        return (size_t)map_axis(z, nz, bcz, s) * plane;
-    };
     struct Raw {
-        Cell<T, NV> q, d;
+        C q;
         float s;
     };
     auto issue = [&](Raw &r, size_t c, int z) {
-        const size_t off = zmap(z, r.s);
-        r.q = load_cell<T, NV>(Q, off + c);
-        if (has_d) r.d = load_cell<T, NV>(D, off + c);
+        r.s = 1.f;
+        r.q = load_cell<double, NV>(Q, (size_t)map_axis(z, nz, bcz, r.s) * plane + c);
     };
-    auto apply = [&](const Raw &r, float sx, float sy) -> Cell<T, NV> {
-        Cell<T, NV> c = r.q;
-        if (has_d) {
-#pragma unroll
-            for (int v = 0; v < NV; ++v) c.v[v] += r.d.v[v];
-        }
-        if constexpr (WALLS) apply_bc_sign<T, NV>(c, sx, sy, r.s);
+    auto apply = [&](const Raw &r, float sx, float sy) -> C {
+        C c = r.q;
+        if constexpr (WALLS) apply_bc_sign<double, NV>(c, sx, sy, r.s);
         return c;
     };
 
-    Cell<T, NV> qz[7];
+    C qz[7];
 #pragma unroll
     for (int d = -3; d <= 3; ++d) {
         Raw r;
         issue(r, col, zb + d);
         qz[d + 3] = apply(r, sgx, sgy);
     }
-    Cell<T, NV> hv;
-    if constexpr (HRING) {
-        // halos of planes zb .. zb+3 into ring slots 0..3 (visible after the
-        // first barrier of the march)
-        if (hx >= 0) {
+    // halos of planes zb .. zb+3 into ring slots 0..3 (visible after the
+    // first barrier of the march)
+    if (hx >= 0) {
 #pragma unroll
-            for (int d = 0; d < 4; ++d) {
-                if (zb + d < ze) {
-                    Raw r;
-                    issue(r, hcol, zb + d);
-                    const Cell<T, NV> c = apply(r, hsx, hsy);
+        for (int d = 0; d < 4; ++d) {
+            if (zb + d < ze) {
+                Raw r;
+                issue(r, hcol, zb + d);
+                const C c = apply(r, hsx, hsy);
 #pragma unroll
-                    for (int v = 0; v < NS; ++v) lds[d][v][hy][hx] = c.v[v];
-                }
+                for (int v = 0; v < NS; ++v) lds[d][v][hy][hx] = c.v[v];
             }
         }
-    } else if (hx >= 0) {
-        Raw r;
-        issue(r, hcol, zb);
-        hv = apply(r, hsx, hsy);
     }
     // Drain the prologue loads before the march.  Otherwise the queue and
     // halo registers enter the loop as pending load targets, and the
@@ -438,51 +466,34 @@ __device__ __forceinline__ void linear_tile_centre(const LinArgs &p, int x0, int
     // wait for its own 4-planes-ahead prefetch before the barrier.
     __builtin_amdgcn_s_waitcnt(0);
 
-    const T inv48h = T(p.inv48h), Kc = T(p.K), irho = T(p.invrho), sLLF = T(p.s);
-    const T lap = T(p.lapc);
+    const double inv48h = p.inv48h, Kc = p.K, irho = p.invrho, sLLF = p.s, lap = p.lapc;
 
-    bool nfbad = false;               // non-finite watch of this thread's outputs
-    int buf = 0;                      // slot of plane z
-    int hslot = HRING ? 4 : 0;        // ring slot of plane z + 4
+    bool nfbad = false;   // non-finite watch of this thread's outputs
+    int buf = 0;          // slot of plane z
+    int hslot = 4;        // slot of plane z + 4
     for (int z = zb; z < ze; ++z) {
-        // column plane z+4; halo plane z+4 (ring) or z+1
+        // column and halo of plane z+4
         Raw cq, ch;
         issue(cq, col, z + 4);
-        if (HRING ? (hx >= 0 && z + 4 < ze) : (hx >= 0)) issue(ch, hcol, HRING ? z + 4 : z + 1);
+        if (hx >= 0 && z + 4 < ze) issue(ch, hcol, z + 4);
         const size_t idx = (size_t)z * plane + col;
-        Cell<T, NV> e0, e1, e2;
-        auto epi_loads = [&]() {
-            if constexpr (EPI == EPI_COMB) e0 = NT ? load_cell_nt<T, NV>(U0, idx) : load_cell<T, NV>(U0, idx);
-            if constexpr (F32C) {
-                if (has_d) e0 = load_cell<T, NV>(D, idx);
-                if (fin_stage) {
-                    e1 = load_cell<T, NV>(LO, idx);
-                    e2 = load_cell<T, NV>(Q, idx);
-                }
-            }
-        };
-        // epilogue operands: issued with the plane loads, or just before use
-        // (fewer live registers across the stencil)
-        if (!LATE_EPI && active) epi_loads();
+        C e0;
+        if constexpr (EPI == EPI_COMB) { if (active) e0 = load_cell_nt<double, NV>(U0, idx); }
 #pragma unroll
         for (int v = 0; v < NS; ++v) lds[buf][v][ty + 3][tx + 3] = qz[3].v[v];
-        if (!HRING && hx >= 0) {
-#pragma unroll
-            for (int v = 0; v < NS; ++v) lds[buf][v][hy][hx] = hv.v[v];
-        }
         __syncthreads();
-        Cell<T, NV> r;
+        C r;
         if constexpr (SYS == ACX_ACOUSTIC4) {
-            T accB[4], dAp[3], dAvel = T(0);
+            double accB[4], dAp[3], dAvel = 0.0;
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
-                const T *row = &lds[buf][v][ty + 3][tx + 3];
-                const T xm3 = row[-3], xm2 = row[-2], xm1 = row[-1], xp1 = row[1], xp2 = row[2], xp3 = row[3];
-                const T ym3 = lds[buf][v][ty][tx + 3], ym2 = lds[buf][v][ty + 1][tx + 3];
-                const T ym1 = lds[buf][v][ty + 2][tx + 3];
-                const T yp1 = lds[buf][v][ty + 4][tx + 3], yp2 = lds[buf][v][ty + 5][tx + 3];
-                const T yp3 = lds[buf][v][ty + 6][tx + 3];
-                const T q0 = qz[3].v[v];
+                const double *row = &lds[buf][v][ty + 3][tx + 3];
+                const double xm3 = row[-3], xm2 = row[-2], xm1 = row[-1], xp1 = row[1], xp2 = row[2], xp3 = row[3];
+                const double ym3 = lds[buf][v][ty][tx + 3], ym2 = lds[buf][v][ty + 1][tx + 3];
+                const double ym1 = lds[buf][v][ty + 2][tx + 3];
+                const double yp1 = lds[buf][v][ty + 4][tx + 3], yp2 = lds[buf][v][ty + 5][tx + 3];
+                const double yp3 = lds[buf][v][ty + 6][tx + 3];
+                const double q0 = qz[3].v[v];
                 accB[v] = stencil_B7(xm3, xm2, xm1, q0, xp1, xp2, xp3) + stencil_B7(ym3, ym2, ym1, q0, yp1, yp2, yp3) +
                           stencil_B7(qz[0].v[v], qz[1].v[v], qz[2].v[v], q0, qz[4].v[v], qz[5].v[v], qz[6].v[v]);
                 if (v == 0) {
@@ -502,9 +513,9 @@ __device__ __forceinline__ void linear_tile_centre(const LinArgs &p, int x0, int
             r.v[2] = inv48h * (sLLF * accB[2] - irho * dAp[1]);
             r.v[3] = inv48h * (sLLF * accB[3] - irho * dAp[2]);
         } else {
-            const T *row = &lds[buf][0][ty + 3][tx + 3];
-            const T q0 = qz[3].v[0];
-            const T L = stencil_L7(row[-3], row[-2], row[-1], q0, row[1], row[2], row[3]) +
+            const double *row = &lds[buf][0][ty + 3][tx + 3];
+            const double q0 = qz[3].v[0];
+            const double L = stencil_L7(row[-3], row[-2], row[-1], q0, row[1], row[2], row[3]) +
                         stencil_L7(lds[buf][0][ty][tx + 3], lds[buf][0][ty + 1][tx + 3], lds[buf][0][ty + 2][tx + 3], q0,
                                    lds[buf][0][ty + 4][tx + 3], lds[buf][0][ty + 5][tx + 3], lds[buf][0][ty + 6][tx + 3]) +
                         stencil_L7(qz[0].v[0], qz[1].v[0], qz[2].v[0], q0, qz[4].v[0], qz[5].v[0], qz[6].v[0]);
@@ -513,58 +524,34 @@ __device__ __forceinline__ void linear_tile_centre(const LinArgs &p, int x0, int
         }
 
         if (active) {
-            if (LATE_EPI) epi_loads();
-            Cell<T, NV> o;
+            C o;
             if constexpr (EPI == EPI_RHS) {
                 o = r;
             } else if constexpr (EPI == EPI_AXPY) {
-                const T cc = T(p.c);
+                const double cc = p.c;
 #pragma unroll
                 for (int v = 0; v < NV; ++v) o.v[v] = qz[3].v[v] + cc * r.v[v];
-            } else if constexpr (EPI == EPI_COMB) {
-                const T aa = T(p.a), bb = T(p.b), cc = T(p.c);
+            } else {
+                const double aa = p.a, bb = p.b, cc = p.c;
 #pragma unroll
                 for (int v = 0; v < NV; ++v) o.v[v] = aa * e0.v[v] + bb * qz[3].v[v] + cc * r.v[v];
-            } else {
-                const T bb = T(p.b), cc = T(p.c);
-#pragma unroll
-                for (int v = 0; v < NV; ++v) o.v[v] = (has_d ? bb * e0.v[v] : T(0)) + cc * r.v[v];
-                if (fin_stage) {
-                    Cell<T, NV> nh, nl;
-#pragma unroll
-                    for (int v = 0; v < NV; ++v) {
-                        const float t = (float)e1.v[v] + (float)o.v[v];
-                        float sm, er;
-                        two_sum((float)e2.v[v], t, sm, er);
-                        nh.v[v] = sm;
-                        nl.v[v] = er;
-                    }
-                    store_cell<T, NV>(OUT2, idx, nl);
-                    o = nh;
-                }
             }
-            if (p.nf) finite_acc<T, NV>(nfbad, o);
-            if constexpr (NT) store_cell_nt<T, NV>(OUT, idx, o);
-            else store_cell<T, NV>(OUT, idx, o);
+            if (p.nf) finite_acc<double, NV>(nfbad, o);
+            store_cell_nt<double, NV>(OUT, idx, o);
         }
 
 #pragma unroll
         for (int k = 0; k < 6; ++k) qz[k] = qz[k + 1];
         qz[6] = apply(cq, sgx, sgy);
-        if constexpr (HRING) {
-            // slot of plane z+4 = slot of plane z-1, whose readers all passed
-            // this iteration's barrier
-            if (hx >= 0 && z + 4 < ze) {
-                const Cell<T, NV> c = apply(ch, hsx, hsy);
+        // slot of plane z+4 = slot of plane z-1, whose readers all passed
+        // this iteration's barrier
+        if (hx >= 0 && z + 4 < ze) {
+            const C h = apply(ch, hsx, hsy);
 #pragma unroll
-                for (int v = 0; v < NS; ++v) lds[hslot][v][hy][hx] = c.v[v];
-            }
-            buf = buf == NB - 1 ? 0 : buf + 1;
-            hslot = hslot == NB - 1 ? 0 : hslot + 1;
-        } else {
-            if (hx >= 0) hv = apply(ch, hsx, hsy);
-            buf ^= 1;
+            for (int v = 0; v < NS; ++v) lds[hslot][v][hy][hx] = h.v[v];
         }
+        buf = buf == 4 ? 0 : buf + 1;
+        hslot = hslot == 4 ? 0 : hslot + 1;
     }
     watch_flush(p.nf, nfbad);
 }
