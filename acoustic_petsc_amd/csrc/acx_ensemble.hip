@@ -1,13 +1,19 @@
 // acx_ensemble.hip -- persistent-kernel stepping of a batch of independent
 // acoustic problems (include/acx_ensemble.h).
 //
-// Work items are (problem, column tile, z-chunk) triples numbered
-// problem-major; a workgroup takes the next item from an atomic counter,
-// runs the same tile code as the per-grid linear kernel (acx_linear_core.h),
-// and asks again until the queue is empty, so every workgroup exits once the
-// counter passes the item count.  The counter is cleared by a one-thread
-// kernel before every stage (a kernel node, so the step can be captured in a
-// hipGraph).
+// Work items are (problem, column tile, z-chunk) triples.  The schedule of a
+// configuration is made on the host: each XCD gets a contiguous run of the
+// items with an eighth of the work, so that neighbouring tiles meet in its L2,
+// and each workgroup of the XCD a list of them, the longest items handed out
+// first and each to the workgroup with the least so far.  The kernel runs
+// its list with the same tile code as the per-grid linear kernel
+// (acx_linear_core.h).  (A queue per XCD drawn from with atomics cost more
+// than the tiles' differences in speed: at the end of a stage every workgroup
+// finds eight queues empty, 4000 atomics on one line, about 40 us.)
+#include <algorithm>
+#include <exception>
+#include <functional>
+#include <queue>
 #include <stdlib.h>
 #include <string.h>
 #include <vector>
@@ -20,7 +26,12 @@ struct EnsProblem {
     size_t off;          // first cell
     int n[3];
     int ntx, nty, ntz;
-    int first;           // first work item
+    int zc;              // planes per work item
+};
+
+struct EnsItem {
+    int prob;            // index into the problem table
+    int tile;            // column tile and z-chunk, x fastest, then y, then z
 };
 
 constexpr int ENS_BX = 64;
@@ -32,29 +43,16 @@ static const EnsConfig kConfigs[ENS_NCONFIG] = {{8, 16}, {8, 32}, {8, 64}, {12, 
                                                 {8, 128}, {12, 128}};
 
 template <int BY, int STAGE>
-__global__ void __launch_bounds__(ENS_BX *BY) __attribute__((amdgpu_waves_per_eu(BY / 4)))
-k_ensemble(const EnsProblem *__restrict__ probs, int nprob, int total, unsigned *__restrict__ counter, LinArgs base)
+__global__ void __launch_bounds__(ENS_BX *BY) __attribute__((amdgpu_waves_per_eu(STAGE == F32_LAST ? BY / 4 : 4)))
+k_ensemble(const EnsProblem *__restrict__ probs, const EnsItem *__restrict__ items, const int *__restrict__ first,
+           LinArgs base)
 {
     __shared__ typename Tile32<ACX_ACOUSTIC4, BY>::template Shared<STAGE> lds;
-    __shared__ int s_item;
-    __shared__ int s_first[ENS_MAXP];   // first work item of every problem (ascending)
-    const int tid = threadIdx.y * ENS_BX + threadIdx.x;
-    for (int i = tid; i < nprob; i += ENS_BX * BY) s_first[i] = probs[i].first;
-    for (;;) {
-        if (tid == 0) s_item = (int)atomicAdd(counter, 1u);
-        __syncthreads();
-        const int item = s_item;
-        __syncthreads();   // every thread has read s_item before it is overwritten
-        if (item >= total) break;
-        // the problem of the item: the last p with s_first[p] <= item (binary search)
-        int p = 0, hi = nprob - 1;
-        while (p < hi) {
-            const int mid = (p + hi + 1) >> 1;
-            if (s_first[mid] <= item) p = mid;
-            else hi = mid - 1;
-        }
-        const EnsProblem pr = probs[p];
-        const int local = item - pr.first;
+    const int end = first[blockIdx.x + 1];
+    for (int k = first[blockIdx.x]; k < end; ++k) {
+        const EnsItem it = items[k];
+        const EnsProblem pr = probs[it.prob];
+        const int local = it.tile;
         LinArgs a = base;
         a.nx = pr.n[0];
         a.ny = pr.n[1];
@@ -69,13 +67,12 @@ k_ensemble(const EnsProblem *__restrict__ probs, int nprob, int total, unsigned 
         a.out = static_cast<float *>(base.out) + o;
         a.out2 = base.out2 ? static_cast<float *>(base.out2) + o : nullptr;
         const int x0 = (local % pr.ntx) * ENS_BX, y0 = ((local / pr.ntx) % pr.nty) * BY;
+        a.zc = pr.zc;
         const int zb = (local / (pr.ntx * pr.nty)) * a.zc;
         linear_tile32<ACX_ACOUSTIC4, BY, STAGE, false>(a, x0, y0, zb, lds);
         __syncthreads();   // LDS is reused by the next item
     }
 }
-
-__global__ void k_clear(unsigned *c) { *c = 0u; }
 
 } // namespace acx
 
@@ -84,57 +81,157 @@ using namespace acx;
 struct acx_ensemble {
     int nprob;
     double h;
-    std::vector<EnsProblem> probs;      // for the current configuration
+    std::vector<size_t> off;            // first cell of every problem
     std::vector<int> dims;
     size_t ncell;
     EnsProblem *d_probs;
-    unsigned *d_counter;
+    EnsItem *d_items[2];               // schedules of the current configuration: stages 1-3, last stage
+    int *d_first[2];
+    size_t max_items, max_blocks;      // their sizes
     float *hi[2], *lo[2], *d0, *d1;
     int cur;                           // index of the current (hi, lo)
     int config;
-    int persistent_blocks[2];          // per rows-per-tile variant (8, 12)
+    int blocks[2][3];                  // persistent grid per rows-per-tile variant (8, 12) and stage kind
     hipGraphExec_t graph;
     double graph_dt;
     int graph_config, graph_cur;
     hipStream_t graph_stream;
 };
 
-static int ens_layout(acx_ensemble *e)
+// The problems of a configuration: each one's planes divided evenly into
+// chunks of at most the configuration's zc.
+static std::vector<EnsProblem> ens_problems(const acx_ensemble *e, const EnsConfig &c)
 {
-    const EnsConfig c = kConfigs[e->config];
-    int first = 0;
-    size_t off = 0;
-    e->probs.resize(e->nprob);
+    std::vector<EnsProblem> probs(e->nprob);
     for (int p = 0; p < e->nprob; ++p) {
-        EnsProblem &q = e->probs[p];
+        EnsProblem &q = probs[p];
         for (int d = 0; d < 3; ++d) q.n[d] = e->dims[3 * p + d];
-        q.off = off;
+        q.off = e->off[p];
         q.ntx = (q.n[0] + ENS_BX - 1) / ENS_BX;
         q.nty = (q.n[1] + c.by - 1) / c.by;
-        const int zc = c.zc < q.n[2] ? c.zc : q.n[2];
-        q.ntz = (q.n[2] + zc - 1) / zc;
-        q.first = first;
-        first += q.ntx * q.nty * q.ntz;
-        off += (size_t)q.n[0] * q.n[1] * q.n[2];
+        q.ntz = (q.n[2] + c.zc - 1) / c.zc;
+        q.zc = (q.n[2] + q.ntz - 1) / q.ntz;
     }
-    return hip_check(hipMemcpy(e->d_probs, e->probs.data(), sizeof(EnsProblem) * e->nprob, hipMemcpyHostToDevice),
-                     "ensemble table");
+    return probs;
 }
 
-static int ens_total(const acx_ensemble *e)
+static size_t ens_count(const std::vector<EnsProblem> &probs)
 {
-    const EnsProblem &l = e->probs.back();
-    return l.first + l.ntx * l.nty * l.ntz;
+    size_t n = 0;
+    for (const EnsProblem &q : probs) n += (size_t)q.ntx * q.nty * q.ntz;
+    return n;
+}
+
+// Lists of the items per workgroup (blocks b, b + 8, ... run on XCD b % 8);
+// returns the work of the busiest, zc + 10 planes per item.
+static double ens_schedule(const std::vector<EnsProblem> &probs, int blocks, std::vector<EnsItem> &items,
+                           std::vector<int> &first)
+{
+    std::vector<EnsItem> all;
+    double work = 0.0, most = 0.0;
+    for (int p = 0; p < (int)probs.size(); ++p) {
+        const int n = probs[p].ntx * probs[p].nty * probs[p].ntz;
+        for (int t = 0; t < n; ++t) all.push_back({p, t});
+        work += (double)n * (probs[p].zc + 10);
+    }
+    std::vector<std::vector<EnsItem>> list(blocks);
+    size_t k = 0;
+    double done = 0.0;
+    for (int x = 0; x < kNumXcd; ++x) {
+        // this XCD's share of the items, longest first
+        std::vector<EnsItem> part;
+        const double upto = work * (x + 1) / kNumXcd;
+        for (; k < all.size() && (x == kNumXcd - 1 || done + 0.5 * (probs[all[k].prob].zc + 10) < upto); ++k) {
+            part.push_back(all[k]);
+            done += probs[all[k].prob].zc + 10;
+        }
+        std::stable_sort(part.begin(), part.end(),
+                         [&](const EnsItem &a, const EnsItem &b) { return probs[a.prob].zc > probs[b.prob].zc; });
+        using Load = std::pair<double, int>;   // (work so far, workgroup)
+        std::priority_queue<Load, std::vector<Load>, std::greater<Load>> least;
+        for (int b = x; b < blocks; b += kNumXcd) least.push({0.0, b});
+        for (const EnsItem &i : part) {
+            Load l = least.top();
+            least.pop();
+            list[l.second].push_back(i);
+            l.first += probs[i.prob].zc + 10;
+            most = std::max(most, l.first);
+            least.push(l);
+        }
+    }
+    items.clear();
+    first.assign(1, 0);
+    for (const auto &l : list) {
+        items.insert(items.end(), l.begin(), l.end());
+        first.push_back((int)items.size());
+    }
+    return most;
+}
+
+static int ens_layout(acx_ensemble *e)
+try {
+    const EnsConfig &c = kConfigs[e->config];
+    const std::vector<EnsProblem> probs = ens_problems(e, c);
+    int rc = hip_check(hipMemcpy(e->d_probs, probs.data(), sizeof(EnsProblem) * e->nprob, hipMemcpyHostToDevice),
+                       "ensemble table");
+    for (int k = 0; k < 2 && !rc; ++k) {
+        std::vector<EnsItem> items;
+        std::vector<int> first;
+        ens_schedule(probs, e->blocks[c.by == 8 ? 0 : 1][k ? F32_LAST : F32_MID], items, first);
+        rc = hip_check(hipMemcpy(e->d_items[k], items.data(), sizeof(EnsItem) * items.size(), hipMemcpyHostToDevice),
+                       "ensemble schedule");
+        if (!rc)
+            rc = hip_check(hipMemcpy(e->d_first[k], first.data(), sizeof(int) * first.size(), hipMemcpyHostToDevice),
+                           "ensemble schedule");
+    }
+    return rc;
+} catch (const std::exception &x) {
+    return set_error(ACX_EHIP, "ensemble schedule: %s", x.what());
+}
+
+// Configuration until tuned: by the work of the busiest workgroup in the
+// last, longest stage, and three quarters of the longest item for what the
+// workgroups differ in speed (a plane of a 12-row tile takes about 1.3 times
+// as long as one of 8 rows).  us per step, this choice and the best of the
+// eight: 48 problems of 64 .. 160 cells an edge 3444 and 3383, 12 of 64 .. 128
+// 451, 5 330; with the atomic queue and its fixed default 3709, 615, 380.
+static int ens_default_config(const acx_ensemble *e)
+try {
+    int best = 0;
+    double best_t = -1.0;
+    for (int c = 0; c < ENS_NCONFIG; ++c) {
+        std::vector<EnsItem> items;
+        std::vector<int> first;
+        const bool r8 = kConfigs[c].by == 8;
+        const std::vector<EnsProblem> probs = ens_problems(e, kConfigs[c]);
+        int longest = 0;
+        for (const EnsProblem &q : probs) longest = std::max(longest, q.zc);
+        const double t = (ens_schedule(probs, e->blocks[r8 ? 0 : 1][F32_LAST], items, first) + 0.75 * (longest + 10)) *
+                         (r8 ? 1.0 : 1.3);
+        if (best_t < 0 || t < best_t) {
+            best_t = t;
+            best = c;
+        }
+    }
+    return best;
+} catch (const std::exception &) {
+    return 1;   // 8 rows, 32 planes
+}
+
+template <int BY, int STAGE>
+static int ens_launch(const acx_ensemble *e, const LinArgs &a, hipStream_t s)
+{
+    hipLaunchKernelGGL((k_ensemble<BY, STAGE>), dim3(e->blocks[BY == 8 ? 0 : 1][STAGE]), dim3(ENS_BX, BY), 0, s, e->d_probs,
+                       e->d_items[STAGE == F32_LAST], e->d_first[STAGE == F32_LAST], a);
+    return hip_check(hipGetLastError(), "ensemble launch");
 }
 
 template <int BY>
-static int ens_launch(acx_ensemble *e, const LinArgs &a, hipStream_t s)
+static int ens_launch(const acx_ensemble *e, const LinArgs &a, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_clear, dim3(1), dim3(1), 0, s, e->d_counter);
-    const int nb = e->persistent_blocks[BY == 8 ? 0 : 1];
-    auto k = a.final_stage ? k_ensemble<BY, F32_LAST> : a.d ? k_ensemble<BY, F32_MID> : k_ensemble<BY, F32_FIRST>;
-    hipLaunchKernelGGL(k, dim3(nb), dim3(ENS_BX, BY), 0, s, e->d_probs, e->nprob, ens_total(e), e->d_counter, a);
-    return hip_check(hipGetLastError(), "ensemble launch");
+    return a.final_stage ? ens_launch<BY, F32_LAST>(e, a, s)
+           : a.d         ? ens_launch<BY, F32_MID>(e, a, s)
+                         : ens_launch<BY, F32_FIRST>(e, a, s);
 }
 
 static int ens_stage(acx_ensemble *e, const float *D, float *OUT, float *OUT2, double b, double c, int final_stage,
@@ -150,7 +247,6 @@ static int ens_stage(acx_ensemble *e, const float *D, float *OUT, float *OUT2, d
     a.b = b;
     a.c = c;
     a.final_stage = final_stage;
-    a.zc = kConfigs[e->config].zc;
     a.K = 1.0;
     a.invrho = 1.0;
     a.s = 1.0;
@@ -188,15 +284,16 @@ int acx_ensemble_create(int nprob, const int32_t *n, double h, acx_ensemble **ou
     e->h = h;
     e->dims.assign(n, n + 3 * nprob);
     e->ncell = 0;
-    for (int p = 0; p < nprob; ++p) e->ncell += (size_t)n[3 * p] * n[3 * p + 1] * n[3 * p + 2];
-    e->config = 1;   // rows 8, z-chunk 32 until tuned
+    for (int p = 0; p < nprob; ++p) {
+        e->off.push_back(e->ncell);
+        e->ncell += (size_t)n[3 * p] * n[3 * p + 1] * n[3 * p + 2];
+    }
     (void)nonfinite_word();   // the watch word exists before any capture
     e->graph = nullptr;
     e->graph_stream = nullptr;
     const size_t bytes = e->ncell * 4 * sizeof(float);
     int rc = ACX_OK;
     rc = rc ? rc : hip_check(hipMalloc(&e->d_probs, sizeof(EnsProblem) * nprob), "ensemble alloc");
-    rc = rc ? rc : hip_check(hipMalloc(&e->d_counter, sizeof(unsigned)), "ensemble alloc");
     for (int k = 0; k < 2 && !rc; ++k) {
         rc = hip_check(hipMalloc(&e->hi[k], bytes), "ensemble alloc");
         rc = rc ? rc : hip_check(hipMalloc(&e->lo[k], bytes), "ensemble alloc");
@@ -207,19 +304,26 @@ int acx_ensemble_create(int nprob, const int32_t *n, double h, acx_ensemble **ou
         hipMemset(e->hi[0], 0, bytes);
         hipMemset(e->lo[0], 0, bytes);
         e->cur = 0;
-        int dev = 0, cus = 0, b8 = 0, b12 = 0, f8 = 0, f12 = 0;
-        hipGetDevice(&dev);
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-        // persistent grid: blocks that fit at once, the fewer of the stage kinds (the first has the fewest registers)
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&b8, k_ensemble<8, F32_MID>, ENS_BX * 8, 0);
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&b12, k_ensemble<12, F32_MID>, ENS_BX * 12, 0);
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&f8, k_ensemble<8, F32_LAST>, ENS_BX * 8, 0);
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&f12, k_ensemble<12, F32_LAST>, ENS_BX * 12, 0);
-        b8 = f8 < b8 ? f8 : b8;
-        b12 = f12 < b12 ? f12 : b12;
-        e->persistent_blocks[0] = cus * (b8 > 0 ? b8 : 1);
-        e->persistent_blocks[1] = cus * (b12 > 0 ? b12 : 1);
-        rc = ens_layout(e);
+        // persistent grids: the blocks that fit at once
+        auto fit = [](const void *kernel, int by) {
+            int n = 0;
+            if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kernel, ENS_BX * by, 0) != hipSuccess || n < 1) n = 1;
+            return n * device_cus();
+        };
+        e->blocks[0][F32_FIRST] = fit(reinterpret_cast<const void *>(&k_ensemble<8, F32_FIRST>), 8);
+        e->blocks[0][F32_MID] = fit(reinterpret_cast<const void *>(&k_ensemble<8, F32_MID>), 8);
+        e->blocks[0][F32_LAST] = fit(reinterpret_cast<const void *>(&k_ensemble<8, F32_LAST>), 8);
+        e->blocks[1][F32_FIRST] = fit(reinterpret_cast<const void *>(&k_ensemble<12, F32_FIRST>), 12);
+        e->blocks[1][F32_MID] = fit(reinterpret_cast<const void *>(&k_ensemble<12, F32_MID>), 12);
+        e->blocks[1][F32_LAST] = fit(reinterpret_cast<const void *>(&k_ensemble<12, F32_LAST>), 12);
+        for (const EnsConfig &c : kConfigs) e->max_items = std::max(e->max_items, ens_count(ens_problems(e, c)));
+        for (const auto &b : e->blocks) e->max_blocks = std::max(e->max_blocks, (size_t)*std::max_element(b, b + 3));
+        for (int k = 0; k < 2 && !rc; ++k) {
+            rc = hip_check(hipMalloc(&e->d_items[k], sizeof(EnsItem) * e->max_items), "ensemble alloc");
+            rc = rc ? rc : hip_check(hipMalloc(&e->d_first[k], sizeof(int) * (e->max_blocks + 1)), "ensemble alloc");
+        }
+        e->config = ens_default_config(e);
+        rc = rc ? rc : ens_layout(e);
     }
     if (rc) {
         acx_ensemble_destroy(e);
@@ -234,7 +338,10 @@ int acx_ensemble_destroy(acx_ensemble *e)
     if (!e) return ACX_OK;
     if (e->graph) hipGraphExecDestroy(e->graph);
     hipFree(e->d_probs);
-    hipFree(e->d_counter);
+    for (int k = 0; k < 2; ++k) {
+        hipFree(e->d_items[k]);
+        hipFree(e->d_first[k]);
+    }
     for (int k = 0; k < 2; ++k) {
         hipFree(e->hi[k]);
         hipFree(e->lo[k]);
@@ -248,7 +355,7 @@ int acx_ensemble_destroy(acx_ensemble *e)
 int acx_ensemble_offsets(const acx_ensemble *e, size_t *offsets)
 {
     if (!e || !offsets) return set_error(ACX_EINVAL, "ensemble: bad arguments");
-    for (int p = 0; p < e->nprob; ++p) offsets[p] = e->probs[p].off;
+    for (int p = 0; p < e->nprob; ++p) offsets[p] = e->off[p];
     offsets[e->nprob] = e->ncell;
     return ACX_OK;
 }

@@ -114,9 +114,10 @@ __device__ __forceinline__ void linear_tile32(const LinArgs &p, int x0, int y0, 
     const size_t col = (size_t)my * nx + mx;
 
     // halo cell of this thread (x halo for rows 0..BY-1, y halo for cols
-    // 0..BX-1); threads without one load their own column again
-    int hx = -1, hy = -1;
-    size_t hcol = col;
+    // 0..BX-1); threads without one load one cell per wavefront and write it
+    // to the plane's unused corner, so that no branch holds back the loads
+    int hx = 0, hy = 0;
+    size_t hcol = (size_t)__builtin_amdgcn_readfirstlane(my) * nx + __builtin_amdgcn_readfirstlane(mx);
     float hsx = 1.f, hsy = 1.f;
     if (tid < Tile::NHALO) {
         int t = tid;
@@ -178,9 +179,9 @@ __device__ __forceinline__ void linear_tile32(const LinArgs &p, int x0, int y0, 
         qq = load(Q + zoff, colb);
         if constexpr (HAS_D) dd = load(D + zoff, colb);
     };
-    auto load_halo = [&]() {
-        hq = load(Q + zoff, hcolb);
-        if constexpr (HAS_D) hd = load(D + zoff, hcolb);
+    auto load_halo = [&](C &qq, C &dd) {
+        qq = load(Q + zoff, hcolb);
+        if constexpr (HAS_D) dd = load(D + zoff, hcolb);
     };
     auto value = [&](const C &a, const C &b, float sx, float sy, float sz) -> C {
         C c = a;
@@ -191,17 +192,15 @@ __device__ __forceinline__ void linear_tile32(const LinArgs &p, int x0, int y0, 
         if constexpr (WALLS) apply_bc_sign<float, NV>(c, sx, sy, sz);
         return c;
     };
-    auto stage = [&](int buf, const C &own) {
+    auto stage = [&](int buf, const C &own, const C &hq, const C &hd, float zs) {
         typename Tile::Entry e;
 #pragma unroll
         for (int v = 0; v < NS; ++v) e.v[v] = own.v[v];
         lds.q[buf][ty + 3][tx + 3] = e;
-        if (hx >= 0) {
-            const C h = value(hq, hd, hsx, hsy, zs);
+        const C h = value(hq, hd, hsx, hsy, zs);
 #pragma unroll
-            for (int v = 0; v < NS; ++v) e.v[v] = h.v[v];
-            lds.q[buf][hy][hx] = e;
-        }
+        for (int v = 0; v < NS; ++v) e.v[v] = h.v[v];
+        lds.q[buf][hy][hx] = e;
     };
     // In-plane part without the centre's share.  The nearest neighbours, which
     // carry the largest weight, enter as differences from the centre q0 (exact
@@ -239,21 +238,19 @@ __device__ __forceinline__ void linear_tile32(const LinArgs &p, int x0, int y0, 
         }
     };
 
-    // prologue: planes zb-3 .. zb+2, the in-plane parts of the last three
+    // prologue: planes zb-3 .. zb+2 and the halos of the last three all in
+    // flight at once, then plane zb+3, then the in-plane parts
     {
-        C dd[6];
+        C dd[6], ph[3], pd[3];
         float sz[6];
-        size_t zo[6];
         seek(zb - 3);
 #pragma unroll
         for (int k = 0; k < 6; ++k) {
             load_column(q[2 + k], dd[k]);
+            if (k >= 3) load_halo(ph[k - 3], pd[k - 3]);
             sz[k] = zs;
-            zo[k] = zoff;
             step(zb - 2 + k);
         }
-        const size_t znext = zoff;
-        const float snext = zs;
 #pragma unroll
         for (int k = 0; k < 6; ++k) {
             if (k >= 3) {
@@ -262,22 +259,19 @@ __device__ __forceinline__ void linear_tile32(const LinArgs &p, int x0, int y0, 
             }
             q[2 + k] = value(q[2 + k], dd[k], sgx, sgy, sz[k]);
         }
+        load_column(hi[0], d);
+        load_halo(hq, hd);
+        if constexpr (LAST) lo = load_cell_nt<float, NV>(LO, (size_t)zb * plane + col);
 #pragma unroll
         for (int k = 3; k < 6; ++k) {
-            asm volatile("" ::: "memory");   // no later load earlier: the prologue's registers set the kernel's
-            zoff = zo[k];
-            zs = sz[k];
-            load_halo();
-            stage(k & 1, q[2 + k]);
+            stage(k & 1, q[2 + k], ph[k - 3], pd[k - 3], sz[k]);
             __syncthreads();
             in_plane(k & 1, q[2 + k], xy[2 + k]);
+            // formed here, not when it is needed: the neighbours of three
+            // planes at once would set the kernel's registers
+#pragma unroll
+            for (int v = 0; v < NS; ++v) asm volatile("" : "+v"(xy[2 + k][v]));
         }
-        asm volatile("" ::: "memory");
-        zoff = znext;
-        zs = snext;
-        load_column(hi[0], d);
-        load_halo();
-        if constexpr (LAST) lo = load_cell_nt<float, NV>(LO, (size_t)zb * plane + col);
     }
 
     // epilogue factors: the RHS in units of s/(48 h) (WAVE2: c^2/(48 h^2))
@@ -293,10 +287,10 @@ __device__ __forceinline__ void linear_tile32(const LinArgs &p, int x0, int y0, 
         q[u] = value(hi[u], d, sgx, sgy, zs);
         if constexpr (HAS_D) lds.d[u & 3][ty][tx] = d;
         const bool more = j < ze;   // planes ze .. ze+2 serve the z-stencils only
-        if (more) stage(u & 1, q[u]);
+        if (more) stage(u & 1, q[u], hq, hd, zs);
         step(j + 1);
         load_column(hi[(u + 1) & 7], d);
-        load_halo();
+        load_halo(hq, hd);
         if (more) {
             __syncthreads();
             in_plane(u & 1, q[u], xy[u]);

@@ -1,5 +1,5 @@
 """Batched ensemble of independent acoustic problems stepped by one persistent
-kernel over a tile work queue (include/acx_ensemble.h)."""
+kernel over a schedule of tiles (include/acx_ensemble.h)."""
 import ctypes as _C
 
 import numpy as np

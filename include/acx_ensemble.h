@@ -1,15 +1,15 @@
 /*
  * acx_ensemble.h -- a batch of independent 3D acoustic problems stepped by
- * one persistent kernel over a shared tile work queue.
+ * one persistent kernel over a schedule of tiles.
  *
  * No counterpart in the reference (each acoustic_petsc program runs one grid,
  * 3d/weno4/plane_wave/hype.c:102-183).  Every problem is the ACOUSTIC4
  * operator with the shipped linear CWENO4 weights on its own periodic grid
  * (edge lengths may differ per problem and axis, common cell size h), stepped
  * with the compensated FP32 SSP-RK3 of acx_ssp_rks3_step_f32c.  One stage is
- * one launch of a persistent kernel whose workgroups pull (problem, tile,
- * z-chunk) items from an atomic counter; a step (counter resets + 4 stage
- * launches) can be captured once in a hipGraph and replayed.  The result of
+ * one launch of a persistent kernel whose workgroups run lists of (problem,
+ * tile, z-chunk) items made per configuration; a step (4 stage launches) can be
+ * captured once in a hipGraph and replayed.  The result of
  * every problem is bitwise the result of the single-problem FP32 stepper.
  */
 #ifndef ACX_ENSEMBLE_H
