@@ -36,17 +36,6 @@ namespace acx {
 
 enum { EPI_RHS = 0, EPI_AXPY = 1, EPI_COMB = 2, EPI_F32C = 3 };
 
-// Face-averaged values of one component from its axis coefficients.
-__device__ __forceinline__ void face_q(float c0, const Axis3<float> &a, float (&fm)[3], float (&fp)[3])
-{
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-        const float even = c0 + a.c2[d] * float(1.0 / 6.0), odd = 0.5f * a.c1[d] + a.c3[d] * float(1.0 / 20.0);
-        fm[d] = even - odd;
-        fp[d] = even + odd;
-    }
-}
-
 // Flux across a face normal to axis d from left (+face) and right (-face)
 // states: 1/2 (F(Q_L) + F(Q_R) - s (Q_R - Q_L)), F_p = K u_n, F_un = p / rho0.
 __device__ __forceinline__ void face_flux(int d, const float (&L)[4], const float (&R)[4], float K, float irho, float s,
@@ -75,18 +64,22 @@ struct CwLds {
 
 // Waves per SIMD the register allocation aims for.  The selective patch
 // marches a few hundred marked tiles of zc + 2 planes each, and the time of one
-// tile's march is what counts: with 2 waves per SIMD (one block per CU, no
-// spills) against 4 (two blocks per CU, at most 128 VGPRs, 60 spilled), a
-// steep pulse's selective step took 1.146 -> 1.076 ms at 256^3 (232 marked
-// tiles, one round either way) and the same 3.14 ms at 384^3 (508 tiles: two
-// rounds against one).  The full-grid kernel keeps the registers too.
+// tile's march is what counts: one block per CU without spills (2 waves per
+// SIMD) beat two blocks per CU with 60 spilled registers (1.076 against 1.146
+// ms for a steep pulse's step at 256^3, 232 marked tiles, one round either
+// way).  A 256^3 patch is 57 (first stage) to 61 us (last), of which the vector
+// instructions of ten planes issue for about 43; it was 84 us with
+// cweno_weights + cweno_combine, a linear branch of its own and each epilogue
+// load waited for at its place.  The full-grid kernel keeps the registers too.
 template <bool SEL>
 struct CwWaves {
     static constexpr int min_per_simd = SEL ? 2 : 1;
 };
 
 // WALLS = false: every axis periodic (wrap-only index maps, no ghost signs).
-template <bool SEL, bool WALLS>
+// STAGE: F32_FIRST no increment D yet; F32_MID reads D; F32_LAST also adds the
+// step's increment to the state HI + LO.
+template <bool SEL, bool WALLS, int STAGE>
 __global__ void __launch_bounds__(CwLds::BX *CwLds::BY) __attribute__((amdgpu_waves_per_eu(CwWaves<SEL>::min_per_simd)))
 k_cweno(CwArgs p)
 {
@@ -94,6 +87,7 @@ k_cweno(CwArgs p)
     using L = CwLds;
     constexpr int NV = 4, NS = L::NS, BX = L::BX, BY = L::BY, NT = BX * BY;
     constexpr int LX = L::LX, LY = L::LY;
+    constexpr bool HAS_D = STAGE != F32_FIRST, LAST = STAGE == F32_LAST;
     static_assert(BX == 32, "x exchange uses 32-lane row shuffles");
     extern __shared__ __align__(16) unsigned char smem[];
     T(*ring)[NS][LY][LX] = reinterpret_cast<T(*)[NS][LY][LX]>(smem);
@@ -140,60 +134,59 @@ k_cweno(CwArgs p)
         float rsx[PER], rsy[PER];
 #pragma unroll
         for (int r = 0; r < PER; ++r) {
-            const int idx = tid + r * NT;
-            rcol[r] = 0;
+            const int idx = min(tid + r * NT, NREG - 1);
             rsx[r] = rsy[r] = 1.f;
-            if (idx < NREG) {
-                const int lx = idx % LX, ly = idx / LX;
-                rcol[r] = (uint32_t)(map_axis(gy0 - 2 + ly, ny, ky, rsy[r]) * nx + map_axis(gx0 - 2 + lx, nx, kx, rsx[r]));
-            }
+            const int lx = idx % LX, ly = idx / LX;
+            rcol[r] = (uint32_t)(map_axis(gy0 - 2 + ly, ny, ky, rsy[r]) * nx + map_axis(gx0 - 2 + lx, nx, kx, rsx[r]));
         }
-        const bool has_d = D != nullptr;
         auto zoff = [&](int z, float &s) -> size_t {
             s = 1.f;
             return (size_t)map_axis(z, nz, kz, s) * plane;
         };
         auto slot = [](int m) { return ((m % L::NR) + L::NR) % L::NR; };
-        // Plane loads keep the raw words; the FP32 increment and the ghost sign
-        // are applied when the plane is stored, so no wait sits at the load.
+        // Every load of the march is unconditional, on clamped cells and
+        // planes, so that the compiler counts the loads in flight and waits
+        // for the words it needs: loads under a branch were waited for at the
+        // branch's end, one memory latency each and up to four a plane.  Plane
+        // loads keep the raw words; the FP32 increment and the ghost sign are
+        // applied when the plane is stored.
         struct Raw {
-            Cell<T, NV> q, d;
+            Cell<T, NV> q[PER], d[PER];
             float s;
         };
-        auto load_plane = [&](int z, Raw(&buf)[PER]) {
-            float s;
-            const size_t off = zoff(z, s);
+        auto load_plane = [&](int z, Raw &buf) {
+            const size_t off = zoff(z, buf.s);
 #pragma unroll
-            for (int r = 0; r < PER; ++r)
-                if (tid + r * NT < NREG) {
-                    buf[r].q = load_cell<T, NV>(Q, off + rcol[r]);
-                    if (has_d) buf[r].d = load_cell<T, NV>(D, off + rcol[r]);
-                    buf[r].s = s;
-                }
+            for (int r = 0; r < PER; ++r) {
+                buf.q[r] = load_cell<T, NV>(Q, off + rcol[r]);
+                if constexpr (HAS_D) buf.d[r] = load_cell<T, NV>(D, off + rcol[r]);
+            }
         };
-        auto store_plane = [&](int z, const Raw(&buf)[PER]) {
+        auto store_plane = [&](int z, const Raw &buf) {
             const int sl = slot(z);
 #pragma unroll
             for (int r = 0; r < PER; ++r) {
                 const int idx = tid + r * NT;
                 if (idx < NREG) {
-                    Cell<T, NV> c = buf[r].q;
-                    if (has_d) {
+                    Cell<T, NV> c = buf.q[r];
+                    if constexpr (HAS_D) {
 #pragma unroll
-                        for (int v = 0; v < NV; ++v) c.v[v] += buf[r].d.v[v];
+                        for (int v = 0; v < NV; ++v) c.v[v] += buf.d[r].v[v];
                     }
-                    if constexpr (WALLS) apply_bc_sign<T, NV>(c, rsx[r], rsy[r], buf[r].s);
+                    if constexpr (WALLS) apply_bc_sign<T, NV>(c, rsx[r], rsy[r], buf.s);
 #pragma unroll
                     for (int v = 0; v < NS; ++v) ring[sl][v][idx / LX][idx % LX] = c.v[v];
                 }
             }
         };
 
-        // prologue: planes zb-3 .. zb+1
-        for (int z = zb - 3; z <= zb + 1; ++z) {
-            Raw b0[PER];
-            load_plane(z, b0);
-            store_plane(z, b0);
+        // prologue: planes zb-3 .. zb+1, all requested before the first is stored
+        {
+            Raw b0[5];
+#pragma unroll
+            for (int k = 0; k < 5; ++k) load_plane(zb - 3 + k, b0[k]);
+#pragma unroll
+            for (int k = 0; k < 5; ++k) store_plane(zb - 3 + k, b0[k]);
         }
         __syncthreads();
 
@@ -203,41 +196,30 @@ k_cweno(CwArgs p)
         for (int v = 0; v < NS; ++v) { zp_prev[v] = T(0); Fz_prev[v] = T(0); dxy_prev[v] = T(0); }
         const int lx = tx + 2, ly = ty + 2;
 
+        // Plane m+3 is requested in iteration m-1, right after the plane before
+        // it went to LDS, and stored in iteration m.
         uint8_t fl_next = 0xff;
-        // Selective patch: plane m+3 is requested in iteration m-1, right
-        // after the plane before it went to LDS, instead of at the start of
-        // iteration m.  (The compiler waits for these loads together with the
-        // epilogue operands, before the results of iteration m-1 are stored,
-        // so they overlap that iteration's fluxes.)  Measured with one block
-        // per CU on a steep pulse at 256^3, in two runs beside a reference
-        // build that took 1.15-1.16 ms in both: 1.135 -> 1.076 ms per step.
-        Raw nxt_sel[PER];
-        if constexpr (SEL) {
+        Raw nxt;
+        {
             float s;
-            fl_next = p.flags[zoff(zb - 1, s) + ocol];
-            load_plane(zb + 2, nxt_sel);
+            if constexpr (SEL) fl_next = p.flags[zoff(zb - 1, s) + ocol];
+            load_plane(min(zb + 2, ze + 2), nxt);
         }
         for (int m = zb - 1; m <= ze; ++m) {
-            // prefetch plane m+3 of the region, the flags of plane m+1 and the
-            // epilogue operands of plane m-1
-            Raw nxt_full[PER];
-            Raw(&nxt)[PER] = SEL ? nxt_sel : nxt_full;
+            // the flags of plane m+1 and the epilogue operands of plane m-1
             const bool pf = m + 3 <= ze + 2;
-            if (!SEL && pf) load_plane(m + 3, nxt);
             const uint8_t fl = fl_next;
             if constexpr (SEL) {
                 float s;
-                if (m + 1 <= ze) fl_next = p.flags[zoff(m + 1, s) + ocol];
+                fl_next = p.flags[zoff(min(m + 1, ze), s) + ocol];
             }
             const bool fin = m >= zb + 1 && interior;
-            const size_t cell = (size_t)(m - 1) * plane + ocol;
+            const size_t cell = (size_t)max(m - 1, zb) * plane + ocol;
             Cell<T, NV> e0, e1, e2;
-            if (fin) {
-                if (has_d) e0 = load_cell<T, NV>(D, cell);
-                if (p.final_stage) {
-                    e1 = load_cell<T, NV>(LO, cell);
-                    e2 = load_cell<T, NV>(Q, cell);
-                }
+            if constexpr (HAS_D) e0 = load_cell<T, NV>(D, cell);
+            if constexpr (LAST) {
+                e1 = load_cell<T, NV>(LO, cell);
+                e2 = load_cell<T, NV>(Q, cell);
             }
             const int sm2 = slot(m - 2), s0 = slot(m - 1), s1 = slot(m), s2 = slot(m + 1), sp2 = slot(m + 2);
             T fpx[NS], fmx[NS], fpy[NS], fmz[NS], fpz[NS];
@@ -287,18 +269,8 @@ k_cweno(CwArgs p)
                     }
                 };
 
-                Axis3<T> ax;
-                bool full = true;
-                if constexpr (SEL) full = (fl >> v) & 1;
-                if (full) {
-                    cweno_axes_lds<T>(get, p, ax);
-                } else {
-                    axis_linear(get(1), get(2), get(0), get(3), get(4), ax.c1[0], ax.c2[0], ax.c3[0]);
-                    axis_linear(get(5), get(6), get(0), get(7), get(8), ax.c1[1], ax.c2[1], ax.c3[1]);
-                    axis_linear(get(9), get(10), get(0), get(11), get(12), ax.c1[2], ax.c2[2], ax.c3[2]);
-                }
                 T m3[3], p3[3];
-                face_q(get(0), ax, m3, p3);
+                cweno_faces<ACX_ACOUSTIC4, T>(get, p, !SEL || ((fl >> v) & 1), m3, p3);
                 fmx[v] = m3[0]; fpx[v] = p3[0];
                 s_fym[v][ty][tx] = m3[1];
                 fpy[v] = p3[1];
@@ -308,7 +280,7 @@ k_cweno(CwArgs p)
             __syncthreads();   // B1: -y states visible; every read of plane m-1 is done
 
             if (pf) store_plane(m + 3, nxt);   // into the slot of plane m-2
-            if (SEL && m + 4 <= ze + 2) load_plane(m + 4, nxt);
+            load_plane(min(m + 4, ze + 2), nxt);
 
             T Fx[NS], Fy[NS];
             {
@@ -344,8 +316,8 @@ k_cweno(CwArgs p)
                     for (int v = 0; v < 4; ++v) r.v[v] = -ih * (dxy_prev[v] + (Fz[v] - Fz_prev[v]));
                     Cell<T, NV> o;
 #pragma unroll
-                    for (int v = 0; v < NV; ++v) o.v[v] = (has_d ? T(p.b) * e0.v[v] : T(0)) + T(p.c) * r.v[v];
-                    if (p.final_stage) {
+                    for (int v = 0; v < NV; ++v) o.v[v] = (HAS_D ? T(p.b) * e0.v[v] : T(0)) + T(p.c) * r.v[v];
+                    if constexpr (LAST) {
                         Cell<T, NV> nh, nl;
 #pragma unroll
                         for (int v = 0; v < NV; ++v) {
@@ -375,7 +347,7 @@ k_cweno(CwArgs p)
     watch_flush(p.nf, nfbad);
 }
 
-// FP64 stage kernel, bound by FP64 issue (cweno_faces64: about 265 of the 300
+// FP64 stage kernel, bound by FP64 issue (cweno_faces: about 265 of the 300
 // FP64 instructions per cell and component).  A thread reconstructs at most
 // two of the components: an ACOUSTIC4 block is 32 x 12 columns times two halves
 // (waves 0-5 p and u, waves 6-11 v and w), a WAVE2 block 32 x 16 columns on
@@ -583,7 +555,7 @@ k_cweno64(CwArgs p)
                 }
             };
             double fm[3], fp[3];
-            cweno_faces64<SYS>(get, p, fm, fp);
+            cweno_faces<SYS, double>(get, p, true, fm, fp);
             fmx[k] = fm[0]; fpx[k] = fp[0];
             F[k] = AC ? -sL * (fm[2] - zp_prev[k]) : fm[2] + zp_prev[k];
             if constexpr (AC) {
@@ -780,7 +752,7 @@ int launch_cweno_tilemask(const CwArgs &a, const uint8_t *flags, uint8_t *mask, 
     return hip_check(hipGetLastError(), "tile list launch");
 }
 
-template <bool SEL, bool WALLS>
+template <bool SEL, bool WALLS, int STAGE>
 static int launch_cw32_w(const CwArgs &a, hipStream_t s)
 {
     constexpr int BX = CW_BX, BY = CW_BY;
@@ -794,7 +766,7 @@ static int launch_cw32_w(const CwArgs &a, hipStream_t s)
         if (!per_cu) {
             int n = 0;
             if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                    &n, reinterpret_cast<const void *>(&k_cweno<SEL, WALLS>), BX * BY,
+                    &n, reinterpret_cast<const void *>(&k_cweno<SEL, WALLS, STAGE>), BX * BY,
                     CwLds::bytes) != hipSuccess || n <= 0)
                 n = 1;
             per_cu = n;
@@ -809,7 +781,7 @@ static int launch_cw32_w(const CwArgs &a, hipStream_t s)
         if (!per_cu_sel) {
             int n = 0;
             if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                    &n, reinterpret_cast<const void *>(&k_cweno<SEL, WALLS>), BX * BY,
+                    &n, reinterpret_cast<const void *>(&k_cweno<SEL, WALLS, STAGE>), BX * BY,
                     CwLds::bytes) != hipSuccess || n <= 0)
                 n = 1;
             per_cu_sel = n;
@@ -819,7 +791,7 @@ static int launch_cw32_w(const CwArgs &a, hipStream_t s)
     constexpr size_t lds = CwLds::bytes;
     static bool attr_set = false;
     if (!attr_set) {
-        int rc = hip_check(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_cweno<SEL, WALLS>),
+        int rc = hip_check(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_cweno<SEL, WALLS, STAGE>),
                                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds),
                            "k_cweno LDS attribute");
         if (rc) return rc;
@@ -827,7 +799,7 @@ static int launch_cw32_w(const CwArgs &a, hipStream_t s)
     }
     dim3 blk(BX, BY, 1);
     dim3 grd((unsigned)blocks, 1, 1);
-    hipLaunchKernelGGL((k_cweno<SEL, WALLS>), grd, blk, lds, s, b);
+    hipLaunchKernelGGL((k_cweno<SEL, WALLS, STAGE>), grd, blk, lds, s, b);
     return hip_check(hipGetLastError(), "k_cweno launch");
 }
 
@@ -872,9 +844,11 @@ static int launch_cw64_e(const CwArgs &a, hipStream_t s)
 template <bool SEL>
 static int launch_cw32(const CwArgs &a, hipStream_t s)
 {
-    if (a.bc[0] != ACX_PERIODIC || a.bc[1] != ACX_PERIODIC || a.bc[2] != ACX_PERIODIC)
-        return launch_cw32_w<SEL, true>(a, s);
-    return launch_cw32_w<SEL, false>(a, s);
+    const bool walls = a.bc[0] != ACX_PERIODIC || a.bc[1] != ACX_PERIODIC || a.bc[2] != ACX_PERIODIC;
+    if (a.final_stage)
+        return walls ? launch_cw32_w<SEL, true, F32_LAST>(a, s) : launch_cw32_w<SEL, false, F32_LAST>(a, s);
+    if (a.d) return walls ? launch_cw32_w<SEL, true, F32_MID>(a, s) : launch_cw32_w<SEL, false, F32_MID>(a, s);
+    return walls ? launch_cw32_w<SEL, true, F32_FIRST>(a, s) : launch_cw32_w<SEL, false, F32_FIRST>(a, s);
 }
 
 int launch_cweno(const CwArgs &a, int sys, int epi, bool fp32, bool selective, hipStream_t s)

@@ -222,28 +222,18 @@ __device__ __forceinline__ T cweno_axes(const T (&s)[33], const CwArgs &p, Axis3
     return wt;
 }
 
-// Full CWENO4 from values held in LDS, get(q) returning stencil slot q: the
-// weights are formed group by group, then the 13 axis values are read again
-// for the combination (the memory clobbers keep the compiler from holding all
-// 33 values live across the weight arithmetic).
-template <typename T, typename Get>
-__device__ __forceinline__ void cweno_axes_lds(Get get, const CwArgs &p, Axis3<T> &o)
-{
-    T wt, w3[7];
-    cweno_weights<T>(get, p, wt, w3);
-    asm volatile("" ::: "memory");
-    cweno_combine<T>(get(0), get(1), get(2), get(3), get(4), get(5), get(6), get(7), get(8), get(9), get(10),
-                     get(11), get(12), wt, w3, p, o);
-}
-
-// FP64 CWENO4 of one cell and component straight to its six face quantities
+// CWENO4 of one cell and component straight to its six face quantities
 // (ACOUSTIC4: face-averaged values; WAVE2: h times the face-averaged normal
 // gradients), the same scheme as cweno_weights + cweno_combine in far fewer
-// operations.  The stage kernel is bound by FP64 issue, so the operation
-// count is what it costs: about 240 FP64 instructions per cell and component,
-// 3 of them reciprocals, against 515 with 9.  get(q): stencil slots of
+// operations.  The stage kernels are bound by the issue of these operations:
+// about 240 FP64 instructions per cell and component, 3 of them reciprocals,
+// against 515 with 9; in FP32 about 280 with 9 against 515 with 9 (the patch of
+// a 256^3 selective stage 84 -> 66 us).  get(q): stencil slots of
 // cweno_weights.  The memory clobbers keep one group of LDS values live at a
-// time.
+// time.  cweno_faces with full = false (per lane) gives the linear 4th-order
+// polynomial: the same combination with n1 = n2 = 0 and the c3 share alone, so
+// a wavefront with both kinds of lanes runs the common part once (66 -> 58 us
+// with the loads of k_cweno).
 //
 // Per axis, from the first differences e1 .. e4 of m2, m1, u0, p1, p2:
 //   A, B, C = e4-e3, e3-e2, e2-e1 (second), a, c = A-B, B-C (third),
@@ -265,49 +255,43 @@ __device__ __forceinline__ void cweno_axes_lds(Get get, const CwArgs &p, Axis3<T
 //   2 c1  = S - n1 a - n2 c + n4 (g3s - 11/60)/g4 T
 //   2 c2  = B + n1 a - n2 c - n4 g3s/g4 F
 //   12 c3 = n4/g4 T
-// The eight reciprocals 1/IS come from two, each of a product of four IS
-// (in range whenever IS^4 is), each refined to full precision.
-template <int SYS, typename Get>
-__device__ __forceinline__ void cweno_faces64(Get get, const CwArgs &p, double (&fm)[3], double (&fp)[3])
+// In FP64 the eight reciprocals 1/IS come from two, each of a product of four IS
+// (in range whenever IS^4 is), each refined to full precision.  In FP32, where
+// (IS + eps)^4 ~ 1e-48 underflows, the weights are gamma (IS_min / IS)^4.
+template <int SYS, typename T, typename Get>
+__device__ __forceinline__ void cweno_weights4(Get get, const CwArgs &p, const T (&S)[3], const T (&B)[3],
+                                               const T (&a)[3], const T (&c)[3], const T (&e2)[3], const T (&e3)[3],
+                                               const T (&A)[3], const T (&Cc)[3], T (&n)[6], T &is, T &ke, T &ko)
 {
-    const double k13 = 13.0 / 3.0, k7 = 7.0 / 6.0, eps = 4.0e-12;
-    const double u0 = get(0);
-    double S[3], B[3], a[3], c[3];
-    double C[3], P[3], M[3], is4;
+    const T k13 = T(13.0 / 3.0), k7 = T(7.0 / 6.0), eps = T(4.0e-12);
+    T C[3], P[3], M[3], is4;
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
-        const double m2 = get(1 + 4 * d), m1 = get(2 + 4 * d), p1 = get(3 + 4 * d), p2 = get(4 + 4 * d);
-        const double e1 = m1 - m2, e2 = u0 - m1, e3 = p1 - u0, e4 = p2 - p1;
-        const double A = e4 - e3, Cc = e2 - e1;
-        B[d] = e3 - e2;
-        S[d] = e2 + e3;
-        a[d] = A - B[d];
-        c[d] = B[d] - Cc;
-        const double T = a[d] + c[d];
-        const double D1 = fma(2.0, e3, -A), D2 = fma(2.0, e2, Cc);
-        C[d] = fma(S[d], S[d], fma(k13 * B[d], B[d], 0.5 * eps));   // a sum of two carries eps
-        P[d] = fma(D1, D1, (k13 * A) * A);
-        M[d] = fma(D2, D2, (k13 * Cc) * Cc);
-        const double t = fma(S[d], -1.0 / 3.0, 1.1125 * T);
-        is4 = d == 0 ? T * t : fma(T, t, is4);
+        const T G = a[d] + c[d];
+        const T D1 = fma(T(2), e3[d], -A[d]), D2 = fma(T(2), e2[d], Cc[d]);
+        C[d] = fma(S[d], S[d], fma(k13 * B[d], B[d], T(0.5) * eps));   // a sum of two carries eps
+        P[d] = fma(D1, D1, (k13 * A[d]) * A[d]);
+        M[d] = fma(D2, D2, (k13 * Cc[d]) * Cc[d]);
+        const T t = fma(S[d], T(-1.0 / 3.0), T(1.1125) * G);
+        is4 = d == 0 ? G * t : fma(G, t, is4);
     }
-    const double Cyz = C[1] + C[2], Czx = C[2] + C[0], Cxy = C[0] + C[1];
-    double t0 = Cyz + (C[0] - 0.5 * eps);
+    const T Cyz = C[1] + C[2], Czx = C[2] + C[0], Cxy = C[0] + C[1];
+    T t0 = Cyz + (C[0] - T(0.5) * eps);
     is4 += t0;
     asm volatile("" ::: "memory");
     // twice the mixed derivatives of one pair of axes
-    auto pair = [&](int q, double Sa, double Sb, double &al, double &be, double &ph, double &ps, double &m) {
-        const double pp = get(q), pm = get(q + 1), mp = get(q + 2), mm = get(q + 3);
+    auto pair = [&](int q, T Sa, T Sb, T &al, T &be, T &ph, T &ps, T &m) {
+        const T pp = get(q), pm = get(q + 1), mp = get(q + 2), mm = get(q + 3);
         al = (pp - pm) - Sb;
         be = (mp - mm) - Sb;
         ph = (pp - mp) - Sa;
-        const double x = al - be;
+        const T x = al - be;
         ps = ph - x;
         m = x * x;
     };
-    double q[6], Mxy, Myz, Mzx;
+    T q[6], Mxy, Myz, Mzx;
     {
-        double al, be, ph, ps;
+        T al, be, ph, ps;
         pair(13, S[0], S[1], al, be, ph, ps, Mxy);   // (x, y): x+, x-, y+, y-
         q[0] = al * al; q[1] = be * be; q[2] = ph * ph; q[3] = ps * ps;
         asm volatile("" ::: "memory");
@@ -318,51 +302,88 @@ __device__ __forceinline__ void cweno_faces64(Get get, const CwArgs &p, double (
         q[4] = fma(al, al, q[4]); q[5] = fma(be, be, q[5]); q[0] = fma(ph, ph, q[0]); q[1] = fma(ps, ps, q[1]);
     }
     asm volatile("" ::: "memory");
-    const double Ms = (Mxy + Myz) + Mzx;
-    const double Q = ((q[0] + q[1]) + (q[2] + q[3])) + (q[4] + q[5]);
-    t0 = fma(0.25 * k7, Ms, t0);
-    is4 = fma(2.35, Q, is4);
-    is4 = fma(0.25 * k7 - 2.35, Ms, is4);
+    const T Ms = (Mxy + Myz) + Mzx;
+    const T Q = ((q[0] + q[1]) + (q[2] + q[3])) + (q[4] + q[5]);
+    t0 = fma(T(0.25) * k7, Ms, t0);
+    is4 = fma(T(2.35), Q, is4);
+    is4 = fma(T(0.25 * 7.0 / 6.0 - 2.35), Ms, is4);
     {
-        const double z = ((get(25) - get(26)) - (get(27) - get(29))) - ((get(28) - get(30)) - (get(31) - get(32)));
-        is4 = fma((61.0 / 768.0) * z, z, is4);
+        const T z = ((get(25) - get(26)) - (get(27) - get(29))) - ((get(28) - get(30)) - (get(31) - get(32)));
+        is4 = fma(T(61.0 / 768.0) * z, z, is4);
     }
-    const double t1 = fma(k7, fma(0.25, Myz, q[0]), P[0] + Cyz), t2 = fma(k7, fma(0.25, Myz, q[1]), M[0] + Cyz);
-    const double t3 = fma(k7, fma(0.25, Mzx, q[2]), P[1] + Czx), t4 = fma(k7, fma(0.25, Mzx, q[3]), M[1] + Czx);
-    const double t5 = fma(k7, fma(0.25, Mxy, q[4]), P[2] + Cxy), t6 = fma(k7, fma(0.25, Mxy, q[5]), M[2] + Cxy);
+    const T t1 = fma(k7, fma(T(0.25), Myz, q[0]), P[0] + Cyz), t2 = fma(k7, fma(T(0.25), Myz, q[1]), M[0] + Cyz);
+    const T t3 = fma(k7, fma(T(0.25), Mzx, q[2]), P[1] + Czx), t4 = fma(k7, fma(T(0.25), Mzx, q[3]), M[1] + Czx);
+    const T t5 = fma(k7, fma(T(0.25), Mxy, q[4]), P[2] + Cxy), t6 = fma(k7, fma(T(0.25), Mxy, q[5]), M[2] + Cxy);
 
     // gamma / IS^4, p = 4 (reconstruction.c:205-218)
-    auto inv4 = [](double &w, double &x, double &y, double &z) {
-        const double wx = w * x, yz = y * z;
-        const double r = rcp64_full(wx * yz);
-        const double rwx = r * yz, ryz = r * wx;
-        const double iw = rwx * x, ix = rwx * w, iy = ryz * z, iz = ryz * y;
-        w = iw; x = ix; y = iy; z = iz;
-    };
-    double r4 = is4, r0 = t0, r1 = t1, r2 = t2, r3 = t3, r5 = t4, r6 = t5, r7 = t6;
-    inv4(r4, r0, r1, r2);
-    inv4(r3, r5, r6, r7);
-    auto pow4 = [](double r) { const double r2 = r * r; return r2 * r2; };
-    double w4 = p.g4 * pow4(r4);
-    double n[6] = {pow4(r1), pow4(r2), pow4(r3), pow4(r5), pow4(r6), pow4(r7)};
-    const double sided = ((n[0] + n[1]) + (n[2] + n[3])) + (n[4] + n[5]);
-    const double it = rcp64_full(fma(p.g3s, sided, fma(p.g3c, pow4(r0), w4)));
-    const double is = p.g3s * it;
+    T r4, r0;
+    if constexpr (sizeof(T) == 8) {
+        auto inv4 = [](T &w, T &x, T &y, T &z) {
+            const T wx = w * x, yz = y * z;
+            const T r = rcp64_full(wx * yz);
+            const T rwx = r * yz, ryz = r * wx;
+            const T iw = rwx * x, ix = rwx * w, iy = ryz * z, iz = ryz * y;
+            w = iw; x = ix; y = iy; z = iz;
+        };
+        r4 = is4; r0 = t0; n[0] = t1; n[1] = t2; n[2] = t3; n[3] = t4; n[4] = t5; n[5] = t6;
+        inv4(r4, r0, n[0], n[1]);
+        inv4(n[2], n[3], n[4], n[5]);
+    } else {
+        const T tm = fminf(fminf(fminf(is4, t0), fminf(t1, t2)), fminf(fminf(t3, t4), fminf(t5, t6)));
+        auto ratio = [&](T t) { return tm * __builtin_amdgcn_rcpf(t); };
+        r4 = ratio(is4); r0 = ratio(t0);
+        n[0] = ratio(t1); n[1] = ratio(t2); n[2] = ratio(t3); n[3] = ratio(t4); n[4] = ratio(t5); n[5] = ratio(t6);
+    }
+    auto pow4 = [](T r) { const T r2 = r * r; return r2 * r2; };
+    const T g3s = T(p.g3s);
+    T w4 = T(p.g4) * pow4(r4);
+#pragma unroll
+    for (int k = 0; k < 6; ++k) n[k] = pow4(n[k]);
+    const T sided = ((n[0] + n[1]) + (n[2] + n[3])) + (n[4] + n[5]);
+    const T sum = fma(g3s, sided, fma(T(p.g3c), pow4(r0), w4));
+    T it;
+    if constexpr (sizeof(T) == 8) it = rcp64_full(sum);
+    else it = __builtin_amdgcn_rcpf(sum);
+    is = g3s * it;
     w4 *= it;
-    const double ke = p.k2 * w4, ko = (SYS == ACX_ACOUSTIC4 ? p.k1a : p.k1w) * w4;
+    ke = T(p.k2) * w4;
+    ko = T(SYS == ACX_ACOUSTIC4 ? p.k1a : p.k1w) * w4;
+}
+
+template <int SYS, typename T, typename Get>
+__device__ __forceinline__ void cweno_faces(Get get, const CwArgs &p, bool full, T (&fm)[3], T (&fp)[3])
+{
+    const T u0 = get(0);
+    T S[3], B[3], a[3], c[3], n[6] = {};
+    T e2[3], e3[3], A[3], Cc[3];
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
-        const double h1 = n[2 * d] * a[d], h2 = n[2 * d + 1] * c[d];
-        const double T = a[d] + c[d], F = a[d] - c[d];
-        const double E = fma(-ke, F, fma(is, h1 - h2, B[d]));
-        const double O = fma(ko, T, fma(-is, h1 + h2, S[d]));
+        const T m2 = get(1 + 4 * d), m1 = get(2 + 4 * d), p1 = get(3 + 4 * d), p2 = get(4 + 4 * d);
+        const T e1 = m1 - m2, e4 = p2 - p1;
+        e2[d] = u0 - m1;
+        e3[d] = p1 - u0;
+        A[d] = e4 - e3[d];
+        Cc[d] = e2[d] - e1;
+        B[d] = e3[d] - e2[d];
+        S[d] = e2[d] + e3[d];
+        a[d] = A[d] - B[d];
+        c[d] = B[d] - Cc[d];
+    }
+    T is = T(0), ke = T(0), ko = T(-1.0 / 6.0);
+    if (full) cweno_weights4<SYS, T>(get, p, S, B, a, c, e2, e3, A, Cc, n, is, ke, ko);
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        const T h1 = n[2 * d] * a[d], h2 = n[2 * d + 1] * c[d];
+        const T G = a[d] + c[d], F = a[d] - c[d];
+        const T E = fma(-ke, F, fma(is, h1 - h2, B[d]));
+        const T O = fma(ko, G, fma(-is, h1 + h2, S[d]));
         if constexpr (SYS == ACX_ACOUSTIC4) {
-            const double even = fma(1.0 / 12.0, E, u0);
-            fm[d] = fma(-0.25, O, even);
-            fp[d] = fma(0.25, O, even);
+            const T even = fma(T(1.0 / 12.0), E, u0);
+            fm[d] = fma(T(-0.25), O, even);
+            fp[d] = fma(T(0.25), O, even);
         } else {
-            fm[d] = 0.5 * (O - E);
-            fp[d] = 0.5 * (O + E);
+            fm[d] = T(0.5) * (O - E);
+            fp[d] = T(0.5) * (O + E);
         }
     }
 }

@@ -8,6 +8,10 @@
 
 namespace acx {
 
+// Stages of a compensated FP32 step by what they read: no increment yet, the
+// increment, the increment and the state the step ends in.
+enum { F32_FIRST = 0, F32_MID = 1, F32_LAST = 2 };
+
 // Arguments of the fused linear stage kernel (acx_linear.hip).
 struct LinArgs {
     const void *q;     // stage input (F32C: the HI part of the base state)
@@ -43,7 +47,7 @@ struct CwArgs {
     double a, b, c;
     double K, invrho, s, inv_h, c2;
     double g4, g3c, g3s, inv_g4;   // linear weights: gamma_R4, gamma_R3[0], gamma_R3[1..6], 1/gamma_R4
-    // FP64 combination (cweno_faces64): (g3s - 11/60)/g4 plus the share of c3
+    // the combination of cweno_faces: (g3s - 11/60)/g4 plus the share of c3
     // in the odd part (ACOUSTIC4 1/60, WAVE2 1/10, over g4), and g3s/g4
     double k1a, k1w, k2;
     unsigned *nf;                  // non-finite watch word (host-mapped; null: no watch)

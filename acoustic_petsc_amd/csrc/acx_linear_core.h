@@ -53,7 +53,6 @@ enum { EPI_RHS = 0, EPI_AXPY = 1, EPI_COMB = 2, EPI_F32C = 3 };
 // 279, 418, 697 at the copy's rate; the step 2.51 -> 2.23 ms, at 256^3 0.72 ->
 // 0.66 ms.  Its error against 64-bit steps is lower too (one step of
 // ACOUSTIC4 7.7e-9 -> 7.4e-9, of WAVE2 7.9e-7 -> 7.3e-7).
-enum { F32_FIRST = 0, F32_MID = 1, F32_LAST = 2 };
 
 template <int SYS, int BY>
 struct Tile32 {
