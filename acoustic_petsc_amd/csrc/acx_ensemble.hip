@@ -69,7 +69,7 @@ k_ensemble(const EnsProblem *__restrict__ probs, const EnsItem *__restrict__ ite
         const int x0 = (local % pr.ntx) * ENS_BX, y0 = ((local / pr.ntx) % pr.nty) * BY;
         a.zc = pr.zc;
         const int zb = (local / (pr.ntx * pr.nty)) * a.zc;
-        linear_tile32<ACX_ACOUSTIC4, BY, STAGE, false>(a, x0, y0, zb, lds);
+        linear_tile32<ACX_ACOUSTIC4, BY, STAGE, false, true>(a, x0, y0, zb, lds);
         __syncthreads();   // LDS is reused by the next item
     }
 }

@@ -11,26 +11,38 @@
 //
 // Layout: 2.5D blocking.  A block owns a BX x BY column tile and marches a
 // chunk of z-planes.  Each plane is read once: staged in LDS with an x/y
-// halo of 3 (double-buffered, one barrier per plane) for its in-plane
-// stencils, and pushed into a per-thread register queue that supplies the
-// z-stencil three planes later.  HBM traffic per stage is one read of Q
+// halo of 3 (one barrier per plane) for its in-plane stencils, and kept in
+// per-thread registers for the z-stencils.  HBM traffic per stage is one read of Q
 // (+ U0) and one write of OUT; halo rows are read by neighbouring tiles at
 // the same plane index, so they meet in L2 (tiles are ordered per XCD).
 #include "acx_linear_core.h"
 
 namespace acx {
 
-// Centre-plane march with the 5-plane halo ring (acx_linear_core.h), FP64, on
-// 32 x 16 tiles.  WALLS = false is the all-periodic instantiation (no ghost
-// signs).
-template <int SYS, int EPI, bool WALLS>
+// FP64 march (acx_linear_core.h).  WALLS = false is the all-periodic
+// instantiation (no ghost signs, offsets inside a plane in 32 bits).
+template <int SYS, int EPI, bool WALLS, int MEM>
+__global__ void __launch_bounds__(512)
+k_linear64(LinArgs p)
+{
+    using Tile = Tile64<SYS>;
+    __shared__ typename Tile::Lds lds;
+    const int tile = xcd_logical_tile(blockIdx.x, gridDim.x);
+    const int x0 = (tile % p.ntx) * Tile::BX, y0 = ((tile / p.ntx) % p.nty) * Tile::BY, zb = (tile / (p.ntx * p.nty)) * p.zc;
+    linear_tile64<SYS, EPI, WALLS, MEM>(p, x0, y0, zb, lds);
+}
+
+// Centre-plane march with the 5-plane halo ring (acx_linear_core.h), FP64
+// ACOUSTIC4 on 32 x 16 tiles.  WALLS = false is the all-periodic instantiation
+// (no ghost signs).
+template <int EPI, bool WALLS>
 __global__ void __launch_bounds__(32 * 16)
 k_linear(LinArgs p)
 {
-    __shared__ double lds[5][LinTile<SYS, 32, 16>::NS][16 + 6][32 + 6];
+    __shared__ double lds[5][LinTile::NV][LinTile::BY + 6][LinTile::BX + 6];
     const int tile = xcd_logical_tile(blockIdx.x, gridDim.x);
     const int x0 = (tile % p.ntx) * 32, y0 = ((tile / p.ntx) % p.nty) * 16, zb = (tile / (p.ntx * p.nty)) * p.zc;
-    linear_tile_centre<SYS, 32, 16, EPI, WALLS>(p, x0, y0, zb, lds);
+    linear_tile_centre<EPI, WALLS>(p, x0, y0, zb, lds);
 }
 
 // LDS-DMA march (acx_linear_core.h): FP64 ACOUSTIC4 RHS / AXPY stages on
@@ -72,79 +84,45 @@ static int launch_linear_dma(const LinArgs &a, hipStream_t s)
     return hip_check(hipGetLastError(), "k_linear_dma launch");
 }
 
-// WAVE2 RHS / AXPY stages on the same march: 80 KB of LDS, two blocks per CU
-// (registers capped for 4 waves per SIMD).
-template <int EPI>
-__global__ void __launch_bounds__(DmaPlan::BX *DmaPlan::BY) __attribute__((amdgpu_waves_per_eu(4)))
-k_linear_dma_w2(LinArgs p)
-{
-    __shared__ __attribute__((aligned(16))) unsigned char ring[DmaPlanW2::NSLOT * DmaPlanW2::SLOT];
-    const int tile = xcd_logical_tile(blockIdx.x, gridDim.x);
-    const int x0 = (tile % p.ntx) * DmaPlan::BX, y0 = ((tile / p.ntx) % p.nty) * DmaPlan::BY;
-    const int zb = (tile / (p.ntx * p.nty)) * p.zc;
-    linear_tile_dma_w2<EPI>(p, x0, y0, zb, ring);
-}
-
-template <int EPI>
-static int launch_linear_dma_w2(const LinArgs &a, hipStream_t s)
-{
-    LinArgs b = a;
-    b.ntx = (a.nx + DmaPlan::BX - 1) / DmaPlan::BX;
-    b.nty = (a.ny + DmaPlan::BY - 1) / DmaPlan::BY;
-    static int per_cu = 0;
-    if (!per_cu) {
-        int n = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, reinterpret_cast<const void *>(&k_linear_dma_w2<EPI>),
-                                                         DmaPlan::BX * DmaPlan::BY, 0) != hipSuccess || n <= 0)
-            n = 1;
-        per_cu = n;
-    }
-    if (b.zc <= 0) b.zc = auto_zc(b.ntx, b.nty, a.nz, device_cus() * per_cu, 10);
-    b.ntz = (a.nz + b.zc - 1) / b.zc;
-    hipLaunchKernelGGL(k_linear_dma_w2<EPI>, dim3((unsigned)(b.ntx * b.nty * b.ntz)), dim3(DmaPlan::BX, DmaPlan::BY),
-                       0, s, b);
-    return hip_check(hipGetLastError(), "k_linear_dma_w2 launch");
-}
-
 // ---------------------------------------------------------------------------
 
-template <int SYS, int EPI, bool WALLS>
+// One round model for both marches.  Slots are the CUs, also where two blocks
+// of the WAVE2 kernel fit one: with chunks half as long the WAVE2 stages of 256^3
+// took 159 us (combining) and 84.6 (the others) instead of 139 and 79.7.
+template <int SYS, int EPI, bool WALLS, int MEM>
+static int launch_linear64_w(const LinArgs &a, hipStream_t s)
+{
+    using Tile = Tile64<SYS>;
+    LinArgs b = a;
+    b.ntx = (a.nx + Tile::BX - 1) / Tile::BX;
+    b.nty = (a.ny + Tile::BY - 1) / Tile::BY;
+    if (b.zc <= 0) b.zc = auto_zc(b.ntx, b.nty, a.nz, device_cus(), 10);
+    b.ntz = (a.nz + b.zc - 1) / b.zc;
+    hipLaunchKernelGGL((k_linear64<SYS, EPI, WALLS, MEM>), dim3(b.ntx * b.nty * b.ntz), dim3(Tile::BX, Tile::BY), 0, s, b);
+    return hip_check(hipGetLastError(), "k_linear64 launch");
+}
+
+template <int EPI, bool WALLS>
 static int launch_linear_v(const LinArgs &a, hipStream_t s)
 {
     LinArgs b = a;
-    b.ntx = (a.nx + 31) / 32;
-    b.nty = (a.ny + 15) / 16;
-    if (b.zc <= 0) {
-        // workgroups of this instantiation that fit a CU at once (queried once)
-        static int per_cu = 0;
-        if (!per_cu) {
-            int n = 0;
-            if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                    &n, reinterpret_cast<const void *>(&k_linear<SYS, EPI, WALLS>), 32 * 16, 0) != hipSuccess || n <= 0)
-                n = 1;
-            per_cu = n;
-        }
-        // At most two blocks per CU count as slots: the round model takes the
-        // smallest z-chunk that fills one round, and with four co-resident
-        // blocks of the WAVE2 kernel that was 32 planes at 256^3, whose z-halo
-        // re-reads cost more than the round saved (measured at 256^3: WAVE2
-        // step 0.458 ms with the COMB stage at 32 planes, 0.450 at 64).
-        b.zc = auto_zc(b.ntx, b.nty, a.nz, device_cus() * (per_cu < 2 ? per_cu : 2), 10);
-    }
+    b.ntx = (a.nx + LinTile::BX - 1) / LinTile::BX;
+    b.nty = (a.ny + LinTile::BY - 1) / LinTile::BY;
+    if (b.zc <= 0) b.zc = auto_zc(b.ntx, b.nty, a.nz, device_cus(), 10);
     b.ntz = (a.nz + b.zc - 1) / b.zc;
-    hipLaunchKernelGGL((k_linear<SYS, EPI, WALLS>), dim3(b.ntx * b.nty * b.ntz), dim3(32, 16), 0, s, b);
+    hipLaunchKernelGGL((k_linear<EPI, WALLS>), dim3(b.ntx * b.nty * b.ntz), dim3(LinTile::BX, LinTile::BY), 0, s, b);
     return hip_check(hipGetLastError(), "k_linear launch");
 }
 
 // FP32 compensated stages (linear_tile32).
-template <int SYS, int BY, int STAGE, bool WALLS>
+template <int SYS, int BY, int STAGE, bool WALLS, bool STREAM>
 __global__ void __launch_bounds__(64 * BY) __attribute__((amdgpu_waves_per_eu(BY / 4)))
 k_linear32(LinArgs p)
 {
     __shared__ typename Tile32<SYS, BY>::template Shared<STAGE> lds;
     const int tile = xcd_logical_tile(blockIdx.x, gridDim.x);
     const int x0 = (tile % p.ntx) * 64, y0 = ((tile / p.ntx) % p.nty) * BY, zb = (tile / (p.ntx * p.nty)) * p.zc;
-    linear_tile32<SYS, BY, STAGE, WALLS>(p, x0, y0, zb, lds);
+    linear_tile32<SYS, BY, STAGE, WALLS, STREAM>(p, x0, y0, zb, lds);
 }
 
 // Tiles of 64 x 12 columns (one block of 12 wavefronts per CU, at most 168
@@ -152,6 +130,13 @@ k_linear32(LinArgs p)
 // larger tile takes about 1.3 times as long for 1.5 times the cells.
 // Measured, us per step: 384^3 2235 with 12 rows, 2490 with 8; 256^3 (22 tiles
 // of 12 rows in y, two rounds; 32 of 8 rows, one round) 713 and 647.
+//
+// Results stay in the caches (STREAM = false) up to CACHED32_BYTES a field (a
+// stage reads up to three fields and writes two): us per step, cached against
+// streaming, ACOUSTIC4 128^3 92 against 103, 150 x 131 x 90 86 / 105, 160^3 183
+// / 190, 192^3 299 / 274; WAVE2 128^3 55 / 64, 192^3 153 / 164, 256^3 433 / 407.
+constexpr size_t CACHED32_BYTES = 80ull << 20;
+
 template <int SYS, int STAGE, bool WALLS>
 static int launch_linear32_w(const LinArgs &a, hipStream_t s)
 {
@@ -166,8 +151,13 @@ static int launch_linear32_w(const LinArgs &a, hipStream_t s)
     if (b.zc <= 0) b.zc = big ? z12 : z8;
     b.ntz = (a.nz + b.zc - 1) / b.zc;
     const dim3 grd((unsigned)(b.ntx * b.nty * b.ntz));
-    if (big) hipLaunchKernelGGL((k_linear32<SYS, 12, STAGE, WALLS>), grd, dim3(64, 12), 0, s, b);
-    else hipLaunchKernelGGL((k_linear32<SYS, 8, STAGE, WALLS>), grd, dim3(64, 8), 0, s, b);
+    const bool cached = (size_t)a.nx * a.ny * a.nz * Tile32<SYS, 8>::NV * 4 <= CACHED32_BYTES;
+    const void *k = big ? (cached ? reinterpret_cast<const void *>(&k_linear32<SYS, 12, STAGE, WALLS, false>)
+                                  : reinterpret_cast<const void *>(&k_linear32<SYS, 12, STAGE, WALLS, true>))
+                        : (cached ? reinterpret_cast<const void *>(&k_linear32<SYS, 8, STAGE, WALLS, false>)
+                                  : reinterpret_cast<const void *>(&k_linear32<SYS, 8, STAGE, WALLS, true>));
+    void *args[] = {&b};
+    if (int rc = hip_check(hipLaunchKernel(k, grd, dim3(64, big ? 12 : 8), args, 0, s), "k_linear32 launch")) return rc;
     return hip_check(hipGetLastError(), "k_linear32 launch");
 }
 
@@ -184,25 +174,41 @@ static int launch_linear32(const LinArgs &a, hipStream_t s)
     return general ? launch_linear32_w<SYS, F32_FIRST, true>(a, s) : launch_linear32_w<SYS, F32_FIRST, false>(a, s);
 }
 
-// FP64 stages: all-periodic RHS and AXPY stages take the LDS-DMA march, the
-// others the centre-plane march.
+// FP64 stages.  Where a field is at most CACHED_BYTES, linear_tile64 with
+// cached results (a stage's result is the next one's input, and the 256 MB
+// last-level cache holds two fields).  Above, results stream, WAVE2 stays with
+// linear_tile64, all-periodic ACOUSTIC4 RHS and AXPY stages take the LDS-DMA
+// march and the other ACOUSTIC4 stages the centre-plane march.  Measured, us
+// per step (all periodic, walled):
+//                   others         linear_tile64   linear_tile64
+//                                  streaming       cached
+//   ACOUSTIC4 128^3   158, 155       157, 160        114, 116
+//   ACOUSTIC4 192^3   436, 459       462, 464        466, 465
+//   WAVE2 128^3       73.7, 68.2     73.1, 73.3      59.2, 58.7
+//   WAVE2 192^3       217, 208       195, 195        195, 192
+//   WAVE2 224^3       318, 346       317, 317        333, 333
+//   WAVE2 384^3       1679, 1758     1683, 1674      1778, 1768
+constexpr size_t CACHED_BYTES = 128ull << 20;
+
 template <int SYS, int EPI>
 static int launch_linear64(const LinArgs &a, hipStream_t s)
 {
     const bool walls = a.bc[0] != ACX_PERIODIC || a.bc[1] != ACX_PERIODIC || a.bc[2] != ACX_PERIODIC;
-    if constexpr (SYS == ACX_ACOUSTIC4 && (EPI == EPI_RHS || EPI == EPI_AXPY)) {
-        // the LDS-DMA march (measured at 256^3: AXPY stage 207 -> 196 us,
-        // step 0.958 -> 0.905 ms): periodic grids whose plane offsets fit 32 bits
-        if (!walls && (size_t)a.nx * a.ny * 4 < 0x7fffffffu)
-            return launch_linear_dma<EPI>(a, s);
+    const size_t plane_bytes = (size_t)a.nx * a.ny * Tile64<SYS>::NV * 8;
+    if (plane_bytes * a.nz <= CACHED_BYTES)
+        return walls ? launch_linear64_w<SYS, EPI, true, MEM_CACHED>(a, s)
+                     : launch_linear64_w<SYS, EPI, false, MEM_CACHED>(a, s);
+    if constexpr (SYS == ACX_ACOUSTIC4) {
+        if constexpr (EPI != EPI_COMB) {
+            // plane offsets in 32 bits
+            if (!walls && (size_t)a.nx * a.ny * 4 < 0x7fffffffu) return launch_linear_dma<EPI>(a, s);
+        }
+        return walls ? launch_linear_v<EPI, true>(a, s) : launch_linear_v<EPI, false>(a, s);
+    } else {
+        if ((size_t)a.nx * 16 >= 0x7fff0000u) return launch_linear64_w<SYS, EPI, true, MEM_WIDE>(a, s);
+        return walls || plane_bytes > 0xffffffffu ? launch_linear64_w<SYS, EPI, true, MEM_STREAM>(a, s)
+                                                  : launch_linear64_w<SYS, EPI, false, MEM_STREAM>(a, s);
     }
-    if constexpr (SYS == ACX_WAVE2 && (EPI == EPI_RHS || EPI == EPI_AXPY)) {
-        // measured: the WAVE2 step 0.485 -> 0.459 ms at 256^3, 1.904 -> 1.760 ms
-        // at 384^3, bit-identical to the halo-ring kernel
-        if (!walls && (size_t)a.nx * a.ny * 2 < 0x7fffffffu)
-            return launch_linear_dma_w2<EPI>(a, s);
-    }
-    return walls ? launch_linear_v<SYS, EPI, true>(a, s) : launch_linear_v<SYS, EPI, false>(a, s);
 }
 
 int launch_linear(const LinArgs &a, int sys, int epi, bool fp32, hipStream_t s)

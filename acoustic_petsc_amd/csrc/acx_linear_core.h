@@ -8,14 +8,6 @@
 
 namespace acx {
 
-template <int SYS, int BX, int BY>
-struct LinTile {
-    static constexpr int NV = SYS == ACX_ACOUSTIC4 ? 4 : 2;   // components in memory
-    static constexpr int NS = SYS == ACX_ACOUSTIC4 ? 4 : 1;   // components in the stencil
-    static constexpr int LX = BX + 6, LY = BY + 6;
-    static constexpr int NHALO = 6 * BX + 6 * BY;              // star stencil: no plane corners
-};
-
 // Epilogue kinds
 enum { EPI_RHS = 0, EPI_AXPY = 1, EPI_COMB = 2, EPI_F32C = 3 };
 
@@ -42,7 +34,8 @@ enum { EPI_RHS = 0, EPI_AXPY = 1, EPI_COMB = 2, EPI_F32C = 3 };
 // - the sums s_k = q(+k) + q(-k) over the axes are taken before the weights
 //   (the differences of A7 likewise), in units of s/(48 h);
 // - a cell is one 16-byte LDS entry (12 16-byte reads);
-// - results are stored through a buffer descriptor per wavefront row, whose
+// - results are stored (STREAM: nontemporal, for fields beyond the last-level
+//   cache) through a buffer descriptor per wavefront row, whose
 //   bound drops the columns past the grid: without a branch around the store
 //   the compiler can count it, and waits for a plane's loads alone instead of
 //   for every load and store before them;
@@ -72,22 +65,22 @@ struct Tile32 {
 typedef unsigned acx_u32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned acx_u32x2 __attribute__((ext_vector_type(2)));
 
-// Nontemporal store of this lane's cell of a wavefront row: row points at the
-// row's first cell (wave-uniform), bytes bounds the cells that exist.
-template <int NV>
-__device__ __forceinline__ void store_row_nt(float *row, unsigned bytes, const Cell<float, NV> &c)
+// Store of this lane's cell of a wavefront row (STREAM: nontemporal): row points
+// at the row's first cell (wave-uniform), bytes bounds the cells that exist.
+template <int NV, bool STREAM>
+__device__ __forceinline__ void store_row(float *row, unsigned bytes, const Cell<float, NV> &c)
 {
     const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(row, 0, (int)bytes, 0x00020000);
     const int off = (int)__lane_id() * NV * 4;
     if constexpr (NV == 4)
         __builtin_amdgcn_raw_buffer_store_b128(
             acx_u32x4{__float_as_uint(c.v[0]), __float_as_uint(c.v[1]), __float_as_uint(c.v[2]), __float_as_uint(c.v[3])},
-            r, off, 0, 2);
+            r, off, 0, STREAM ? 2 : 0);
     else
-        __builtin_amdgcn_raw_buffer_store_b64(acx_u32x2{__float_as_uint(c.v[0]), __float_as_uint(c.v[1])}, r, off, 0, 2);
+        __builtin_amdgcn_raw_buffer_store_b64(acx_u32x2{__float_as_uint(c.v[0]), __float_as_uint(c.v[1])}, r, off, 0, STREAM ? 2 : 0);
 }
 
-template <int SYS, int BY, int STAGE, bool WALLS>
+template <int SYS, int BY, int STAGE, bool WALLS, bool STREAM>
 __device__ __forceinline__ void linear_tile32(const LinArgs &p, int x0, int y0, int zb,
                                               typename Tile32<SYS, BY>::template Shared<STAGE> &lds)
 {
@@ -143,6 +136,7 @@ __device__ __forceinline__ void linear_tile32(const LinArgs &p, int x0, int y0, 
     auto load = [](const float *plane_base, Off o) {
         return load_cell<float, NV>(reinterpret_cast<const float *>(reinterpret_cast<const char *>(plane_base) + o), 0);
     };
+    auto load_lo = [&](size_t cell) { return STREAM ? load_cell_nt<float, NV>(LO, cell) : load_cell<float, NV>(LO, cell); };
     // the plane loaded next, its offset and its ghost sign
     int zi = 0;
     size_t zoff = 0;
@@ -260,7 +254,7 @@ __device__ __forceinline__ void linear_tile32(const LinArgs &p, int x0, int y0, 
         }
         load_column(hi[0], d);
         load_halo(hq, hd);
-        if constexpr (LAST) lo = load_cell_nt<float, NV>(LO, (size_t)zb * plane + col);
+        if constexpr (LAST) lo = load_lo((size_t)zb * plane + col);
 #pragma unroll
         for (int k = 3; k < 6; ++k) {
             stage(k & 1, q[2 + k], ph[k - 3], pd[k - 3], sz[k]);
@@ -332,11 +326,11 @@ __device__ __forceinline__ void linear_tile32(const LinArgs &p, int x0, int y0, 
             C nh, nl;
 #pragma unroll
             for (int v = 0; v < NV; ++v) two_sum(hi[uc].v[v], lo.v[v] + o.v[v], nh.v[v], nl.v[v]);
-            store_row_nt<NV>(static_cast<float *>(p.out2) + out, row_bytes, nl);
+            store_row<NV, STREAM>(static_cast<float *>(p.out2) + out, row_bytes, nl);
             o = nh;
-            lo = load_cell_nt<float, NV>(LO, (size_t)min(c + 1, ze - 1) * plane + col);
+            lo = load_lo((size_t)min(c + 1, ze - 1) * plane + col);
         }
-        store_row_nt<NV>(static_cast<float *>(p.out) + out, row_bytes, o);
+        store_row<NV, STREAM>(static_cast<float *>(p.out) + out, row_bytes, o);
         if constexpr (LAST) {
             C w = o;
 #pragma unroll
@@ -366,20 +360,26 @@ __device__ __forceinline__ void linear_tile32(const LinArgs &p, int x0, int y0, 
     watch_flush(p.nf, nfbad);
 }
 
-// Centre-plane march (FP64): the own column's z-queue holds planes z-3 .. z+3
-// before plane z is computed, and plane z (with its x/y halo) is staged in LDS
-// and finished in the same iteration.  The halo of plane z+4 is loaded
-// together with the column's plane z+4, i.e. at the iteration in which the
-// neighbouring tiles load those cells as their interior, so the shared rows
-// are still in L2; it waits in its slot of a 5-plane LDS ring until plane z+4
-// is computed.  Epilogue operands and results stream past L2 (nontemporal),
-// leaving L2 to the stage input that neighbouring tiles re-read as halo.
-template <int SYS, int BX, int BY, int EPI, bool WALLS>
+// Centre-plane march for FP64 ACOUSTIC4 fields beyond the last-level cache: the
+// own column's z-queue holds planes z-3 .. z+3 before plane z is computed, and
+// plane z (with its x/y halo) is staged in LDS and finished in the same
+// iteration.  The halo of plane z+4 is loaded together with the column's plane
+// z+4, i.e. at the iteration in which the neighbouring tiles load those cells
+// as their interior, so the shared rows are still in L2; it waits in its slot
+// of a 5-plane LDS ring until plane z+4 is computed.  Epilogue operands and
+// results stream past L2 (nontemporal), leaving L2 to the stage input that
+// neighbouring tiles re-read as halo.
+struct LinTile {
+    static constexpr int BX = 32, BY = 16, NV = 4;
+    static constexpr int NHALO = 6 * BX + 6 * BY;              // star stencil: no plane corners
+};
+
+template <int EPI, bool WALLS>
 __device__ __forceinline__ void linear_tile_centre(const LinArgs &p, int x0, int y0, int zb,
-                                                   double (&lds)[5][LinTile<SYS, BX, BY>::NS][BY + 6][BX + 6])
+                                                   double (&lds)[5][LinTile::NV][LinTile::BY + 6][LinTile::BX + 6])
 {
-    using Tile = LinTile<SYS, BX, BY>;
-    constexpr int NV = Tile::NV, NS = Tile::NS;
+    using Tile = LinTile;
+    constexpr int NV = Tile::NV, BX = Tile::BX, BY = Tile::BY;
     using C = Cell<double, NV>;
     static_assert(BX * BY >= Tile::NHALO, "every halo cell of a plane needs a thread of its own");
 
@@ -449,7 +449,7 @@ __device__ __forceinline__ void linear_tile_centre(const LinArgs &p, int x0, int
                 issue(r, hcol, zb + d);
                 const C c = apply(r, hsx, hsy);
 #pragma unroll
-                for (int v = 0; v < NS; ++v) lds[d][v][hy][hx] = c.v[v];
+                for (int v = 0; v < NV; ++v) lds[d][v][hy][hx] = c.v[v];
             }
         }
     }
@@ -459,7 +459,7 @@ __device__ __forceinline__ void linear_tile_centre(const LinArgs &p, int x0, int
     // wait for its own 4-planes-ahead prefetch before the barrier.
     __builtin_amdgcn_s_waitcnt(0);
 
-    const double inv48h = p.inv48h, Kc = p.K, irho = p.invrho, sLLF = p.s, lap = p.lapc;
+    const double inv48h = p.inv48h, Kc = p.K, irho = p.invrho, sLLF = p.s;
 
     bool nfbad = false;   // non-finite watch of this thread's outputs
     int buf = 0;          // slot of plane z
@@ -473,48 +473,37 @@ __device__ __forceinline__ void linear_tile_centre(const LinArgs &p, int x0, int
         C e0;
         if constexpr (EPI == EPI_COMB) { if (active) e0 = load_cell_nt<double, NV>(U0, idx); }
 #pragma unroll
-        for (int v = 0; v < NS; ++v) lds[buf][v][ty + 3][tx + 3] = qz[3].v[v];
+        for (int v = 0; v < NV; ++v) lds[buf][v][ty + 3][tx + 3] = qz[3].v[v];
         __syncthreads();
         C r;
-        if constexpr (SYS == ACX_ACOUSTIC4) {
-            double accB[4], dAp[3], dAvel = 0.0;
+        double accB[4], dAp[3], dAvel = 0.0;
 #pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const double *row = &lds[buf][v][ty + 3][tx + 3];
-                const double xm3 = row[-3], xm2 = row[-2], xm1 = row[-1], xp1 = row[1], xp2 = row[2], xp3 = row[3];
-                const double ym3 = lds[buf][v][ty][tx + 3], ym2 = lds[buf][v][ty + 1][tx + 3];
-                const double ym1 = lds[buf][v][ty + 2][tx + 3];
-                const double yp1 = lds[buf][v][ty + 4][tx + 3], yp2 = lds[buf][v][ty + 5][tx + 3];
-                const double yp3 = lds[buf][v][ty + 6][tx + 3];
-                const double q0 = qz[3].v[v];
-                accB[v] = stencil_B7(xm3, xm2, xm1, q0, xp1, xp2, xp3) + stencil_B7(ym3, ym2, ym1, q0, yp1, yp2, yp3) +
-                          stencil_B7(qz[0].v[v], qz[1].v[v], qz[2].v[v], q0, qz[4].v[v], qz[5].v[v], qz[6].v[v]);
-                if (v == 0) {
-                    dAp[0] = stencil_A7(xm3, xm2, xm1, xp1, xp2, xp3);
-                    dAp[1] = stencil_A7(ym3, ym2, ym1, yp1, yp2, yp3);
-                    dAp[2] = stencil_A7(qz[0].v[0], qz[1].v[0], qz[2].v[0], qz[4].v[0], qz[5].v[0], qz[6].v[0]);
-                } else if (v == 1) {
-                    dAvel += stencil_A7(xm3, xm2, xm1, xp1, xp2, xp3);
-                } else if (v == 2) {
-                    dAvel += stencil_A7(ym3, ym2, ym1, yp1, yp2, yp3);
-                } else {
-                    dAvel += stencil_A7(qz[0].v[3], qz[1].v[3], qz[2].v[3], qz[4].v[3], qz[5].v[3], qz[6].v[3]);
-                }
+        for (int v = 0; v < 4; ++v) {
+            const double *row = &lds[buf][v][ty + 3][tx + 3];
+            const double xm3 = row[-3], xm2 = row[-2], xm1 = row[-1], xp1 = row[1], xp2 = row[2], xp3 = row[3];
+            const double ym3 = lds[buf][v][ty][tx + 3], ym2 = lds[buf][v][ty + 1][tx + 3];
+            const double ym1 = lds[buf][v][ty + 2][tx + 3];
+            const double yp1 = lds[buf][v][ty + 4][tx + 3], yp2 = lds[buf][v][ty + 5][tx + 3];
+            const double yp3 = lds[buf][v][ty + 6][tx + 3];
+            const double q0 = qz[3].v[v];
+            accB[v] = stencil_B7(xm3, xm2, xm1, q0, xp1, xp2, xp3) + stencil_B7(ym3, ym2, ym1, q0, yp1, yp2, yp3) +
+                      stencil_B7(qz[0].v[v], qz[1].v[v], qz[2].v[v], q0, qz[4].v[v], qz[5].v[v], qz[6].v[v]);
+            if (v == 0) {
+                dAp[0] = stencil_A7(xm3, xm2, xm1, xp1, xp2, xp3);
+                dAp[1] = stencil_A7(ym3, ym2, ym1, yp1, yp2, yp3);
+                dAp[2] = stencil_A7(qz[0].v[0], qz[1].v[0], qz[2].v[0], qz[4].v[0], qz[5].v[0], qz[6].v[0]);
+            } else if (v == 1) {
+                dAvel += stencil_A7(xm3, xm2, xm1, xp1, xp2, xp3);
+            } else if (v == 2) {
+                dAvel += stencil_A7(ym3, ym2, ym1, yp1, yp2, yp3);
+            } else {
+                dAvel += stencil_A7(qz[0].v[3], qz[1].v[3], qz[2].v[3], qz[4].v[3], qz[5].v[3], qz[6].v[3]);
             }
-            r.v[0] = inv48h * (sLLF * accB[0] - Kc * dAvel);
-            r.v[1] = inv48h * (sLLF * accB[1] - irho * dAp[0]);
-            r.v[2] = inv48h * (sLLF * accB[2] - irho * dAp[1]);
-            r.v[3] = inv48h * (sLLF * accB[3] - irho * dAp[2]);
-        } else {
-            const double *row = &lds[buf][0][ty + 3][tx + 3];
-            const double q0 = qz[3].v[0];
-            const double L = stencil_L7(row[-3], row[-2], row[-1], q0, row[1], row[2], row[3]) +
-                        stencil_L7(lds[buf][0][ty][tx + 3], lds[buf][0][ty + 1][tx + 3], lds[buf][0][ty + 2][tx + 3], q0,
-                                   lds[buf][0][ty + 4][tx + 3], lds[buf][0][ty + 5][tx + 3], lds[buf][0][ty + 6][tx + 3]) +
-                        stencil_L7(qz[0].v[0], qz[1].v[0], qz[2].v[0], q0, qz[4].v[0], qz[5].v[0], qz[6].v[0]);
-            r.v[0] = qz[3].v[1];     // du/dt = v (rhs_function.c:330)
-            r.v[1] = lap * L;
         }
+        r.v[0] = inv48h * (sLLF * accB[0] - Kc * dAvel);
+        r.v[1] = inv48h * (sLLF * accB[1] - irho * dAp[0]);
+        r.v[2] = inv48h * (sLLF * accB[2] - irho * dAp[1]);
+        r.v[3] = inv48h * (sLLF * accB[3] - irho * dAp[2]);
 
         if (active) {
             C o;
@@ -541,10 +530,325 @@ __device__ __forceinline__ void linear_tile_centre(const LinArgs &p, int x0, int
         if (hx >= 0 && z + 4 < ze) {
             const C h = apply(ch, hsx, hsy);
 #pragma unroll
-            for (int v = 0; v < NS; ++v) lds[hslot][v][hy][hx] = h.v[v];
+            for (int v = 0; v < NV; ++v) lds[hslot][v][hy][hx] = h.v[v];
         }
         buf = buf == 4 ? 0 : buf + 1;
         hslot = hslot == 4 ? 0 : hslot + 1;
+    }
+    watch_flush(p.nf, nfbad);
+}
+
+// FP64 march (every WAVE2 stage, and the ACOUSTIC4 stages of fields that fit the
+// last-level cache).  The own column's ring holds planes c-3 .. c+3 when plane
+// c is finished; plane c is staged in LDS over the halo that already waits there.
+// Column and halo of plane c+4 are loaded together, at the iteration in which
+// the neighbouring tiles load those cells as their interior, so the shared
+// rows are still in L2; the halo is put into its slot of a 4-plane LDS ring an
+// iteration later.  Every load and store is unconditional (clamped planes,
+// out-of-range buffer stores): the compiler then counts what is in flight and
+// a load has a whole iteration to arrive.  (In the centre-plane march above
+// a plane's loads are waited for in the iteration that issues them.)
+//   Bound, ACOUSTIC4: 24 16-byte LDS reads a thread and plane, 0.75 us for
+//   the 512 threads of a CU, and about 160 FP64 instructions, 0.53 us.  A walled
+//   step at 150 x 131 x 90 took 150 us with the centre-plane march, 155 with
+//   this one and streaming results, 114 with cached ones.  Finishing plane c
+//   from in-plane parts kept for three planes, as in FP32, took three more
+//   iterations a chunk (combining stage 41 -> 47 us); loading the base states
+//   together with the columns, 45.
+//   LDS: an ACOUSTIC4 cell as two 16-byte halves, (p, u) and (v, w), in
+//   arrays of their own, so that neighbouring lanes read neighbouring words.
+//   Tile: 32 x 16 columns (a wavefront is two rows of 32).
+template <int SYS>
+struct Tile64 {
+    static constexpr int BX = 32, BY = 16;
+    static constexpr int NV = SYS == ACX_ACOUSTIC4 ? 4 : 2;   // components in memory
+    static constexpr int NS = SYS == ACX_ACOUSTIC4 ? 4 : 1;   // components in the stencil
+    static constexpr int LX = BX + 6, LY = BY + 6;
+    static constexpr int NHALO = 6 * BX + 6 * BY;              // star stencil: no plane corners
+    static constexpr int NP = SYS == ACX_ACOUSTIC4 ? 2 : 1;
+    using Word = typename std::conditional<SYS == ACX_ACOUSTIC4, double2, double>::type;
+    struct Lds { Word q[4][NP][LY][LX]; };
+};
+
+// Store of this lane's cell of a wavefront's two rows (STREAM: nontemporal):
+// row points at the first row's first cell (wave-uniform), off at the lane's
+// cell behind it (beyond bytes: no store).
+constexpr unsigned kNoStore = 0x80000000u;   // above every bound
+template <int NV, bool STREAM>
+__device__ __forceinline__ void store_cell_buf(double *row, unsigned bytes, unsigned off, const Cell<double, NV> &c)
+{
+    const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(row, 0, (int)bytes, 0x00020000);
+#pragma unroll
+    for (int k = 0; k < NV; k += 2) {
+        union { double d[2]; acx_u32x4 u; } w;
+        w.d[0] = c.v[k];
+        w.d[1] = c.v[k + 1];
+        __builtin_amdgcn_raw_buffer_store_b128(w.u, r, (int)off + 8 * k, 0, STREAM ? 2 : 0);
+    }
+}
+
+// MEM_CACHED: results and base states may stay in the caches, for fields small
+// enough that the next stage finds them there; MEM_STREAM: nontemporal; MEM_WIDE:
+// the same for rows of 2 GB or longer (a store descriptor for each of the two
+// rows).
+enum { MEM_CACHED = 0, MEM_STREAM = 1, MEM_WIDE = 2 };
+
+template <int SYS, int EPI, bool WALLS, int MEM>
+__device__ __forceinline__ void linear_tile64(const LinArgs &p, int x0, int y0, int zb, typename Tile64<SYS>::Lds &lds)
+{
+    using Tile = Tile64<SYS>;
+    constexpr int NV = Tile::NV, NS = Tile::NS, BX = Tile::BX, BY = Tile::BY;
+    constexpr bool AC = SYS == ACX_ACOUSTIC4, COMB = EPI == EPI_COMB, STREAM = MEM != MEM_CACHED, WIDE = MEM == MEM_WIDE;
+    using C = Cell<double, NV>;
+    static_assert(BX * BY >= Tile::NHALO, "every halo cell of a plane needs a thread of its own");
+
+    const double *__restrict__ Q = static_cast<const double *>(p.q);
+    const double *__restrict__ U0 = static_cast<const double *>(p.u0);
+    const int nx = p.nx, ny = p.ny, nz = p.nz;
+    const int tx = threadIdx.x, ty = threadIdx.y, tid = ty * BX + tx;
+    const int ze = min(zb + p.zc, nz);
+    const size_t plane = (size_t)nx * ny;
+    const int bcx = WALLS ? p.bc[0] : 0, bcy = WALLS ? p.bc[1] : 0, bcz = WALLS ? p.bc[2] : 0;
+
+    // own column
+    float sgx = 1.f, sgy = 1.f;
+    const int mx = map_axis(x0 + tx, nx, bcx, sgx);
+    const int my = map_axis(y0 + ty, ny, bcy, sgy);
+    const size_t col = (size_t)my * nx + mx;
+
+    // halo cell of this thread; threads without one load one cell per
+    // wavefront and write it to the plane's unused corner
+    int hx = 0, hy = 0;
+    size_t hcol = (size_t)__builtin_amdgcn_readfirstlane(my) * nx + __builtin_amdgcn_readfirstlane(mx);
+    float hsx = 1.f, hsy = 1.f;
+    if (tid < Tile::NHALO) {
+        int t = tid;
+        if (t < 6 * BY) {            // x halo: 3 left, 3 right per row
+            const int row = t / 6, k = t % 6;
+            hy = row + 3;
+            hx = k < 3 ? k : BX + k;  // 0,1,2 | BX+3..BX+5
+        } else {
+            t -= 6 * BY;
+            const int colx = t % BX, k = t / BX;
+            hx = colx + 3;
+            hy = k < 3 ? k : BY + k;
+        }
+        const int gx = map_axis(x0 + hx - 3, nx, bcx, hsx);
+        const int gy = map_axis(y0 + hy - 3, ny, bcy, hsy);
+        hcol = (size_t)gy * nx + gx;
+    }
+
+    // byte offsets inside a plane: 32 bits in the all-periodic instantiation
+    using Off = typename std::conditional<WALLS, size_t, uint32_t>::type;
+    const Off colb = (Off)(col * NV * 8), hcolb = (Off)(hcol * NV * 8);
+    auto load = [](const double *plane_base, Off o) {
+        return load_cell<double, NV>(reinterpret_cast<const double *>(reinterpret_cast<const char *>(plane_base) + o), 0);
+    };
+    auto load_u0 = [&](int z) {
+        const double *u = reinterpret_cast<const double *>(reinterpret_cast<const char *>(U0 + (size_t)z * plane * NV) + colb);
+        return STREAM ? load_cell_nt<double, NV>(u, 0) : load_cell<double, NV>(u, 0);
+    };
+    // the plane loaded next, its offset and its ghost sign
+    int zi = 0;
+    size_t zoff = 0;
+    float zs = 1.f;
+    auto seek = [&](int z) {
+        zs = 1.f;
+        zi = map_axis(z, nz, bcz, zs);
+        zoff = (size_t)zi * plane * NV;
+    };
+    auto step = [&](int z) {   // from plane z - 1 to z
+        if constexpr (WALLS) {
+            seek(z);
+        } else {
+            ++zi;
+            zoff = zi == nz ? 0 : zoff + plane * NV;
+            zi = zi == nz ? 0 : zi;
+        }
+    };
+    // this wavefront's rows of the results
+    const int ty0 = __builtin_amdgcn_readfirstlane(ty);
+    const bool active = tx < nx - x0 && y0 + ty < ny;
+    const unsigned pair_bytes = (unsigned)(nx + BX) * NV * 8u;
+    const unsigned off = active ? (unsigned)tx * NV * 8u + (WIDE ? 0u : (unsigned)(ty - ty0) * (unsigned)nx * NV * 8u) : kNoStore;
+    const size_t row0 = (size_t)(y0 + ty0) * nx + x0;
+    auto store = [&](int c, const C &o) {
+        double *row = static_cast<double *>(p.out) + ((size_t)c * plane + row0) * NV;
+        if constexpr (!WIDE) {
+            store_cell_buf<NV, STREAM>(row, pair_bytes, off, o);
+        } else {
+            store_cell_buf<NV, STREAM>(row, BX * NV * 8u, ty == ty0 ? off : kNoStore, o);
+            store_cell_buf<NV, STREAM>(row + (size_t)nx * NV, BX * NV * 8u, ty != ty0 ? off : kNoStore, o);
+        }
+    };
+
+    C q[8];    // ring, slot (plane - zb + 3) & 7: the column's planes c-3 .. c+3 (signed), c+4 as loaded
+    C h[2];    // halo cells of planes c+3, c+4, slot (plane - zb) & 1
+    C e0;      // COMB: base state of plane c
+
+    auto value = [&](C c, float sx, float sy, float sz) -> C {
+        if constexpr (WALLS) apply_bc_sign<double, NV>(c, sx, sy, sz);
+        return c;
+    };
+    auto put = [&](int buf, int y, int x, const C &c) {
+        if constexpr (AC) {
+            lds.q[buf][0][y][x] = make_double2(c.v[0], c.v[1]);
+            lds.q[buf][1][y][x] = make_double2(c.v[2], c.v[3]);
+        } else {
+            lds.q[buf][0][y][x] = c.v[0];
+        }
+    };
+    // In-plane part without the centre's share.  The nearest neighbours, which
+    // carry the largest weight, enter as differences from the centre q0 (exact
+    // for smooth data): B7 = s3 - 6 s2 + 15 (s1 - 2 q0) + 10 q0 per axis, L7 =
+    // -s3 + 2 s2 + 49 (s1 - 2 q0) - 2 q0.
+    // a: the A7 sums, u along x plus v along y, p along x, p along y.
+    const double sLLF = p.s, Kc = p.K, irho = p.invrho;
+    auto in_plane = [&](int buf, const C &q0, double (&o)[NS], double (&a)[3]) {
+#pragma unroll
+        for (int part = 0; part < Tile::NP; ++part) {
+            const auto &P = lds.q[buf][part];
+            auto ring = [&](int k, double wB, double wA, bool first) {
+                const auto xp = P[ty + 3][tx + 3 + k], xm = P[ty + 3][tx + 3 - k];
+                const auto yp = P[ty + 3 + k][tx + 3], ym = P[ty + 3 - k][tx + 3];
+                auto sum = [&](double xpv, double xmv, double ypv, double ymv, double c) {
+                    return k == 1 ? ((xpv - c) + (xmv - c)) + ((ypv - c) + (ymv - c)) : (xpv + xmv) + (ypv + ymv);
+                };
+                auto acc = [&](double &r, double w, double t) { r = first ? t : fma(w, t, r); };
+                if constexpr (AC) {
+                    const double s0 = sum(xp.x, xm.x, yp.x, ym.x, q0.v[2 * part]);
+                    const double s1 = sum(xp.y, xm.y, yp.y, ym.y, q0.v[2 * part + 1]);
+                    acc(o[2 * part], wB, s0);
+                    acc(o[2 * part + 1], wB, s1);
+                    if (part == 0) {
+                        acc(a[1], wA, xp.x - xm.x);
+                        acc(a[2], wA, yp.x - ym.x);
+                        acc(a[0], wA, xp.y - xm.y);
+                    } else {
+                        a[0] = fma(wA, yp.x - ym.x, a[0]);
+                    }
+                } else {
+                    const double s0 = sum(xp, xm, yp, ym, q0.v[0]);
+                    acc(o[0], wB, first ? -s0 : s0);
+                }
+            };
+            ring(3, 1.0, 1.0, true);
+            ring(1, AC ? 15.0 : 49.0, 37.0, false);
+            ring(2, AC ? -6.0 : 2.0, -8.0, false);
+        }
+    };
+
+    // prologue: planes zb-3 .. zb+3 and the halos of the last four all in
+    // flight at once
+    size_t hoff = 0;   // plane of the halo loaded next (those past the chunk are not needed)
+    {
+        C ph[3];
+        float sz[6];
+        seek(zb - 3);
+#pragma unroll
+        for (int k = 0; k < 6; ++k) {
+            q[k] = load(Q + zoff, colb);
+            if (k >= 3) {
+                if (zb + k - 3 < ze) hoff = zoff;
+                ph[k - 3] = load(Q + hoff, hcolb);
+            }
+            sz[k] = zs;
+            step(zb - 2 + k);
+        }
+        q[6] = load(Q + zoff, colb);
+        if (zb + 3 < ze) hoff = zoff;
+        h[1] = load(Q + hoff, hcolb);
+        if constexpr (COMB) e0 = load_u0(zb);
+#pragma unroll
+        for (int k = 0; k < 6; ++k) {
+            q[k] = value(q[k], sgx, sgy, sz[k]);
+            if (k >= 3) put(k - 3, hy, hx, value(ph[k - 3], hsx, hsy, sz[k]));
+        }
+    }
+
+    const double cc = EPI == EPI_RHS ? 1.0 : p.c, cF = AC ? cc * p.inv48h : cc * p.lapc;
+    bool nfbad = false;   // non-finite watch of this thread's outputs
+
+    // iteration of plane c = zb + u (mod 8)
+    auto body = [&](auto uu, int c) {
+        constexpr int u = decltype(uu)::value;
+        const float z3 = zs;   // sign of plane c+3
+        step(c + 4);
+        q[(u + 7) & 7] = load(Q + zoff, colb);
+        if (c + 4 < ze) hoff = zoff;
+        h[u & 1] = load(Q + hoff, hcolb);
+        const C &zm3 = q[u], &zm2 = q[(u + 1) & 7], &zm1 = q[(u + 2) & 7], &q0 = q[(u + 3) & 7];
+        const C &zp1 = q[(u + 4) & 7], &zp2 = q[(u + 5) & 7];
+        C &zp3 = q[(u + 6) & 7];
+        put(u & 3, ty + 3, tx + 3, q0);
+        zp3 = value(zp3, sgx, sgy, z3);
+        __syncthreads();
+        double xy[NS], a[3];
+        in_plane(u & 3, q0, xy, a);
+        // halo of plane c+3 over plane c-1, which everyone has read
+        put((u + 3) & 3, hy, hx, value(h[(u + 1) & 1], hsx, hsy, z3));
+        C r, o;
+        if constexpr (AC) {
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const double s1 = (zp1.v[v] - q0.v[v]) + (zm1.v[v] - q0.v[v]);
+                const double s2 = zp2.v[v] + zm2.v[v], s3 = zp3.v[v] + zm3.v[v];
+                r.v[v] = sLLF * (xy[v] + fma(15.0, s1, fma(30.0, q0.v[v], fma(-6.0, s2, s3))));
+            }
+            auto A = [&](int v) {
+                const double t1 = zp1.v[v] - zm1.v[v], t2 = zp2.v[v] - zm2.v[v], t3 = zp3.v[v] - zm3.v[v];
+                return fma(-8.0, t2, fma(37.0, t1, t3));
+            };
+            r.v[0] = fma(-Kc, a[0] + A(3), r.v[0]);
+            r.v[1] = fma(-irho, a[1], r.v[1]);
+            r.v[2] = fma(-irho, a[2], r.v[2]);
+            r.v[3] = fma(-irho, A(0), r.v[3]);
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                if constexpr (EPI == EPI_RHS) o.v[v] = cF * r.v[v];
+                else if constexpr (EPI == EPI_AXPY) o.v[v] = fma(cF, r.v[v], q0.v[v]);
+                else o.v[v] = fma(cF, r.v[v], fma(p.b, q0.v[v], p.a * e0.v[v]));
+            }
+        } else {
+            const double s1 = (zp1.v[0] - q0.v[0]) + (zm1.v[0] - q0.v[0]);
+            const double s2 = zp2.v[0] + zm2.v[0], s3 = zp3.v[0] + zm3.v[0];
+            const double l = xy[0] + fma(49.0, s1, fma(-6.0, q0.v[0], fma(2.0, s2, -s3)));
+            const double v = q0.v[1];   // du/dt = v (rhs_function.c:330)
+            if constexpr (EPI == EPI_RHS) {
+                o.v[0] = v;
+                o.v[1] = cF * l;
+            } else if constexpr (EPI == EPI_AXPY) {
+                o.v[0] = fma(cc, v, q0.v[0]);
+                o.v[1] = fma(cF, l, v);
+            } else {
+                o.v[0] = fma(cc, v, fma(p.b, q0.v[0], p.a * e0.v[0]));
+                o.v[1] = fma(cF, l, fma(p.b, v, p.a * e0.v[1]));
+            }
+        }
+        if constexpr (COMB) e0 = load_u0(min(c + 1, ze - 1));
+        store(c, o);
+        C w = o;
+#pragma unroll
+        for (int v = 0; v < NV; ++v) w.v[v] = active ? o.v[v] : 0.0;
+        finite_acc<double, NV>(nfbad, w);
+    };
+    for (int c = zb;; c += 8) {
+        body(std::integral_constant<int, 0>{}, c);
+        if (c + 1 >= ze) break;
+        body(std::integral_constant<int, 1>{}, c + 1);
+        if (c + 2 >= ze) break;
+        body(std::integral_constant<int, 2>{}, c + 2);
+        if (c + 3 >= ze) break;
+        body(std::integral_constant<int, 3>{}, c + 3);
+        if (c + 4 >= ze) break;
+        body(std::integral_constant<int, 4>{}, c + 4);
+        if (c + 5 >= ze) break;
+        body(std::integral_constant<int, 5>{}, c + 5);
+        if (c + 6 >= ze) break;
+        body(std::integral_constant<int, 6>{}, c + 6);
+        if (c + 7 >= ze) break;
+        body(std::integral_constant<int, 7>{}, c + 7);
+        if (c + 8 >= ze) break;
     }
     watch_flush(p.nf, nfbad);
 }
@@ -775,129 +1079,6 @@ __device__ __forceinline__ void linear_tile_dma(const LinArgs &p, int x0, int y0
         }
     }
     // every load issued has been waited for by the last iteration (vmcnt 0)
-    watch_flush(p.nf, nfbad);
-}
-
-// The LDS-DMA march for the FP64 WAVE2 system (u, v: 16 bytes per cell, one
-// slot entry), RHS and AXPY stages on all-periodic grids: 6 slots of 13.4 KB,
-// so two 512-thread blocks fit a CU.  du/dt = v, dv/dt = c^2 Lap(u) with the
-// L7 stencil per axis (3d/weno4/plane_wave/rhs_function.c:326-338 with the
-// shipped linear weights).
-struct DmaPlanW2 {
-    static constexpr int NE = DmaPlan::NE;                       // 836 cells per plane
-    static constexpr int SLOT = NE * 16;                         // 13376 bytes
-    static constexpr int NSLOT = 6;
-    static constexpr int NCHUNK = (NE + 63) / 64;                // 14 wavefront loads per plane
-    static constexpr int MAXJ = (NCHUNK + DmaPlan::NWAVE - 1) / DmaPlan::NWAVE;   // 2
-};
-
-template <int EPI>
-__device__ __forceinline__ void linear_tile_dma_w2(const LinArgs &p, int x0, int y0, int zb, unsigned char *ring)
-{
-    using D = DmaPlan;
-    using W = DmaPlanW2;
-    static_assert(EPI == EPI_RHS || EPI == EPI_AXPY, "LDS-DMA march: RHS and AXPY stages");
-    const double *__restrict__ Q = static_cast<const double *>(p.q);
-    double *__restrict__ OUT = static_cast<double *>(p.out);
-    const int nx = p.nx, ny = p.ny, nz = p.nz;
-    const int tx = threadIdx.x, ty = threadIdx.y, tid = ty * D::BX + tx;
-    const int wave = tid >> 6, lane = tid & 63;
-    const int ze = min(zb + p.zc, nz);
-    const bool active = (x0 + tx < nx) && (y0 + ty < ny);
-    const size_t plane = (size_t)nx * ny;
-
-    const int nj = wave + D::NWAVE * (W::MAXJ - 1) < W::NCHUNK ? W::MAXJ : W::MAXJ - 1;
-    uint32_t eoff[W::MAXJ];
-    bool eok[W::MAXJ];
-#pragma unroll
-    for (int j = 0; j < W::MAXJ; ++j) {
-        const int e = (wave + D::NWAVE * j) * 64 + lane;
-        eok[j] = j < nj && e < W::NE;
-        const int r = e / D::RW, c = e - r * D::RW;
-        int gx = x0 + c - 3, gy = y0 + r - 3;
-        gx = gx < 0 ? gx + nx : (gx >= nx ? gx - nx : gx);
-        gy = gy < 0 ? gy + ny : (gy >= ny ? gy - ny : gy);
-        eoff[j] = eok[j] ? (uint32_t)(((size_t)gy * nx + gx) * 2) : 0u;
-    }
-    auto slot_of = [&](int z) { return (z - zb + 3) % W::NSLOT; };
-    auto issue = [&](int z, int slot) {
-        int zz = z % nz;
-        zz = zz < 0 ? zz + nz : zz;
-        const double *src = Q + (size_t)zz * plane * 2;
-        unsigned char *dst = ring + slot * W::SLOT;
-#pragma unroll
-        for (int j = 0; j < W::MAXJ; ++j) {
-            if (j < nj) {
-                const unsigned lds = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)(
-                    (__attribute__((address_space(3))) unsigned char *)(dst + (wave + D::NWAVE * j) * 1024)));
-                const double *g = src + eoff[j];
-                if (eok[j])
-                    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
-                                 :: "s"(lds), "v"(g) : "memory", "m0");
-            }
-        }
-    };
-    // vmcnt: all loads, or all but the nj of the most recent plane
-    auto wait_planes = [&](bool keep_last) {
-        if (!keep_last) __builtin_amdgcn_s_waitcnt(0x0F70);
-        else if (nj == 2) __builtin_amdgcn_s_waitcnt(0x0F72);
-        else __builtin_amdgcn_s_waitcnt(0x0F71);
-    };
-    auto cell_at = [&](int slot, int r, int c) -> double2 {
-        return *reinterpret_cast<const double2 *>(ring + slot * W::SLOT + (r * D::RW + c) * 16);
-    };
-    auto u_at = [&](int slot, int r, int c) -> double {
-        return *reinterpret_cast<const double *>(ring + slot * W::SLOT + (r * D::RW + c) * 16);
-    };
-
-    for (int d = 0; d < W::NSLOT; ++d) issue(zb - 3 + d, d);
-    wait_planes(false);
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-    double2 qz[7];
-#pragma unroll
-    for (int d = 0; d < 6; ++d) qz[d + 1] = cell_at(d, ty + 3, tx + 3);
-    qz[0] = qz[1];
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-    issue(zb + 3, slot_of(zb + 3));
-    if (zb + 4 <= ze + 2) issue(zb + 4, slot_of(zb + 4));
-
-    const double lap = p.lapc;
-    const size_t col = (size_t)(y0 + ty) * nx + (x0 + tx);
-    bool nfbad = false;
-    for (int z = zb; z < ze; ++z) {
-        wait_planes(z + 4 <= ze + 2);
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
-        if (z + 5 <= ze + 2) issue(z + 5, slot_of(z + 5));
-        const int s0 = slot_of(z);
-#pragma unroll
-        for (int k = 0; k < 6; ++k) qz[k] = qz[k + 1];
-        qz[6] = cell_at(slot_of(z + 3), ty + 3, tx + 3);
-        const double q0 = qz[3].x;
-        const double lx = stencil_L7(u_at(s0, ty + 3, tx), u_at(s0, ty + 3, tx + 1), u_at(s0, ty + 3, tx + 2), q0,
-                                     u_at(s0, ty + 3, tx + 4), u_at(s0, ty + 3, tx + 5), u_at(s0, ty + 3, tx + 6));
-        const double ly = stencil_L7(u_at(s0, ty, tx + 3), u_at(s0, ty + 1, tx + 3), u_at(s0, ty + 2, tx + 3), q0,
-                                     u_at(s0, ty + 4, tx + 3), u_at(s0, ty + 5, tx + 3), u_at(s0, ty + 6, tx + 3));
-        const double lz = stencil_L7(qz[0].x, qz[1].x, qz[2].x, q0, qz[4].x, qz[5].x, qz[6].x);
-        Cell<double, 2> r;
-        r.v[0] = qz[3].y;                 // du/dt = v
-        r.v[1] = lap * ((lx + ly) + lz);
-        if (active) {
-            Cell<double, 2> o;
-            if constexpr (EPI == EPI_RHS) {
-                o = r;
-            } else {
-                const double cc = p.c;
-                o.v[0] = qz[3].x + cc * r.v[0];
-                o.v[1] = qz[3].y + cc * r.v[1];
-            }
-            if (p.nf) finite_acc<double, 2>(nfbad, o);
-            __builtin_nontemporal_store(acx_dbl2{o.v[0], o.v[1]},
-                                        reinterpret_cast<acx_dbl2 *>(OUT + ((size_t)z * plane + col) * 2));
-        }
-    }
     watch_flush(p.nf, nfbad);
 }
 
