@@ -19,8 +19,7 @@
 // Layout: a block covers BX x BY reconstruction columns, the outer ring being
 // the face-neighbour halo of the (BX-2) x (BY-2) output tile, and marches a
 // chunk of z-planes with the planes of its stencil region in an LDS ring (the
-// next plane is loaded one iteration ahead into registers and stored after
-// the last read of the slot it replaces).  x-neighbour face states move by
+// next plane is loaded one iteration ahead into registers).  x-neighbour face states move by
 // lane shuffles inside a 32-lane row, y-neighbours through LDS,
 // z-neighbours stay in registers.  k_cweno: the compensated FP32 stage, whose
 // selective mode (per-cell flags) replaces the full CWENO by the linear
@@ -50,16 +49,18 @@ __device__ __forceinline__ void face_flux(int d, const float (&L)[4], const floa
 }
 
 // FP32 compensated stage.  Shared-memory plan of one block (dynamic LDS):
-//   ring  [5][NS][BY+4][BX+4]  planes m-2 .. m+2 of the stencil region
-//   fym   [NS][BY][BX]         -y face state of each reconstruction column
-//   Fy    [NS][BY][BX]         flux through the +y face of each column
+//   ring  [6][NS][BY+4][BX+4]  planes m-2 .. m+3 of the stencil region
+//   fy    [2][NS][2][BY][BX]   -y and +y face states of each reconstruction column
+// Iteration m reads planes m-2 .. m+2 and takes plane m+3 over plane m-3; with
+// two sets of face states and both y fluxes formed by each thread one barrier
+// a plane is enough.
 struct CwLds {
     static constexpr int BX = 32, BY = 16;   // reconstruction columns per block (output tile 30 x 14)
     static constexpr int NS = 4;
     static constexpr int LX = BX + 4, LY = BY + 4;
-    static constexpr int NR = 5;
+    static constexpr int NR = 6;
     static constexpr size_t ring = (size_t)NR * NS * LY * LX;
-    static constexpr size_t bytes = (ring + 2ull * NS * BY * BX) * sizeof(float);
+    static constexpr size_t bytes = (ring + 4ull * NS * BY * BX) * sizeof(float);
 };
 
 // Waves per SIMD the register allocation aims for.  The selective patch
@@ -67,10 +68,10 @@ struct CwLds {
 // tile's march is what counts: one block per CU without spills (2 waves per
 // SIMD) beat two blocks per CU with 60 spilled registers (1.076 against 1.146
 // ms for a steep pulse's step at 256^3, 232 marked tiles, one round either
-// way).  A 256^3 patch is 57 (first stage) to 61 us (last), of which the vector
+// way).  A 256^3 patch is 55 (first stage) to 59 us (last), of which the vector
 // instructions of ten planes issue for about 43; it was 84 us with
 // cweno_weights + cweno_combine, a linear branch of its own and each epilogue
-// load waited for at its place.  The full-grid kernel keeps the registers too.
+// load waited for at its place, and 57 to 61 with two barriers a plane.  The full-grid kernel keeps the registers too.
 template <bool SEL>
 struct CwWaves {
     static constexpr int min_per_simd = SEL ? 2 : 1;
@@ -91,8 +92,7 @@ k_cweno(CwArgs p)
     static_assert(BX == 32, "x exchange uses 32-lane row shuffles");
     extern __shared__ __align__(16) unsigned char smem[];
     T(*ring)[NS][LY][LX] = reinterpret_cast<T(*)[NS][LY][LX]>(smem);
-    T(*s_fym)[BY][BX] = reinterpret_cast<T(*)[BY][BX]>(smem + L::ring * sizeof(T));
-    T(*s_Fy)[BY][BX] = reinterpret_cast<T(*)[BY][BX]>(smem + (L::ring + (size_t)NS * BY * BX) * sizeof(T));
+    T(*s_fy)[NS][2][BY][BX] = reinterpret_cast<T(*)[NS][2][BY][BX]>(smem + L::ring * sizeof(T));
 
     const T *__restrict__ Q = static_cast<const T *>(p.q);
     const T *__restrict__ D = static_cast<const T *>(p.d);
@@ -207,7 +207,7 @@ k_cweno(CwArgs p)
         }
         for (int m = zb - 1; m <= ze; ++m) {
             // the flags of plane m+1 and the epilogue operands of plane m-1
-            const bool pf = m + 3 <= ze + 2;
+            const int set = (m - zb) & 1;
             const uint8_t fl = fl_next;
             if constexpr (SEL) {
                 float s;
@@ -222,7 +222,7 @@ k_cweno(CwArgs p)
                 e2 = load_cell<T, NV>(Q, cell);
             }
             const int sm2 = slot(m - 2), s0 = slot(m - 1), s1 = slot(m), s2 = slot(m + 1), sp2 = slot(m + 2);
-            T fpx[NS], fmx[NS], fpy[NS], fmz[NS], fpz[NS];
+            T fpx[NS], fmx[NS], fpy[NS], fmy[NS], fmz[NS], fpz[NS];
 #pragma unroll
             for (int v = 0; v < NS; ++v) {
                 const T(*P0)[LX] = ring[s0][v];
@@ -272,36 +272,33 @@ k_cweno(CwArgs p)
                 T m3[3], p3[3];
                 cweno_faces<ACX_ACOUSTIC4, T>(get, p, !SEL || ((fl >> v) & 1), m3, p3);
                 fmx[v] = m3[0]; fpx[v] = p3[0];
-                s_fym[v][ty][tx] = m3[1];
-                fpy[v] = p3[1];
+                fmy[v] = m3[1]; fpy[v] = p3[1];
+                s_fy[set][v][0][ty][tx] = m3[1];
+                s_fy[set][v][1][ty][tx] = p3[1];
                 fmz[v] = m3[2]; fpz[v] = p3[2];
                 asm volatile("" ::: "memory");   // one component's stencil live at a time
             }
-            __syncthreads();   // B1: -y states visible; every read of plane m-1 is done
-
-            if (pf) store_plane(m + 3, nxt);   // into the slot of plane m-2
+            // over plane m-3, last read before the barrier of iteration m-1
+            if (m + 3 <= ze + 2) store_plane(m + 3, nxt);
             load_plane(min(m + 4, ze + 2), nxt);
+            __syncthreads();   // y states and plane m+3 visible; every read of plane m-2 is done
 
-            T Fx[NS], Fy[NS];
+            T dxy[NS];
             {
-                T Lf[NS], Rf[NS];
+                T Fx[NS], Fy[NS], Fym[NS], Lf[NS], Rf[NS];
 #pragma unroll
                 for (int v = 0; v < NS; ++v) { Lf[v] = fpx[v]; Rf[v] = __shfl_down(fmx[v], 1, 32); }
                 face_flux(0, Lf, Rf, K, irho, sL, Fx);
+                // rows without a neighbour are no outputs
+                const int up = min(ty + 1, BY - 1), dn = max(ty - 1, 0);
 #pragma unroll
-                for (int v = 0; v < NS; ++v) { Lf[v] = fpy[v]; Rf[v] = ty + 1 < BY ? s_fym[v][ty + 1][tx] : T(0); }
-                face_flux(1, Lf, Rf, K, irho, sL, Fy);
-            }
+                for (int v = 0; v < NS; ++v) Rf[v] = s_fy[set][v][0][up][tx];
+                face_flux(1, fpy, Rf, K, irho, sL, Fy);
 #pragma unroll
-            for (int v = 0; v < NS; ++v) s_Fy[v][ty][tx] = Fy[v];
-            __syncthreads();   // B2: fluxes and plane m+2 visible
-
-            T dxy[NS];
+                for (int v = 0; v < NS; ++v) Lf[v] = s_fy[set][v][1][dn][tx];
+                face_flux(1, Lf, fmy, K, irho, sL, Fym);
 #pragma unroll
-            for (int v = 0; v < NS; ++v) {
-                const T Fxm = __shfl_up(Fx[v], 1, 32);
-                const T Fym = ty > 0 ? s_Fy[v][ty - 1][tx] : T(0);
-                dxy[v] = (Fx[v] - Fxm) + (Fy[v] - Fym);
+                for (int v = 0; v < NS; ++v) dxy[v] = (Fx[v] - __shfl_up(Fx[v], 1, 32)) + (Fy[v] - Fym[v]);
             }
 
             if (m >= zb) {
@@ -361,9 +358,13 @@ k_cweno(CwArgs p)
 // (outputs are 78 % of the reconstructed columns instead of 82 %).  The WAVE2
 // RHS at 70 x 45 x 61 with walls: 31.8 -> 22.0 us.
 //
-// The LDS ring holds four planes, m-1 .. m+2 (each thread keeps its own
-// columns' m-1 and m-2 in registers); the plane m+3 is requested at the start
-// of iteration m and goes into the slot of plane m-1 after it.  x-neighbour
+// The LDS ring holds the four planes m-1 .. m+2 of iteration m (each thread
+// keeps its own columns' m-1 and m-2 in registers) and takes plane m+3, which
+// was requested an iteration before, into a fifth slot; with two sets of the
+// exchanged states one barrier a plane is enough.  Against a 4-plane ring and a
+// second barrier, us per step: ACOUSTIC4 256^3 4408 -> 4400, 64^3 151.7 ->
+// 149.5; WAVE2 70 x 45 x 61 67.6 -> 64.5, 150 x 131 x 90 160 -> 154, 256^3 1338
+// -> 1352.  x-neighbour
 // face states move by lane shuffles inside a 32-lane row; y-neighbour states
 // and, across the two halves of the block, the coupled states (p with v at
 // y faces, p with w at z faces; p with u at x faces are in one thread) go
@@ -378,11 +379,11 @@ struct Cw64 {
     static constexpr int WPE = SYS == ACX_ACOUSTIC4 ? 3 : 4;  // waves per SIMD
     static constexpr int LX = BX + 4, LY = BY + 4, NREG = LX * LY;
     static constexpr int CS = NREG + 4;                       // doubles per component of a slot
-    static constexpr int NR = 4;
+    static constexpr int NR = 5;
     static constexpr int SLOT = NS * CS;
     static constexpr int EX = NS * 2 * NCOL;                  // -y and +y face states
     static constexpr int EZ = SYS == ACX_ACOUSTIC4 ? 2 * NCOL : 0;   // p and w sums at the lower z face
-    static constexpr size_t bytes = (size_t)(NR * SLOT + EX + EZ) * sizeof(double);
+    static constexpr size_t bytes = (size_t)(NR * SLOT + 2 * (EX + EZ)) * sizeof(double);
     static constexpr int NLD = NREG * NV / 2;                 // 16-byte loads of one plane
     static constexpr int PER = (NLD + NT - 1) / NT;
 };
@@ -396,8 +397,7 @@ k_cweno64(CwArgs p)
     constexpr bool AC = SYS == ACX_ACOUSTIC4;
     extern __shared__ __align__(16) unsigned char smem[];
     double *const ring = reinterpret_cast<double *>(smem);
-    double *const s_y = ring + L::NR * L::SLOT;   // [component][-y, +y][column]
-    double *const s_z = s_y + L::EX;              // [p, w][column]
+    double *const s_ex = ring + L::NR * L::SLOT;   // two sets of the exchanged states
 
     const double *__restrict__ Q = static_cast<const double *>(p.q);
     const double *__restrict__ U0 = static_cast<const double *>(p.u0);
@@ -467,29 +467,25 @@ k_cweno64(CwArgs p)
     };
     const int cen = (ty + 2) * LX + tx + 2 + v0 * L::CS;   // own column, first own component
 
-    // prologue: planes zb-3 .. zb+1 through the ring; zb-3 only feeds the
-    // column values of iteration zb-1, so its slot is reused for zb+1
+    // prologue: planes zb-3 .. zb+2 in flight at once; zb-3 only feeds the
+    // column values of iteration zb-1, so its slot is the one of zb+2
     double um1[NC], um2[NC];
+    acx_dbl2 nxt[PER];
+    float nsz;
     {
-        acx_dbl2 b0[PER], b1[PER], b2[PER];
-        float s0, s1, s2;
-        load_plane(zb - 3, b0, s0);
-        load_plane(zb - 2, b1, s1);
-        load_plane(zb - 1, b2, s2);
-        store_plane(3, b0, s0);
-        store_plane(0, b1, s1);
-        store_plane(1, b2, s2);
-        load_plane(zb, b1, s1);
+        acx_dbl2 b[5][PER];
+        float sz[5];
+#pragma unroll
+        for (int k = 0; k < 5; ++k) load_plane(zb - 3 + k, b[k], sz[k]);
+        load_plane(zb + 2, nxt, nsz);
+#pragma unroll
+        for (int k = 0; k < 5; ++k) store_plane((k + 4) % L::NR, b[k], sz[k]);
         __syncthreads();
 #pragma unroll
         for (int k = 0; k < NC; ++k) {
-            um2[k] = ring[3 * L::SLOT + cen + k * L::CS];
+            um2[k] = ring[4 * L::SLOT + cen + k * L::CS];
             um1[k] = ring[cen + k * L::CS];
         }
-        load_plane(zb + 1, b0, s0);
-        __syncthreads();
-        store_plane(2, b1, s1);
-        store_plane(3, b0, s0);
         __syncthreads();
     }
 
@@ -500,17 +496,16 @@ k_cweno64(CwArgs p)
     double vcen = 0.0, vcen_prev = 0.0;
     bool nfbad = false;
     int slot = 0;   // of plane m-1
+    auto after = [](int s, int k) { return s + k < L::NR ? s + k : s + k - L::NR; };
     for (int m = zb - 1; m <= ze; ++m) {
-        acx_dbl2 nxt[PER];
-        float nsz = 1.f;
-        const bool pf = m + 3 <= ze + 2;
-        if (pf) load_plane(m + 3, nxt, nsz);
+        double *const s_y = s_ex + ((m - zb) & 1) * (L::EX + L::EZ);   // [component][-y, +y][column]
+        double *const s_z = s_y + L::EX;                               // [p, w][column]
         if constexpr (!AC) {
             float s = 1.f;
             vcen = Q[((size_t)map_axis(m, nz, kz, s) * plane + ocol) * NV + 1];
         }
-        const double *R0 = ring + slot * L::SLOT + cen, *R1 = ring + ((slot + 1) & 3) * L::SLOT + cen;
-        const double *R2 = ring + ((slot + 2) & 3) * L::SLOT + cen, *R3 = ring + ((slot + 3) & 3) * L::SLOT + cen;
+        const double *R0 = ring + slot * L::SLOT + cen, *R1 = ring + after(slot, 1) * L::SLOT + cen;
+        const double *R2 = ring + after(slot, 2) * L::SLOT + cen, *R3 = ring + after(slot, 3) * L::SLOT + cen;
         double fmx[NC], fpx[NC], F[NC];   // F: twice the flux at the face between planes m-1 and m
 #pragma unroll
         for (int k = 0; k < NC; ++k) {
@@ -569,6 +564,10 @@ k_cweno64(CwArgs p)
             asm volatile("" ::: "memory");   // one component's stencil live at a time
         }
 
+        // plane m+3, over plane m-2 (last read before the barrier of iteration
+        // m-1; this iteration's barrier makes it visible)
+        if (m + 3 <= ze + 2) store_plane(after(slot, 4), nxt, nsz);
+        if (m + 4 <= ze + 2) load_plane(m + 4, nxt, nsz);
         // the base state of plane m-1, requested where the registers of the
         // stencils are free again and ahead of the exchange: waited for at its use,
         // right after its load, it cost a memory latency a plane (combining stage
@@ -600,9 +599,8 @@ k_cweno64(CwArgs p)
 #pragma unroll
             for (int k = 0; k < NC; ++k) d[k] = G[k] - __shfl_up(G[k], 1, 32);
         }
-        __syncthreads();   // B1: exchanged states visible; every read of plane m-1 is done
+        __syncthreads();   // exchanged states and plane m+3 visible; every read of plane m-1 is done
 
-        if (pf) store_plane(slot, nxt, nsz);   // into the slot of plane m-1
         // y: both faces from the neighbours' states
         {
             const int up = ty + 1 < BY ? colid + BX : colid, dn = ty > 0 ? colid - BX : colid;
@@ -657,8 +655,7 @@ k_cweno64(CwArgs p)
             Fz_prev[k] = F[k];
         }
         vcen_prev = vcen;
-        slot = (slot + 1) & 3;
-        __syncthreads();   // B2: plane m+3 visible; the exchanged states are read
+        slot = after(slot, 1);
     }
     watch_flush(p.nf, nfbad);
 }
