@@ -21,15 +21,15 @@ namespace acx {
 
 // FP64 march (acx_linear_core.h).  WALLS = false is the all-periodic
 // instantiation (no ghost signs, offsets inside a plane in 32 bits).
-template <int SYS, int EPI, bool WALLS, int MEM>
-__global__ void __launch_bounds__(512)
+template <int SYS, int EPI, bool WALLS, int MEM, int ROWS>
+__global__ void __launch_bounds__(32 * ROWS) __attribute__((amdgpu_waves_per_eu(2)))
 k_linear64(LinArgs p)
 {
-    using Tile = Tile64<SYS>;
+    using Tile = Tile64<SYS, ROWS>;
     __shared__ typename Tile::Lds lds;
     const int tile = xcd_logical_tile(blockIdx.x, gridDim.x);
     const int x0 = (tile % p.ntx) * Tile::BX, y0 = ((tile / p.ntx) % p.nty) * Tile::BY, zb = (tile / (p.ntx * p.nty)) * p.zc;
-    linear_tile64<SYS, EPI, WALLS, MEM>(p, x0, y0, zb, lds);
+    linear_tile64<SYS, EPI, WALLS, MEM, ROWS>(p, x0, y0, zb, lds);
 }
 
 // Centre-plane march with the 5-plane halo ring (acx_linear_core.h), FP64
@@ -86,19 +86,20 @@ static int launch_linear_dma(const LinArgs &a, hipStream_t s)
 
 // ---------------------------------------------------------------------------
 
-// One round model for both marches.  Slots are the CUs, also where two blocks
-// of the WAVE2 kernel fit one: with chunks half as long the WAVE2 stages of 256^3
-// took 159 us (combining) and 84.6 (the others) instead of 139 and 79.7.
-template <int SYS, int EPI, bool WALLS, int MEM>
+// Slots of the round model: the CUs, or two blocks per CU with 8 rows.  (Two
+// for the 16-row WAVE2 kernel, whose registers would allow it, halves its
+// chunks: 256^3 159 us for the combining stage and 84.6 for the others, against
+// 139 and 79.7.)
+template <int SYS, int EPI, bool WALLS, int MEM, int ROWS = 16>
 static int launch_linear64_w(const LinArgs &a, hipStream_t s)
 {
-    using Tile = Tile64<SYS>;
+    using Tile = Tile64<SYS, ROWS>;
     LinArgs b = a;
     b.ntx = (a.nx + Tile::BX - 1) / Tile::BX;
     b.nty = (a.ny + Tile::BY - 1) / Tile::BY;
-    if (b.zc <= 0) b.zc = auto_zc(b.ntx, b.nty, a.nz, device_cus(), 10);
+    if (b.zc <= 0) b.zc = auto_zc(b.ntx, b.nty, a.nz, device_cus() * (16 / ROWS), 10);
     b.ntz = (a.nz + b.zc - 1) / b.zc;
-    hipLaunchKernelGGL((k_linear64<SYS, EPI, WALLS, MEM>), dim3(b.ntx * b.nty * b.ntz), dim3(Tile::BX, Tile::BY), 0, s, b);
+    hipLaunchKernelGGL((k_linear64<SYS, EPI, WALLS, MEM, ROWS>), dim3(b.ntx * b.nty * b.ntz), dim3(Tile::BX, Tile::BY), 0, s, b);
     return hip_check(hipGetLastError(), "k_linear64 launch");
 }
 
@@ -188,13 +189,22 @@ static int launch_linear32(const LinArgs &a, hipStream_t s)
 //   WAVE2 192^3       217, 208       195, 195        195, 192
 //   WAVE2 224^3       318, 346       317, 317        333, 333
 //   WAVE2 384^3       1679, 1758     1683, 1674      1778, 1768
-constexpr size_t CACHED_BYTES = 128ull << 20;
+//
+// Up to HALF_TILE_BYTES tiles of 8 rows, whose two blocks per CU have a barrier
+// of their own each; above, their larger halo costs more.  8 against 16 rows, us
+// per step: ACOUSTIC4 64^3 32.3, 33.5; 150 x 131 x 90 (54 MB) 108, 114; 200 x 150
+// x 100 (96 MB) 202, 195.  WAVE2 96^3 33.2, 35.4; 200 x 150 x 100 (48 MB) 83.1,
+// 86.7.
+constexpr size_t CACHED_BYTES = 128ull << 20, HALF_TILE_BYTES = 64ull << 20;
 
 template <int SYS, int EPI>
 static int launch_linear64(const LinArgs &a, hipStream_t s)
 {
     const bool walls = a.bc[0] != ACX_PERIODIC || a.bc[1] != ACX_PERIODIC || a.bc[2] != ACX_PERIODIC;
-    const size_t plane_bytes = (size_t)a.nx * a.ny * Tile64<SYS>::NV * 8;
+    const size_t plane_bytes = (size_t)a.nx * a.ny * Tile64<SYS, 16>::NV * 8;
+    if (plane_bytes * a.nz <= HALF_TILE_BYTES)
+        return walls ? launch_linear64_w<SYS, EPI, true, MEM_CACHED, 8>(a, s)
+                     : launch_linear64_w<SYS, EPI, false, MEM_CACHED, 8>(a, s);
     if (plane_bytes * a.nz <= CACHED_BYTES)
         return walls ? launch_linear64_w<SYS, EPI, true, MEM_CACHED>(a, s)
                      : launch_linear64_w<SYS, EPI, false, MEM_CACHED>(a, s);

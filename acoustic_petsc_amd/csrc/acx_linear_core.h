@@ -557,10 +557,10 @@ __device__ __forceinline__ void linear_tile_centre(const LinArgs &p, int x0, int
 //   together with the columns, 45.
 //   LDS: an ACOUSTIC4 cell as two 16-byte halves, (p, u) and (v, w), in
 //   arrays of their own, so that neighbouring lanes read neighbouring words.
-//   Tile: 32 x 16 columns (a wavefront is two rows of 32).
-template <int SYS>
+//   Tile: 32 x 16 columns (a wavefront is two rows of 32), or 32 x 8.
+template <int SYS, int ROWS>
 struct Tile64 {
-    static constexpr int BX = 32, BY = 16;
+    static constexpr int BX = 32, BY = ROWS;
     static constexpr int NV = SYS == ACX_ACOUSTIC4 ? 4 : 2;   // components in memory
     static constexpr int NS = SYS == ACX_ACOUSTIC4 ? 4 : 1;   // components in the stencil
     static constexpr int LX = BX + 6, LY = BY + 6;
@@ -593,10 +593,10 @@ __device__ __forceinline__ void store_cell_buf(double *row, unsigned bytes, unsi
 // rows).
 enum { MEM_CACHED = 0, MEM_STREAM = 1, MEM_WIDE = 2 };
 
-template <int SYS, int EPI, bool WALLS, int MEM>
-__device__ __forceinline__ void linear_tile64(const LinArgs &p, int x0, int y0, int zb, typename Tile64<SYS>::Lds &lds)
+template <int SYS, int EPI, bool WALLS, int MEM, int ROWS>
+__device__ __forceinline__ void linear_tile64(const LinArgs &p, int x0, int y0, int zb, typename Tile64<SYS, ROWS>::Lds &lds)
 {
-    using Tile = Tile64<SYS>;
+    using Tile = Tile64<SYS, ROWS>;
     constexpr int NV = Tile::NV, NS = Tile::NS, BX = Tile::BX, BY = Tile::BY;
     constexpr bool AC = SYS == ACX_ACOUSTIC4, COMB = EPI == EPI_COMB, STREAM = MEM != MEM_CACHED, WIDE = MEM == MEM_WIDE;
     using C = Cell<double, NV>;

@@ -103,3 +103,28 @@ def test_rows_of_two_gigabytes(acx, torch_gpu):
     ref = F.view(4, 1, m, 2)
     for j in range(0, k, 4096):   # the same arithmetic: equal to the last bit
         assert torch.equal(got[:, j:j + 4096], ref.expand(4, 4096, m, 2))
+
+
+@pytest.mark.parametrize("system, rep", [("acoustic4", (3, 3, 2)), ("wave2", (3, 3, 4))])
+@pytest.mark.parametrize("bc", [(0, 0, 0), (0, 0, 2)])
+def test_cached_fields_on_sixteen_rows(system, rep, bc, acx, orc, torch_gpu):
+    """Fields of 64 to 128 MB: 16-row tiles, cached results; the small field takes
+    8-row tiles.  The same arithmetic per cell."""
+    torch = torch_gpu
+    kw = dict(h=1.0 / 32, system=acx.ACOUSTIC4 if system == "acoustic4" else acx.WAVE2)
+    bc = tuple(int(k != 0) for k in bc) if system == "wave2" else bc
+    n = (75, 45, 40) if not any(bc) else (75, 45, 40 * rep[2])
+    rep = rep if not any(bc) else (rep[0], rep[1], 1)
+    N = tuple(a * b for a, b in zip(n, rep))
+    small, big = acx.Grid(n=n, bc=bc, **kw), acx.Grid(n=N, bc=bc, **kw)
+    print(f"[case] 16-row tiles n={N} {system} bc={bc}", flush=True)
+    U = make_field(acx, small, 47, "rough")
+    assert rel_l2(acx.rhs(small, torch.from_numpy(U).cuda()).cpu().numpy(), orc.rhs3d(orc_grid(orc, small), U)) <= TOL
+    U, U0 = torch.from_numpy(U).cuda(), torch.from_numpy(make_field(acx, small, 48, "rough")).cuda()
+    B, B0 = _repeat(U, rep), _repeat(U0, rep)
+    assert 64 << 20 < B.numel() * 8 <= 128 << 20 and U.numel() * 8 <= 64 << 20
+    for a, b, c in ((0.0, 0.0, 1.0), (0.0, 1.0, 0.01), (2.0 / 3.0, 1.0 / 3.0, 0.02)):
+        out, ref = torch.empty_like(B), torch.empty_like(U)
+        acx.stage(big, B, B0 if a else None, out, a, b, c)
+        acx.stage(small, U, U0 if a else None, ref, a, b, c)
+        assert torch.equal(out, _repeat(ref, rep))
