@@ -30,7 +30,7 @@ int env_int(const char *name, int dflt)
 }
 
 // Automatic z-chunk of a 2.5D march.  A launch runs in ceil(workgroups /
-// slots) rounds (slots = CUs x workgroups that fit a CU), each about as long
+// slots) rounds (slots = CUs, or places for workgroups), each about as long
 // as one workgroup's march of zc planes plus a fixed start of `start` planes'
 // worth (z-halo planes, prologue); of the even divisions of the planes the one
 // that minimises rounds x (zc + start) is taken, the longer march on a tie.
@@ -39,7 +39,9 @@ int env_int(const char *name, int dflt)
 // a 32^3 WAVE2 step 34 -> 21 us (8 planes: 8 workgroups; 1 plane: 64), the
 // FP32 step at 384^3 2.57 -> 2.50 ms (77 planes instead of 128); the same
 // chunk as before at 256^3.
-int auto_zc(int ntx, int nty, int nz, int slots, int start, double *cost_out)
+// pair > 0: a slot holds two workgroups, which then take `pair` times as long
+// as one alone.
+int auto_zc(int ntx, int nty, int nz, int slots, int start, double *cost_out, double pair)
 {
     int best = nz, prev = 0;
     double best_cost = -1.0;
@@ -48,8 +50,12 @@ int auto_zc(int ntx, int nty, int nz, int slots, int start, double *cost_out)
         if (z == prev) continue;
         prev = z;
         const long long wg = (long long)ntx * nty * ((nz + z - 1) / z);
-        const long long rounds = (wg + slots - 1) / slots;
-        const double cost = (double)rounds * (z + start);
+        double rounds = (double)((wg + slots - 1) / slots);
+        if (pair > 0.0) {
+            const long long full = wg / (2LL * slots), rest = wg - full * 2 * slots;
+            rounds = (double)full * pair + (rest == 0 ? 0.0 : rest <= slots ? 1.0 : pair);
+        }
+        const double cost = rounds * (z + start);
         if (best_cost < 0 || cost < best_cost) {
             best_cost = cost;
             best = z;
