@@ -5,6 +5,7 @@
 #include <type_traits>
 #include "acx_device.h"
 #include "acx_internal.h"
+#include "acx_plan.h"
 
 namespace acx {
 
@@ -917,10 +918,8 @@ __device__ __forceinline__ void linear_tile_dma(const LinArgs &p, int x0, int y0
         const int e = (wave + D::NWAVE * j) * 64 + lane;
         eok[j] = j < nj && e < D::NENT;
         const int h = e / D::NE, idx = e - h * D::NE, r = idx / D::RW, c = idx - r * D::RW;
-        int gx = x0 + c - 3, gy = y0 + r - 3;
-        gx = gx < 0 ? gx + nx : (gx >= nx ? gx - nx : gx);
-        gy = gy < 0 ? gy + ny : (gy >= ny ? gy - ny : gy);
-        eoff[j] = eok[j] ? (uint32_t)(((size_t)gy * nx + gx) * 4 + 2 * h) : 0u;
+        // in 32 bits: the launcher takes planes below 2^31 doubles
+        eoff[j] = eok[j] ? region_cell(x0, y0, 3, r, c, nx, ny) * 4u + 2u * h : 0u;
     }
     auto slot_of = [&](int z) { return (z - zb + 3) % D::NSLOT; };
     auto issue = [&](int z, int slot) {

@@ -128,3 +128,25 @@ def test_cached_fields_on_sixteen_rows(system, rep, bc, acx, orc, torch_gpu):
         acx.stage(big, B, B0 if a else None, out, a, b, c)
         acx.stage(small, U, U0 if a else None, ref, a, b, c)
         assert torch.equal(out, _repeat(ref, rep))
+
+
+@pytest.mark.parametrize("nx, ny", [(1100, 4), (1100, 9), (1100, 17), (4, 1100), (17, 1100), (33, 1100)])
+def test_narrow_grids_above_the_cache(nx, ny, acx, orc, torch_gpu):
+    """Planes narrower than the staged region of a tile (38 x 22 cells), where
+    its last rows or columns lie more than one period past the grid."""
+    torch = torch_gpu
+    kw = dict(h=1.0 / 32, system=acx.ACOUSTIC4)
+    nz = 10
+    rep = (128 << 20) // (nx * ny * nz * 32) + 1
+    small, big = acx.Grid(n=(nx, ny, nz), **kw), acx.Grid(n=(nx, ny, nz * rep), **kw)
+    print(f"[case] narrow march n={big.n}", flush=True)
+    U = make_field(acx, small, 49, "rough")
+    F = torch.from_numpy(orc.rhs3d(orc_grid(orc, small), U)).cuda()
+    U = torch.from_numpy(U).cuda()
+    B = _repeat(U, (1, 1, rep))
+    assert B.numel() * 8 > 128 << 20
+    rel = lambda x, y: float((x - y).norm() / y.norm())  # noqa: E731
+    assert rel(acx.rhs(big, B), _repeat(F, (1, 1, rep))) <= TOL
+    out = torch.empty_like(B)
+    acx.stage(big, B, None, out, 0.0, 1.0, 0.01)
+    assert rel(out, B + 0.01 * _repeat(F, (1, 1, rep))) <= TOL

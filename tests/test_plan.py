@@ -1,0 +1,53 @@
+"""The index and launch rules of csrc/acx_plan.h, compiled for the host: what a
+kernel reads and what a launcher chooses, from sizes alone.  Each case is a
+small program that says nothing when the rule holds.
+"""
+import os
+import subprocess
+
+import pytest
+
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "acoustic_petsc_amd", "csrc")
+
+PROLOGUE = """
+#include <cstdio>
+#include <cstdlib>
+#include "acx_plan.h"
+using namespace acx;
+#define CHECK(c, ...) do { if (!(c)) { std::printf(__VA_ARGS__); std::printf("\\n"); std::exit(1); } } while (0)
+"""
+
+
+@pytest.fixture
+def run_host(tmp_path):
+    def run(body, timeout=60):
+        src, exe = tmp_path / "t.cpp", tmp_path / "t"
+        src.write_text(PROLOGUE + body)
+        subprocess.run(["g++", "-std=c++17", "-O2", "-Wall", "-Werror", f"-I{CSRC}", str(src), "-o", str(exe)], check=True)
+        r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=timeout)
+        assert r.returncode == 0 and r.stdout == "", r.stdout
+    return run
+
+
+# tile and staged region (x, y) of the FP64 LDS-DMA march
+@pytest.mark.parametrize("bx, by, halo", [(32, 16, 3)])
+def test_staged_regions_name_cells_of_the_plane(bx, by, halo, run_host):
+    """Every cell of every tile's region exists, and the cells a stencil needs
+    (up to `halo` around a column of the grid) are the periodic ones."""
+    run_host(f"""
+int main()
+{{
+    const int bx = {bx}, by = {by}, h = {halo};
+    for (int nx = 1; nx <= 70; ++nx)
+        for (int ny = 1; ny <= 70; ++ny)
+            for (int y0 = 0; y0 < ny; y0 += by)
+                for (int x0 = 0; x0 < nx; x0 += bx)
+                    for (int r = 0; r < by + 2 * h; ++r)
+                        for (int c = 0; c < bx + 2 * h; ++c) {{
+                            const uint32_t q = region_cell(x0, y0, h, r, c, nx, ny);
+                            CHECK(q < (uint32_t)(nx * ny), "%d x %d, tile %d %d, row %d column %d: cell %u", nx, ny, x0, y0, r, c, q);
+                            const int x = x0 - h + c, y = y0 - h + r;
+                            CHECK(((int)(q % nx) - x) % nx == 0 && ((int)(q / nx) - y) % ny == 0, "%d x %d: %d %d -> %u", nx, ny, x, y, q);
+                        }}
+}}
+""")
