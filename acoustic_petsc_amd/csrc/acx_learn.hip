@@ -14,6 +14,7 @@
 #include "acx_device.h"
 #include "acx_internal.h"
 #include "acx_cweno_core.h"
+#include "acx_plan.h"
 #include "../../include/acx_learn.h"
 
 namespace acx {
@@ -172,14 +173,23 @@ __global__ void __launch_bounds__(JT_BX *JT_BY) k_judge(const float *__restrict_
     const int tx = threadIdx.x, ty = threadIdx.y, tid = ty * JT_BX + tx;
     const bool active = x0 + tx < nx && y0 + ty < ny;
     const size_t plane = (size_t)nx * ny;
-    auto wrap = [](int q, int n) { return q < 0 ? q + n : (q >= n ? q - n : q); };
+    // the cells of the stencil region this thread loads
+    constexpr int PER = (JT_LX * JT_LY + JT_BX * JT_BY - 1) / (JT_BX * JT_BY);
+    uint32_t rcell[PER];
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+        const int c = tid + u * JT_BX * JT_BY;
+        rcell[u] = region_cell(x0, y0, 2, c / JT_LX, c % JT_LX, nx, ny);
+    }
     // the stencil region of plane zz into ring slot sl (float4 loads, one cell per thread and pass)
     auto load_plane = [&](int zz, int sl) {
         const size_t zo = (size_t)wrap(zz, nz) * plane;
-        for (int c = tid; c < JT_LX * JT_LY; c += JT_BX * JT_BY) {
+#pragma unroll
+        for (int u = 0; u < PER; ++u) {
+            const int c = tid + u * JT_BX * JT_BY;
+            if (c >= JT_LX * JT_LY) break;
             const int ly = c / JT_LX, lx = c - ly * JT_LX;
-            const int gx = wrap(x0 + lx - 2, nx), gy = wrap(y0 + ly - 2, ny);
-            const float4 v = *reinterpret_cast<const float4 *>(HI + (zo + (size_t)gy * nx + gx) * 4);
+            const float4 v = *reinterpret_cast<const float4 *>(HI + (zo + rcell[u]) * 4);
             ring[sl][0][ly][lx] = v.x;
             ring[sl][1][ly][lx] = v.y;
             ring[sl][2][ly][lx] = v.z;

@@ -444,3 +444,28 @@ def test_judge_labels_match_the_fp64_labels(acx, torch_gpu):
     print(f"[case] judge vs FP64 labels: {int(differ.sum())} differ, {int(lab64.sum())} labelled", flush=True)
     assert int(lab64.sum()) > 0
     assert bool((~differ | near).all())
+
+
+@pytest.mark.parametrize("n", [(5, 5, 5), (7, 9, 6), (16, 5, 17), (17, 6, 5)])
+def test_judge_of_narrow_grids_equals_their_repetition(n, acx, torch_gpu):
+    """Grids narrower than the judge's 36 x 12 staged region against the same
+    periodic field repeated along every axis: the same cells, the same bits."""
+    torch = torch_gpu
+    from acoustic_petsc_amd import learn
+    rep = (8, 3, 2)
+    kw = dict(h=1.0 / 16, gamma_hi=0.85, gamma_lo=0.85)
+    N = tuple(a * b for a, b in zip(n, rep))
+    rng = np.random.default_rng(3)
+    u = np.where(rng.random((n[2], n[1], n[0], 4)) < 0.3, 1.0, 0.1) + 0.01 * rng.standard_normal((n[2], n[1], n[0], 4))
+    U = torch.from_numpy(u.astype(np.float32)).cuda()
+    B = U.repeat(rep[2], rep[1], rep[0], 1).contiguous()
+    print(f"[case] judge narrow n={n}", flush=True)
+
+    def judged(m, X):
+        g = acx.Grid(n=m, **kw)
+        return learn.judge(g, X, used=torch.zeros(g.ncells, dtype=torch.uint8, device="cuda"))
+
+    out, miss, worst = judged(n, U)
+    bout, bmiss, bworst = judged(N, B)
+    assert torch.equal(bout.view(N[2], N[1], N[0]), out.view(n[2], n[1], n[0]).repeat(rep[2], rep[1], rep[0]))
+    assert bmiss == miss * rep[0] * rep[1] * rep[2] and bworst == worst and miss > 0

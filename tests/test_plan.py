@@ -29,8 +29,8 @@ def run_host(tmp_path):
     return run
 
 
-# tile and staged region (x, y) of the FP64 LDS-DMA march
-@pytest.mark.parametrize("bx, by, halo", [(32, 16, 3)])
+# tile and halo of the FP64 LDS-DMA march and of the judge of the selective step
+@pytest.mark.parametrize("bx, by, halo", [(32, 16, 3), (32, 8, 2)])
 def test_staged_regions_name_cells_of_the_plane(bx, by, halo, run_host):
     """Every cell of every tile's region exists, and the cells a stencil needs
     (up to `halo` around a column of the grid) are the periodic ones."""
