@@ -12,6 +12,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include "acx_plan.h"
 
 namespace acx {
 
@@ -42,7 +43,6 @@ __device__ __forceinline__ int map_axis(int i, int n, int kind, float &sign)
 // round-robin (id % 8); each XCD has its own L2.  Give XCD x a contiguous run
 // of logical tiles so that tiles sharing halo planes are resident on the
 // same L2 at the same time.  Bijective for any workgroup count.
-constexpr int kNumXcd = 8;
 __device__ __forceinline__ int xcd_logical_tile(int id, int nb)
 {
     const int xcd = id % kNumXcd, slot = id / kNumXcd;

@@ -1,43 +1,25 @@
 // acx_ensemble.hip -- persistent-kernel stepping of a batch of independent
 // acoustic problems (include/acx_ensemble.h).
 //
-// Work items are (problem, column tile, z-chunk) triples.  The schedule of a
-// configuration is made on the host: each XCD gets a contiguous run of the
-// items with an eighth of the work, so that neighbouring tiles meet in its L2,
-// and each workgroup of the XCD a list of them, the longest items handed out
-// first and each to the workgroup with the least so far.  The kernel runs
-// its list with the same tile code as the per-grid linear kernel
-// (acx_linear_core.h).  (A queue per XCD drawn from with atomics cost more
-// than the tiles' differences in speed: at the end of a stage every workgroup
-// finds eight queues empty, 4000 atomics on one line, about 40 us.)
+// The schedule of a configuration is made on the host
+// (acx_ensemble_plan.h); the kernel runs its workgroup's list with the same
+// tile code as the per-grid linear kernel (acx_linear_core.h).  (A queue per
+// XCD drawn from with atomics cost more than the tiles' differences in speed:
+// at the end of a stage every workgroup finds eight queues empty, 4000 atomics
+// on one line, about 40 us.)
 #include <algorithm>
 #include <exception>
-#include <functional>
-#include <queue>
 #include <stdlib.h>
 #include <string.h>
 #include <vector>
+#include "acx_ensemble_plan.h"
 #include "acx_linear_core.h"
 #include "../../include/acx_ensemble.h"
 
 namespace acx {
 
-struct EnsProblem {
-    size_t off;          // first cell
-    int n[3];
-    int ntx, nty, ntz;
-    int zc;              // planes per work item
-};
-
-struct EnsItem {
-    int prob;            // index into the problem table
-    int tile;            // column tile and z-chunk, x fastest, then y, then z
-};
-
-constexpr int ENS_BX = 64;
 constexpr int ENS_MAXP = 256;
 
-struct EnsConfig { int by, zc; };
 constexpr int ENS_NCONFIG = 8;
 static const EnsConfig kConfigs[ENS_NCONFIG] = {{8, 16}, {8, 32}, {8, 64}, {12, 16}, {12, 32}, {12, 64},
                                                 {8, 128}, {12, 128}};
@@ -91,28 +73,17 @@ struct acx_ensemble {
     float *hi[2], *lo[2], *d0, *d1;
     int cur;                           // index of the current (hi, lo)
     int config;
-    int blocks[2][3];                  // persistent grid per rows-per-tile variant (8, 12) and stage kind
+    int grid[2];                       // workgroups each schedule is made for
+    int fit[2][2];                     // the same that fit at once, per rows-per-tile variant (8, 12)
     hipGraphExec_t graph;
     double graph_dt;
     int graph_config, graph_cur;
     hipStream_t graph_stream;
 };
 
-// The problems of a configuration: each one's planes divided evenly into
-// chunks of at most the configuration's zc.
 static std::vector<EnsProblem> ens_problems(const acx_ensemble *e, const EnsConfig &c)
 {
-    std::vector<EnsProblem> probs(e->nprob);
-    for (int p = 0; p < e->nprob; ++p) {
-        EnsProblem &q = probs[p];
-        for (int d = 0; d < 3; ++d) q.n[d] = e->dims[3 * p + d];
-        q.off = e->off[p];
-        q.ntx = (q.n[0] + ENS_BX - 1) / ENS_BX;
-        q.nty = (q.n[1] + c.by - 1) / c.by;
-        q.ntz = (q.n[2] + c.zc - 1) / c.zc;
-        q.zc = (q.n[2] + q.ntz - 1) / q.ntz;
-    }
-    return probs;
+    return ens_problems(e->dims, e->off, c);
 }
 
 static size_t ens_count(const std::vector<EnsProblem> &probs)
@@ -122,67 +93,20 @@ static size_t ens_count(const std::vector<EnsProblem> &probs)
     return n;
 }
 
-// Lists of the items per workgroup (blocks b, b + 8, ... run on XCD b % 8);
-// returns the work of the busiest, zc + 10 planes per item.
-static double ens_schedule(const std::vector<EnsProblem> &probs, int blocks, std::vector<EnsItem> &items,
-                           std::vector<int> &first)
-{
-    std::vector<EnsItem> all;
-    double work = 0.0, most = 0.0;
-    for (int p = 0; p < (int)probs.size(); ++p) {
-        const int n = probs[p].ntx * probs[p].nty * probs[p].ntz;
-        for (int t = 0; t < n; ++t) all.push_back({p, t});
-        work += (double)n * (probs[p].zc + 10);
-    }
-    std::vector<std::vector<EnsItem>> list(blocks);
-    size_t k = 0;
-    double done = 0.0;
-    for (int x = 0; x < kNumXcd; ++x) {
-        // this XCD's share of the items, longest first
-        std::vector<EnsItem> part;
-        const double upto = work * (x + 1) / kNumXcd;
-        for (; k < all.size() && (x == kNumXcd - 1 || done + 0.5 * (probs[all[k].prob].zc + 10) < upto); ++k) {
-            part.push_back(all[k]);
-            done += probs[all[k].prob].zc + 10;
-        }
-        std::stable_sort(part.begin(), part.end(),
-                         [&](const EnsItem &a, const EnsItem &b) { return probs[a.prob].zc > probs[b.prob].zc; });
-        using Load = std::pair<double, int>;   // (work so far, workgroup)
-        std::priority_queue<Load, std::vector<Load>, std::greater<Load>> least;
-        for (int b = x; b < blocks; b += kNumXcd) least.push({0.0, b});
-        for (const EnsItem &i : part) {
-            Load l = least.top();
-            least.pop();
-            list[l.second].push_back(i);
-            l.first += probs[i.prob].zc + 10;
-            most = std::max(most, l.first);
-            least.push(l);
-        }
-    }
-    items.clear();
-    first.assign(1, 0);
-    for (const auto &l : list) {
-        items.insert(items.end(), l.begin(), l.end());
-        first.push_back((int)items.size());
-    }
-    return most;
-}
-
 static int ens_layout(acx_ensemble *e)
 try {
     const EnsConfig &c = kConfigs[e->config];
-    const std::vector<EnsProblem> probs = ens_problems(e, c);
-    int rc = hip_check(hipMemcpy(e->d_probs, probs.data(), sizeof(EnsProblem) * e->nprob, hipMemcpyHostToDevice),
+    const EnsPlan plan = ens_plan(ens_problems(e, c), e->fit[c.by == 8 ? 0 : 1]);
+    int rc = hip_check(hipMemcpy(e->d_probs, plan.probs.data(), sizeof(EnsProblem) * e->nprob, hipMemcpyHostToDevice),
                        "ensemble table");
     for (int k = 0; k < 2 && !rc; ++k) {
-        std::vector<EnsItem> items;
-        std::vector<int> first;
-        ens_schedule(probs, e->blocks[c.by == 8 ? 0 : 1][k ? F32_LAST : F32_MID], items, first);
-        rc = hip_check(hipMemcpy(e->d_items[k], items.data(), sizeof(EnsItem) * items.size(), hipMemcpyHostToDevice),
+        const EnsSchedule &q = plan.schedule[k];
+        rc = hip_check(hipMemcpy(e->d_items[k], q.items.data(), sizeof(EnsItem) * q.items.size(), hipMemcpyHostToDevice),
                        "ensemble schedule");
         if (!rc)
-            rc = hip_check(hipMemcpy(e->d_first[k], first.data(), sizeof(int) * first.size(), hipMemcpyHostToDevice),
+            rc = hip_check(hipMemcpy(e->d_first[k], q.first.data(), sizeof(int) * q.first.size(), hipMemcpyHostToDevice),
                            "ensemble schedule");
+        e->grid[k] = q.blocks();
     }
     return rc;
 } catch (const std::exception &x) {
@@ -200,14 +124,12 @@ try {
     int best = 0;
     double best_t = -1.0;
     for (int c = 0; c < ENS_NCONFIG; ++c) {
-        std::vector<EnsItem> items;
-        std::vector<int> first;
         const bool r8 = kConfigs[c].by == 8;
         const std::vector<EnsProblem> probs = ens_problems(e, kConfigs[c]);
         int longest = 0;
         for (const EnsProblem &q : probs) longest = std::max(longest, q.zc);
-        const double t = (ens_schedule(probs, e->blocks[r8 ? 0 : 1][F32_LAST], items, first) + 0.75 * (longest + 10)) *
-                         (r8 ? 1.0 : 1.3);
+        const EnsSchedule last = ens_schedule(probs, e->fit[r8 ? 0 : 1][ens_schedule_of(F32_LAST)]);
+        const double t = (last.most + 0.75 * (longest + 10)) * (r8 ? 1.0 : 1.3);
         if (best_t < 0 || t < best_t) {
             best_t = t;
             best = c;
@@ -221,8 +143,9 @@ try {
 template <int BY, int STAGE>
 static int ens_launch(const acx_ensemble *e, const LinArgs &a, hipStream_t s)
 {
-    hipLaunchKernelGGL((k_ensemble<BY, STAGE>), dim3(e->blocks[BY == 8 ? 0 : 1][STAGE]), dim3(ENS_BX, BY), 0, s, e->d_probs,
-                       e->d_items[STAGE == F32_LAST], e->d_first[STAGE == F32_LAST], a);
+    constexpr int k = ens_schedule_of(STAGE);
+    hipLaunchKernelGGL((k_ensemble<BY, STAGE>), dim3(e->grid[k]), dim3(ENS_BX, BY), 0, s, e->d_probs, e->d_items[k],
+                       e->d_first[k], a);
     return hip_check(hipGetLastError(), "ensemble launch");
 }
 
@@ -310,14 +233,12 @@ int acx_ensemble_create(int nprob, const int32_t *n, double h, acx_ensemble **ou
             if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kernel, ENS_BX * by, 0) != hipSuccess || n < 1) n = 1;
             return n * device_cus();
         };
-        e->blocks[0][F32_FIRST] = fit(reinterpret_cast<const void *>(&k_ensemble<8, F32_FIRST>), 8);
-        e->blocks[0][F32_MID] = fit(reinterpret_cast<const void *>(&k_ensemble<8, F32_MID>), 8);
-        e->blocks[0][F32_LAST] = fit(reinterpret_cast<const void *>(&k_ensemble<8, F32_LAST>), 8);
-        e->blocks[1][F32_FIRST] = fit(reinterpret_cast<const void *>(&k_ensemble<12, F32_FIRST>), 12);
-        e->blocks[1][F32_MID] = fit(reinterpret_cast<const void *>(&k_ensemble<12, F32_MID>), 12);
-        e->blocks[1][F32_LAST] = fit(reinterpret_cast<const void *>(&k_ensemble<12, F32_LAST>), 12);
+        e->fit[0][0] = fit(reinterpret_cast<const void *>(&k_ensemble<8, F32_MID>), 8);
+        e->fit[0][1] = fit(reinterpret_cast<const void *>(&k_ensemble<8, F32_LAST>), 8);
+        e->fit[1][0] = fit(reinterpret_cast<const void *>(&k_ensemble<12, F32_MID>), 12);
+        e->fit[1][1] = fit(reinterpret_cast<const void *>(&k_ensemble<12, F32_LAST>), 12);
         for (const EnsConfig &c : kConfigs) e->max_items = std::max(e->max_items, ens_count(ens_problems(e, c)));
-        for (const auto &b : e->blocks) e->max_blocks = std::max(e->max_blocks, (size_t)*std::max_element(b, b + 3));
+        for (const auto &b : e->fit) e->max_blocks = std::max(e->max_blocks, (size_t)*std::max_element(b, b + 2));
         for (int k = 0; k < 2 && !rc; ++k) {
             rc = hip_check(hipMalloc(&e->d_items[k], sizeof(EnsItem) * e->max_items), "ensemble alloc");
             rc = rc ? rc : hip_check(hipMalloc(&e->d_first[k], sizeof(int) * (e->max_blocks + 1)), "ensemble alloc");

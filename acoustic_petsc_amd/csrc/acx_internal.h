@@ -5,12 +5,9 @@
 #include <stddef.h>
 #include <stdint.h>
 #include "../../include/acx.h"
+#include "acx_plan.h"
 
 namespace acx {
-
-// Stages of a compensated FP32 step by what they read: no increment yet, the
-// increment, the increment and the state the step ends in.
-enum { F32_FIRST = 0, F32_MID = 1, F32_LAST = 2 };
 
 // Arguments of the fused linear stage kernel (acx_linear.hip).
 struct LinArgs {

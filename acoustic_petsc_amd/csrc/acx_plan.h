@@ -5,6 +5,12 @@
 
 namespace acx {
 
+constexpr int kNumXcd = 8;   // XCDs of the device, each with an L2 of its own
+
+// Stages of a compensated FP32 step by what they read: no increment yet, the
+// increment, the increment and the state the step ends in.
+enum { F32_FIRST = 0, F32_MID = 1, F32_LAST = 2 };
+
 // Index i of a periodic axis of n cells, from anywhere outside it.
 constexpr int wrap(int i, int n)
 {

@@ -51,3 +51,42 @@ int main()
                         }}
 }}
 """)
+
+
+@pytest.mark.parametrize("fit", [(512, 256), (256, 512), (3, 7), (1, 8), (77, 304)])
+def test_ensemble_lists_hold_every_item_once(fit, run_host):
+    """Launched with the workgroups its schedule is made for, each stage runs
+    every (problem, tile, z-chunk) exactly once, and the items cover the grids."""
+    run_host(f"""
+#include <set>
+#include "acx_ensemble_plan.h"
+int main()
+{{
+    const std::vector<int> dims = {{64, 96, 128, 4, 4, 4, 65, 9, 31, 160, 64, 5, 7, 130, 257}};
+    const std::vector<size_t> off = {{0, 1, 2, 3, 4}};
+    const int fit[2] = {{{fit[0]}, {fit[1]}}};
+    for (int by : {{8, 12}})
+        for (int zc : {{16, 32, 64, 128}}) {{
+            const EnsPlan plan = ens_plan(ens_problems(dims, off, {{by, zc}}), fit);
+            long cells = 0;
+            for (const EnsProblem &q : plan.probs) {{
+                CHECK(q.ntx * ENS_BX >= q.n[0] && q.nty * by >= q.n[1] && q.ntz * q.zc >= q.n[2], "tiles short of the grid");
+                CHECK((q.ntz - 1) * q.zc < q.n[2] && q.zc <= zc, "an empty or overlong chunk");
+                cells += (long)q.ntx * q.nty * q.ntz;
+            }}
+            for (int stage : {{F32_FIRST, F32_MID, F32_LAST}}) {{
+                const EnsSchedule &s = plan.schedule[ens_schedule_of(stage)];
+                CHECK(s.blocks() == fit[ens_schedule_of(stage)], "stage %d: lists for %d workgroups", stage, s.blocks());
+                std::set<std::pair<int, int>> seen;
+                for (int b = 0; b < s.blocks(); ++b)
+                    for (int k = s.first[b]; k < s.first[b + 1]; ++k) {{
+                        const EnsItem i = s.items[k];
+                        const EnsProblem &q = plan.probs[i.prob];
+                        CHECK(i.tile >= 0 && i.tile < q.ntx * q.nty * q.ntz, "tile %d of problem %d", i.tile, i.prob);
+                        CHECK(seen.insert({{i.prob, i.tile}}).second, "item twice");
+                    }}
+                CHECK((long)seen.size() == cells && s.items.size() == seen.size(), "stage %d: %zu of %ld items", stage, seen.size(), cells);
+            }}
+        }}
+}}
+""")
