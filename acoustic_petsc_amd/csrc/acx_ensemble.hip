@@ -60,21 +60,27 @@ k_ensemble(const EnsProblem *__restrict__ probs, const EnsItem *__restrict__ ite
 
 using namespace acx;
 
+// A configuration's problems and its two schedules (stages 1-3, last stage).
+struct EnsTables {
+    size_t at;                         // offset in d_tables
+    const EnsProblem *probs;           // device pointers, null until written
+    const EnsItem *items[2];
+    const int *first[2];
+    int grid[2];                       // workgroups each schedule is made for
+};
+
 struct acx_ensemble {
     int nprob;
     double h;
     std::vector<size_t> off;            // first cell of every problem
     std::vector<int> dims;
     size_t ncell;
-    EnsProblem *d_probs;
-    EnsItem *d_items[2];               // schedules of the current configuration: stages 1-3, last stage
-    int *d_first[2];
-    size_t max_items, max_blocks;      // their sizes
+    unsigned char *d_tables;           // problems and schedules of every configuration, each in a place of its own
+    EnsTables tables[ENS_NCONFIG];     // written on a configuration's first use, never again: launches in flight read them
     float *hi[2], *lo[2], *d0, *d1;
     int cur;                           // index of the current (hi, lo)
     int config;
-    int grid[2];                       // workgroups each schedule is made for
-    int fit[2][2];                     // the same that fit at once, per rows-per-tile variant (8, 12)
+    int fit[2][2];                     // workgroups that fit at once per rows-per-tile variant (8, 12) and schedule
     hipGraphExec_t graph;
     double graph_dt;
     int graph_config, graph_cur;
@@ -93,22 +99,41 @@ static size_t ens_count(const std::vector<EnsProblem> &probs)
     return n;
 }
 
-static int ens_layout(acx_ensemble *e)
+// Bytes of a configuration's tables.
+static size_t ens_table_bytes(const acx_ensemble *e, const EnsConfig &c)
+{
+    const int(&fit)[2] = e->fit[c.by == 8 ? 0 : 1];
+    const size_t items = ens_count(ens_problems(e, c));
+    return sizeof(EnsProblem) * e->nprob + 2 * sizeof(EnsItem) * items + sizeof(int) * (fit[0] + 1 + fit[1] + 1);
+}
+
+// Makes and uploads a configuration's tables unless they are there.
+static int ens_layout(acx_ensemble *e, int config)
 try {
-    const EnsConfig &c = kConfigs[e->config];
+    EnsTables &t = e->tables[config];
+    if (t.probs) return ACX_OK;
+    const EnsConfig &c = kConfigs[config];
     const EnsPlan plan = ens_plan(ens_problems(e, c), e->fit[c.by == 8 ? 0 : 1]);
-    int rc = hip_check(hipMemcpy(e->d_probs, plan.probs.data(), sizeof(EnsProblem) * e->nprob, hipMemcpyHostToDevice),
-                       "ensemble table");
-    for (int k = 0; k < 2 && !rc; ++k) {
-        const EnsSchedule &q = plan.schedule[k];
-        rc = hip_check(hipMemcpy(e->d_items[k], q.items.data(), sizeof(EnsItem) * q.items.size(), hipMemcpyHostToDevice),
-                       "ensemble schedule");
-        if (!rc)
-            rc = hip_check(hipMemcpy(e->d_first[k], q.first.data(), sizeof(int) * q.first.size(), hipMemcpyHostToDevice),
-                           "ensemble schedule");
-        e->grid[k] = q.blocks();
+    std::vector<unsigned char> h;
+    auto put = [&](const auto &v) {   // its offset
+        const size_t o = h.size();
+        const unsigned char *b = reinterpret_cast<const unsigned char *>(v.data());
+        h.insert(h.end(), b, b + v.size() * sizeof(v[0]));
+        return o;
+    };
+    const EnsSchedule(&q)[2] = plan.schedule;
+    const size_t at_probs = put(plan.probs);
+    const size_t at_items[2] = {put(q[0].items), put(q[1].items)};
+    const size_t at_first[2] = {put(q[0].first), put(q[1].first)};
+    unsigned char *d = e->d_tables + t.at;
+    if (int rc = hip_check(hipMemcpy(d, h.data(), h.size(), hipMemcpyHostToDevice), "ensemble tables")) return rc;
+    for (int k = 0; k < 2; ++k) {
+        t.items[k] = reinterpret_cast<const EnsItem *>(d + at_items[k]);
+        t.first[k] = reinterpret_cast<const int *>(d + at_first[k]);
+        t.grid[k] = q[k].blocks();
     }
-    return rc;
+    t.probs = reinterpret_cast<const EnsProblem *>(d + at_probs);
+    return ACX_OK;
 } catch (const std::exception &x) {
     return set_error(ACX_EHIP, "ensemble schedule: %s", x.what());
 }
@@ -144,8 +169,8 @@ template <int BY, int STAGE>
 static int ens_launch(const acx_ensemble *e, const LinArgs &a, hipStream_t s)
 {
     constexpr int k = ens_schedule_of(STAGE);
-    hipLaunchKernelGGL((k_ensemble<BY, STAGE>), dim3(e->grid[k]), dim3(ENS_BX, BY), 0, s, e->d_probs, e->d_items[k],
-                       e->d_first[k], a);
+    const EnsTables &t = e->tables[e->config];
+    hipLaunchKernelGGL((k_ensemble<BY, STAGE>), dim3(t.grid[k]), dim3(ENS_BX, BY), 0, s, t.probs, t.items[k], t.first[k], a);
     return hip_check(hipGetLastError(), "ensemble launch");
 }
 
@@ -216,7 +241,6 @@ int acx_ensemble_create(int nprob, const int32_t *n, double h, acx_ensemble **ou
     e->graph_stream = nullptr;
     const size_t bytes = e->ncell * 4 * sizeof(float);
     int rc = ACX_OK;
-    rc = rc ? rc : hip_check(hipMalloc(&e->d_probs, sizeof(EnsProblem) * nprob), "ensemble alloc");
     for (int k = 0; k < 2 && !rc; ++k) {
         rc = hip_check(hipMalloc(&e->hi[k], bytes), "ensemble alloc");
         rc = rc ? rc : hip_check(hipMalloc(&e->lo[k], bytes), "ensemble alloc");
@@ -237,14 +261,14 @@ int acx_ensemble_create(int nprob, const int32_t *n, double h, acx_ensemble **ou
         e->fit[0][1] = fit(reinterpret_cast<const void *>(&k_ensemble<8, F32_LAST>), 8);
         e->fit[1][0] = fit(reinterpret_cast<const void *>(&k_ensemble<12, F32_MID>), 12);
         e->fit[1][1] = fit(reinterpret_cast<const void *>(&k_ensemble<12, F32_LAST>), 12);
-        for (const EnsConfig &c : kConfigs) e->max_items = std::max(e->max_items, ens_count(ens_problems(e, c)));
-        for (const auto &b : e->fit) e->max_blocks = std::max(e->max_blocks, (size_t)*std::max_element(b, b + 2));
-        for (int k = 0; k < 2 && !rc; ++k) {
-            rc = hip_check(hipMalloc(&e->d_items[k], sizeof(EnsItem) * e->max_items), "ensemble alloc");
-            rc = rc ? rc : hip_check(hipMalloc(&e->d_first[k], sizeof(int) * (e->max_blocks + 1)), "ensemble alloc");
+        size_t at = 0;
+        for (int c = 0; c < ENS_NCONFIG; ++c) {
+            e->tables[c].at = at;
+            at += (ens_table_bytes(e, kConfigs[c]) + 255) / 256 * 256;
         }
+        rc = hip_check(hipMalloc(&e->d_tables, at), "ensemble alloc");
         e->config = ens_default_config(e);
-        rc = rc ? rc : ens_layout(e);
+        rc = rc ? rc : ens_layout(e, e->config);
     }
     if (rc) {
         acx_ensemble_destroy(e);
@@ -258,11 +282,7 @@ int acx_ensemble_destroy(acx_ensemble *e)
 {
     if (!e) return ACX_OK;
     if (e->graph) hipGraphExecDestroy(e->graph);
-    hipFree(e->d_probs);
-    for (int k = 0; k < 2; ++k) {
-        hipFree(e->d_items[k]);
-        hipFree(e->d_first[k]);
-    }
+    hipFree(e->d_tables);
     for (int k = 0; k < 2; ++k) {
         hipFree(e->hi[k]);
         hipFree(e->lo[k]);
@@ -310,8 +330,9 @@ int acx_ensemble_copy_out(const acx_ensemble *e, float *hi, float *lo, void *str
 int acx_ensemble_set_config(acx_ensemble *e, int config)
 {
     if (!e || config < 0 || config >= ENS_NCONFIG) return set_error(ACX_EINVAL, "ensemble: config out of range");
-    e->config = config;
-    return ens_layout(e);
+    const int rc = ens_layout(e, config);
+    if (!rc) e->config = config;
+    return rc;
 }
 
 int acx_ensemble_get_config(const acx_ensemble *e) { return e ? e->config : -1; }
