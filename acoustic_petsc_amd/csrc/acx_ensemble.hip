@@ -11,6 +11,7 @@
 #include <exception>
 #include <stdlib.h>
 #include <string.h>
+#include <type_traits>
 #include <vector>
 #include "acx_ensemble_plan.h"
 #include "acx_linear_core.h"
@@ -24,7 +25,8 @@ constexpr int ENS_NCONFIG = 8;
 static const EnsConfig kConfigs[ENS_NCONFIG] = {{8, 16}, {8, 32}, {8, 64}, {12, 16}, {12, 32}, {12, 64},
                                                 {8, 128}, {12, 128}};
 
-template <int BY, int STAGE>
+// WIDE: the march with 64-bit offsets inside a plane (ens_wide).
+template <int BY, int STAGE, bool WIDE>
 __global__ void __launch_bounds__(ENS_BX *BY) __attribute__((amdgpu_waves_per_eu(STAGE == F32_LAST ? BY / 4 : 4)))
 k_ensemble(const EnsProblem *__restrict__ probs, const EnsItem *__restrict__ items, const int *__restrict__ first,
            LinArgs base)
@@ -51,7 +53,7 @@ k_ensemble(const EnsProblem *__restrict__ probs, const EnsItem *__restrict__ ite
         const int x0 = (local % pr.ntx) * ENS_BX, y0 = ((local / pr.ntx) % pr.nty) * BY;
         a.zc = pr.zc;
         const int zb = (local / (pr.ntx * pr.nty)) * a.zc;
-        linear_tile32<ACX_ACOUSTIC4, BY, STAGE, false, true>(a, x0, y0, zb, lds);
+        linear_tile32<ACX_ACOUSTIC4, BY, STAGE, WIDE, true>(a, x0, y0, zb, lds);
         __syncthreads();   // LDS is reused by the next item
     }
 }
@@ -74,6 +76,7 @@ struct acx_ensemble {
     double h;
     std::vector<size_t> off;            // first cell of every problem
     std::vector<int> dims;
+    bool wide;                         // a problem's planes need the march with 64-bit offsets
     size_t ncell;
     unsigned char *d_tables;           // problems and schedules of every configuration, each in a place of its own
     EnsTables tables[ENS_NCONFIG];     // written on a configuration's first use, never again: launches in flight read them
@@ -170,7 +173,12 @@ static int ens_launch(const acx_ensemble *e, const LinArgs &a, hipStream_t s)
 {
     constexpr int k = ens_schedule_of(STAGE);
     const EnsTables &t = e->tables[e->config];
-    hipLaunchKernelGGL((k_ensemble<BY, STAGE>), dim3(t.grid[k]), dim3(ENS_BX, BY), 0, s, t.probs, t.items[k], t.first[k], a);
+    if (e->wide)
+        hipLaunchKernelGGL((k_ensemble<BY, STAGE, true>), dim3(t.grid[k]), dim3(ENS_BX, BY), 0, s, t.probs, t.items[k],
+                           t.first[k], a);
+    else
+        hipLaunchKernelGGL((k_ensemble<BY, STAGE, false>), dim3(t.grid[k]), dim3(ENS_BX, BY), 0, s, t.probs, t.items[k],
+                           t.first[k], a);
     return hip_check(hipGetLastError(), "ensemble launch");
 }
 
@@ -231,6 +239,7 @@ int acx_ensemble_create(int nprob, const int32_t *n, double h, acx_ensemble **ou
     e->nprob = nprob;
     e->h = h;
     e->dims.assign(n, n + 3 * nprob);
+    e->wide = ens_wide(e->dims);
     e->ncell = 0;
     for (int p = 0; p < nprob; ++p) {
         e->off.push_back(e->ncell);
@@ -257,10 +266,15 @@ int acx_ensemble_create(int nprob, const int32_t *n, double h, acx_ensemble **ou
             if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kernel, ENS_BX * by, 0) != hipSuccess || n < 1) n = 1;
             return n * device_cus();
         };
-        e->fit[0][0] = fit(reinterpret_cast<const void *>(&k_ensemble<8, F32_MID>), 8);
-        e->fit[0][1] = fit(reinterpret_cast<const void *>(&k_ensemble<8, F32_LAST>), 8);
-        e->fit[1][0] = fit(reinterpret_cast<const void *>(&k_ensemble<12, F32_MID>), 12);
-        e->fit[1][1] = fit(reinterpret_cast<const void *>(&k_ensemble<12, F32_LAST>), 12);
+        auto fits = [&](auto wide) {
+            constexpr bool W = decltype(wide)::value;
+            e->fit[0][0] = fit(reinterpret_cast<const void *>(&k_ensemble<8, F32_MID, W>), 8);
+            e->fit[0][1] = fit(reinterpret_cast<const void *>(&k_ensemble<8, F32_LAST, W>), 8);
+            e->fit[1][0] = fit(reinterpret_cast<const void *>(&k_ensemble<12, F32_MID, W>), 12);
+            e->fit[1][1] = fit(reinterpret_cast<const void *>(&k_ensemble<12, F32_LAST, W>), 12);
+        };
+        if (e->wide) fits(std::true_type{});
+        else fits(std::false_type{});
         size_t at = 0;
         for (int c = 0; c < ENS_NCONFIG; ++c) {
             e->tables[c].at = at;

@@ -51,6 +51,15 @@ inline std::vector<EnsProblem> ens_problems(const std::vector<int> &dims, const 
     return probs;
 }
 
+// Whether a problem's planes are beyond the 32-bit offsets of the all-periodic
+// march (16 bytes a cell); the whole ensemble then takes the general one.
+inline bool ens_wide(const std::vector<int> &dims)
+{
+    for (size_t p = 0; p + 2 < dims.size(); p += 3)
+        if (plane_beyond_32_bits(dims[p], dims[p + 1], 16)) return true;
+    return false;
+}
+
 // Lists of the items per workgroup: workgroup b runs items[first[b]] ..
 // items[first[b + 1] - 1], so the launch has blocks() workgroups, neither fewer
 // (items would not run) nor more (there is no list for them).

@@ -165,9 +165,8 @@ static int launch_linear32_w(const LinArgs &a, hipStream_t s)
 template <int SYS>
 static int launch_linear32(const LinArgs &a, hipStream_t s)
 {
-    // the all-periodic instantiation keeps offsets inside a plane in 32 bits
     const bool general = a.bc[0] != ACX_PERIODIC || a.bc[1] != ACX_PERIODIC || a.bc[2] != ACX_PERIODIC ||
-                         (size_t)a.nx * a.ny * (SYS == ACX_ACOUSTIC4 ? 16 : 8) > 0xffffffffu;
+                         plane_beyond_32_bits(a.nx, a.ny, SYS == ACX_ACOUSTIC4 ? 16 : 8);
     if (a.final_stage)
         return general ? launch_linear32_w<SYS, F32_LAST, true>(a, s) : launch_linear32_w<SYS, F32_LAST, false>(a, s);
     if (a.d)

@@ -27,4 +27,11 @@ constexpr uint32_t region_cell(int x0, int y0, int halo, int r, int c, int nx, i
     return (uint32_t)wrap(y0 - halo + r, ny) * (uint32_t)nx + (uint32_t)wrap(x0 - halo + c, nx);
 }
 
+// Whether a plane's byte offsets (cells of cell_bytes) need more than the 32
+// bits the all-periodic marches keep them in.
+constexpr bool plane_beyond_32_bits(int nx, int ny, int cell_bytes)
+{
+    return (uint64_t)nx * (uint64_t)ny * (uint64_t)cell_bytes > 0xffffffffu;
+}
+
 } // namespace acx

@@ -146,3 +146,38 @@ def test_configuration_changes_while_steps_are_in_flight(acx, torch_gpu):
         assert np.array_equal(hi[a:b].cpu().numpy(), ref[p][0]), p
         assert np.array_equal(lo[a:b].cpu().numpy(), ref[p][1]), p
     e.close()
+
+
+def test_planes_beyond_32_bit_offsets(acx, torch_gpu):
+    """A problem of 16400 x 16400 x 4 cells (planes of 4.3 GB) that repeats a
+    100 x 100 x 4 one: the same cells, the same bits, also where a byte offset
+    inside a plane passes 2^32 (2^28 cells are 16368 rows and 256 columns, no
+    multiple of the period)."""
+    torch = torch_gpu
+    import ctypes
+    from acoustic_petsc_amd import ensemble as ens
+    m, k = 100, 164
+    N = m * k
+    free, _ = torch.cuda.mem_get_info()
+    if free < 150e9:
+        pytest.skip("needs 150 GB of device memory")
+    h = 1.0 / 32
+    dt = 0.4 * h / 3
+    g = acx.Grid(n=(m, m, 4), h=h)
+    U = torch.from_numpy(np.random.default_rng(9).standard_normal(g.shape())).cuda()
+    s = acx.CompensatedState(g, U)
+    hi, lo = (t.view(4, 1, m, 1, m, 4).expand(4, k, m, k, m, 4).reshape(-1) for t in (s.hi, s.lo))
+    print("[case] ensemble plane beyond 2^32 bytes", flush=True)
+    e = ens.Ensemble([(N, N, 4)], h)
+    ptr = lambda t: ctypes.c_void_p(t.data_ptr())  # noqa: E731
+    L = ens._bind()
+    acx._check(L.acx_ensemble_copy_in(e._h, ptr(hi), ptr(lo), acx._stream()))
+    e.step(dt)
+    acx._check(L.acx_ensemble_copy_out(e._h, ptr(hi), ptr(lo), acx._stream()))
+    s.step(dt)
+    for got, want in ((hi, s.hi), (lo, s.lo)):
+        got = got.view(4, k, m, k, m, 4)
+        for j in range(k):
+            same = torch.equal(got[:, j], want.view(4, m, 1, m, 4).expand(4, m, k, m, 4))
+            assert same, f"rows {m * j} .. {m * j + m - 1}"
+    e.close()

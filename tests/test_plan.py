@@ -90,3 +90,17 @@ int main()
         }}
 }}
 """)
+
+
+def test_plane_offsets_of_32_bits(run_host):
+    """The largest byte offset inside a plane fits 32 bits where the rule says so."""
+    run_host("""
+#include "acx_ensemble_plan.h"
+int main()
+{
+    CHECK(!plane_beyond_32_bits(16384, 16383, 16), "a plane below 2^32 bytes");
+    CHECK(plane_beyond_32_bits(16384, 16384, 16) && plane_beyond_32_bits(16400, 16400, 16), "2^32 bytes and more");
+    CHECK(plane_beyond_32_bits(2147483647, 4, 8) && !plane_beyond_32_bits(1 << 27, 3, 8), "long rows");
+    CHECK(ens_wide({64, 64, 64, 16384, 16384, 4}) && !ens_wide({64, 64, 64, 16384, 16383, 4}), "any problem of a batch");
+}
+""")
