@@ -255,13 +255,27 @@ __device__ __forceinline__ T cweno_axes(const T (&s)[33], const CwArgs &p, Axis3
 //   2 c1  = S - n1 a - n2 c + n4 (g3s - 11/60)/g4 T
 //   2 c2  = B + n1 a - n2 c - n4 g3s/g4 F
 //   12 c3 = n4/g4 T
+// Beside a jump (p1, p2 across it) the smooth sided stencil takes all the
+// weight, n2 -> 1, and B - n2 c would leave the rounding of B, the jump's size,
+// in a result of the size of C, the background's.  Where the sided stencils leave
+// the others less than 1/1024, the sums of that axis start from the dominating
+// stencil instead, with w = 1 - n2 summed from all other weights:
+//   2 c2 = C + w c + n1 a - ...,  2 c1 = 2 e2 + C + w c - n1 a + ...
+// (on the other side A - w a - n2 c and 2 e3 - A + w a - n2 c).  Above 1/1024 the
+// indicators are within a factor of 23 and the jump within 5 of the background.
+// The branch costs 2 % of a 256^3 ACOUSTIC4 step (4.36 -> 4.45 ms), where one
+// wavefront in a hundred takes it, and 3 to 13 % of a 70 x 45 x 61 WAVE2 right-hand
+// side (12.3 -> 12.6 .. 13.8 us), whose odd walls are jumps in a third of the
+// wavefronts; these sums without a branch would add 7 % of the instructions
+// everywhere.
 // In FP64 the eight reciprocals 1/IS come from two, each of a product of four IS
 // (in range whenever IS^4 is), each refined to full precision.  In FP32, where
 // (IS + eps)^4 ~ 1e-48 underflows, the weights are gamma (IS_min / IS)^4.
 template <int SYS, typename T, typename Get>
 __device__ __forceinline__ void cweno_weights4(Get get, const CwArgs &p, const T (&S)[3], const T (&B)[3],
                                                const T (&a)[3], const T (&c)[3], const T (&e2)[3], const T (&e3)[3],
-                                               const T (&A)[3], const T (&Cc)[3], T (&n)[6], T &is, T &ke, T &ko)
+                                               const T (&A)[3], const T (&Cc)[3], T (&n)[6], T &is, T &ke, T &ko,
+                                               T &rest)
 {
     const T k13 = T(13.0 / 3.0), k7 = T(7.0 / 6.0), eps = T(4.0e-12);
     T C[3], P[3], M[3], is4;
@@ -340,11 +354,13 @@ __device__ __forceinline__ void cweno_weights4(Get get, const CwArgs &p, const T
 #pragma unroll
     for (int k = 0; k < 6; ++k) n[k] = pow4(n[k]);
     const T sided = ((n[0] + n[1]) + (n[2] + n[3])) + (n[4] + n[5]);
-    const T sum = fma(g3s, sided, fma(T(p.g3c), pow4(r0), w4));
+    const T central = fma(T(p.g3c), pow4(r0), w4);
+    const T sum = fma(g3s, sided, central);
     T it;
     if constexpr (sizeof(T) == 8) it = rcp64_full(sum);
     else it = __builtin_amdgcn_rcpf(sum);
     is = g3s * it;
+    rest = central * it;
     w4 *= it;
     ke = T(p.k2) * w4;
     ko = T(SYS == ACX_ACOUSTIC4 ? p.k1a : p.k1w) * w4;
@@ -369,14 +385,10 @@ __device__ __forceinline__ void cweno_faces(Get get, const CwArgs &p, bool full,
         a[d] = A[d] - B[d];
         c[d] = B[d] - Cc[d];
     }
-    T is = T(0), ke = T(0), ko = T(-1.0 / 6.0);
-    if (full) cweno_weights4<SYS, T>(get, p, S, B, a, c, e2, e3, A, Cc, n, is, ke, ko);
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-        const T h1 = n[2 * d] * a[d], h2 = n[2 * d + 1] * c[d];
-        const T G = a[d] + c[d], F = a[d] - c[d];
-        const T E = fma(-ke, F, fma(is, h1 - h2, B[d]));
-        const T O = fma(ko, G, fma(-is, h1 + h2, S[d]));
+    T is = T(0), ke = T(0), ko = T(-1.0 / 6.0), rest = T(1);
+    if (full) cweno_weights4<SYS, T>(get, p, S, B, a, c, e2, e3, A, Cc, n, is, ke, ko, rest);
+    // faces of axis d from E = 2 c2 (less the share of c3) and O = 2 c1 (plus it)
+    auto faces = [&](int d, T E, T O) {
         if constexpr (SYS == ACX_ACOUSTIC4) {
             const T even = fma(T(1.0 / 12.0), E, u0);
             fm[d] = fma(T(-0.25), O, even);
@@ -384,6 +396,30 @@ __device__ __forceinline__ void cweno_faces(Get get, const CwArgs &p, bool full,
         } else {
             fm[d] = T(0.5) * (O - E);
             fp[d] = T(0.5) * (O + E);
+        }
+    };
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        const T h1 = n[2 * d] * a[d], h2 = n[2 * d + 1] * c[d];
+        const T G = a[d] + c[d], F = a[d] - c[d];
+        faces(d, fma(-ke, F, fma(is, h1 - h2, B[d])), fma(ko, G, fma(-is, h1 + h2, S[d])));
+    }
+    if (rest < T(1.0 / 1024.0)) {
+        asm volatile("" ::: "memory");   // the axis values are read again
+        const T half = T(0.5) * (((n[0] + n[1]) + (n[2] + n[3])) + (n[4] + n[5]));
+#pragma unroll
+        for (int k = 0; k < 6; ++k) {
+            if (n[k] > half) {
+                const int d = k / 2, m = k % 2;   // m = 0: cells 0, +1, +2 of the axis; 1: 0, -1, -2
+                const T v1 = get(m ? 2 + 4 * d : 3 + 4 * d), v2 = get(m ? 1 + 4 * d : 4 + 4 * d);
+                const T t = v1 - u0, X = (v2 - v1) - t, Y = fma(T(2), t, -X);
+                T others = T(0);
+#pragma unroll
+                for (int q = 0; q < 6; ++q) others += q == k ? T(0) : n[q];
+                const T g = fma(is, others, rest) * (m ? c[d] : a[d]), h = (is * n[k ^ 1]) * (m ? a[d] : c[d]);
+                const T G = a[d] + c[d], F = a[d] - c[d];
+                faces(d, fma(-ke, F, m ? X + (h + g) : X - (h + g)), fma(ko, G, (m ? -Y : Y) + (g - h)));
+            }
         }
     }
 }
