@@ -238,18 +238,17 @@ __device__ __forceinline__ T cweno_axes(const T (&s)[33], const CwArgs &p, Axis3
 // Per axis, from the first differences e1 .. e4 of m2, m1, u0, p1, p2:
 //   A, B, C = e4-e3, e3-e2, e2-e1 (second), a, c = A-B, B-C (third),
 //   S = e2+e3, T = a+c, F = a-c (fourth)
-// and the indicators are formed times 4 (with 4 eps; the weights are ratios):
-//   central       4(cx^2 + 13/3 uxx^2)     = S^2 + 13/3 B^2
-//   one-sided +   4(dx1^2 + 13/3 dxx1^2)   = (2 e3 - A)^2 + 13/3 A^2
-//   one-sided -                              (2 e2 + C)^2 + 13/3 C^2
-//   4th order     4(ux^2 + 13/3 uxx^2 + ux uxxx/5 + 39.06 uxxx^2)
-//                                          = S^2 + 13/3 B^2 + T (1.1125 T - S/3)
-// For a pair of axes with the diagonals pp pm mp mm and the central
-// differences Sa, Sb: al, be = (pp-pm) - Sb, (mp-mm) - Sb and
-// ph, ps = (pp-mp) - Sa, (pm-mm) - Sa are twice the mixed derivatives of the
-// four sided stencils; M = (al-be)^2 = (ph-ps)^2 is 16 u_ab^2, and the mixed
-// third derivatives are (al+be)/4, (ph+ps)/4, whose squares follow from the
-// others: (al+be)^2 = 2(al^2+be^2) - M.
+// and with Sh = S/2 (the central first derivative) the indicators are
+//   central       cx^2 + 13/3 uxx^2        = Sh^2 + 13/12 B^2
+//   one-sided +   dx1^2 + 13/3 dxx1^2      = (e3 - A/2)^2 + 13/12 A^2
+//   one-sided -                              (e2 + C/2)^2 + 13/12 C^2
+//   4th order     ux^2 + 13/3 uxx^2 + ux uxxx/5 + 39.06 uxxx^2
+//                                          = Sh^2 + 13/12 B^2 + T (0.278125 T - Sh/6)
+// For a pair of axes with the diagonals pp pm mp mm: al, be = (pp-pm)/2 - Shb,
+// (mp-mm)/2 - Shb and ph, ps = (pp-mp)/2 - Sha, (pm-mm)/2 - Sha are the mixed
+// derivatives of the four sided stencils; M = (al-be)^2 = (ph-ps)^2 is 4 u_ab^2,
+// and the mixed third derivatives are (al+be)/2, (ph+ps)/2, whose squares follow
+// from the others: (al+be)^2 = 2(al^2+be^2) - M.
 // With normalised weights n4 (R4), n1, n2 (sided +, -) along an axis, and
 // gamma_R4 + sum gamma_R3 = 1, the combination of reconstruction.c:223-257 is
 //   2 c1  = S - n1 a - n2 c + n4 (g3s - 11/60)/g4 T
@@ -277,28 +276,29 @@ __device__ __forceinline__ void cweno_weights4(Get get, const CwArgs &p, const T
                                                const T (&A)[3], const T (&Cc)[3], T (&n)[6], T &is, T &ke, T &ko,
                                                T &rest)
 {
-    const T k13 = T(13.0 / 3.0), k7 = T(7.0 / 6.0), eps = T(4.0e-12);
-    T C[3], P[3], M[3], is4;
+    const T k13 = T(13.0 / 12.0), k7 = T(7.0 / 6.0), eps = T(1.0e-12);
+    T C[3], P[3], M[3], Sh[3], is4;
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
         const T G = a[d] + c[d];
-        const T D1 = fma(T(2), e3[d], -A[d]), D2 = fma(T(2), e2[d], Cc[d]);
-        C[d] = fma(S[d], S[d], fma(k13 * B[d], B[d], T(0.5) * eps));   // a sum of two carries eps
+        const T D1 = fma(T(-0.5), A[d], e3[d]), D2 = fma(T(0.5), Cc[d], e2[d]);
+        Sh[d] = T(0.5) * S[d];
+        C[d] = fma(Sh[d], Sh[d], fma(k13 * B[d], B[d], T(0.5) * eps));   // a sum of two carries eps
         P[d] = fma(D1, D1, (k13 * A[d]) * A[d]);
         M[d] = fma(D2, D2, (k13 * Cc[d]) * Cc[d]);
-        const T t = fma(S[d], T(-1.0 / 3.0), T(1.1125) * G);
+        const T t = fma(Sh[d], T(-1.0 / 6.0), T(0.278125) * G);
         is4 = d == 0 ? G * t : fma(G, t, is4);
     }
     const T Cyz = C[1] + C[2], Czx = C[2] + C[0], Cxy = C[0] + C[1];
     T t0 = Cyz + (C[0] - T(0.5) * eps);
     is4 += t0;
     asm volatile("" ::: "memory");
-    // twice the mixed derivatives of one pair of axes
+    // mixed derivatives of one pair of axes
     auto pair = [&](int q, T Sa, T Sb, T &al, T &be, T &ph, T &ps, T &m) {
         const T pp = get(q), pm = get(q + 1), mp = get(q + 2), mm = get(q + 3);
-        al = (pp - pm) - Sb;
-        be = (mp - mm) - Sb;
-        ph = (pp - mp) - Sa;
+        al = fma(T(0.5), pp - pm, -Sb);
+        be = fma(T(0.5), mp - mm, -Sb);
+        ph = fma(T(0.5), pp - mp, -Sa);
         const T x = al - be;
         ps = ph - x;
         m = x * x;
@@ -306,13 +306,13 @@ __device__ __forceinline__ void cweno_weights4(Get get, const CwArgs &p, const T
     T q[6], Mxy, Myz, Mzx;
     {
         T al, be, ph, ps;
-        pair(13, S[0], S[1], al, be, ph, ps, Mxy);   // (x, y): x+, x-, y+, y-
+        pair(13, Sh[0], Sh[1], al, be, ph, ps, Mxy);   // (x, y): x+, x-, y+, y-
         q[0] = al * al; q[1] = be * be; q[2] = ph * ph; q[3] = ps * ps;
         asm volatile("" ::: "memory");
-        pair(17, S[1], S[2], al, be, ph, ps, Myz);   // (y, z): y+, y-, z+, z-
+        pair(17, Sh[1], Sh[2], al, be, ph, ps, Myz);   // (y, z): y+, y-, z+, z-
         q[2] = fma(al, al, q[2]); q[3] = fma(be, be, q[3]); q[4] = ph * ph; q[5] = ps * ps;
         asm volatile("" ::: "memory");
-        pair(21, S[2], S[0], al, be, ph, ps, Mzx);   // (z, x): z+, z-, x+, x-
+        pair(21, Sh[2], Sh[0], al, be, ph, ps, Mzx);   // (z, x): z+, z-, x+, x-
         q[4] = fma(al, al, q[4]); q[5] = fma(be, be, q[5]); q[0] = fma(ph, ph, q[0]); q[1] = fma(ps, ps, q[1]);
     }
     asm volatile("" ::: "memory");
@@ -323,7 +323,7 @@ __device__ __forceinline__ void cweno_weights4(Get get, const CwArgs &p, const T
     is4 = fma(T(0.25 * 7.0 / 6.0 - 2.35), Ms, is4);
     {
         const T z = ((get(25) - get(26)) - (get(27) - get(29))) - ((get(28) - get(30)) - (get(31) - get(32)));
-        is4 = fma(T(61.0 / 768.0) * z, z, is4);
+        is4 = fma(T(61.0 / 3072.0) * z, z, is4);
     }
     const T t1 = fma(k7, fma(T(0.25), Myz, q[0]), P[0] + Cyz), t2 = fma(k7, fma(T(0.25), Myz, q[1]), M[0] + Cyz);
     const T t3 = fma(k7, fma(T(0.25), Mzx, q[2]), P[1] + Czx), t4 = fma(k7, fma(T(0.25), Mzx, q[3]), M[1] + Czx);

@@ -16,7 +16,7 @@ order of dt^2, is exact to far less than that.
 import numpy as np
 import pytest
 
-from test_gpu_parity import TOL, orc_grid
+from test_gpu_parity import TOL, make_field, orc_grid
 
 pytestmark = pytest.mark.gpu
 
@@ -69,3 +69,25 @@ def test_fp32_step_behind_a_jump(flagged, jump, background, axis, acx, torch_gpu
     err = np.abs(got - ref).max(0) / np.abs(ref).max(0)
     print(f"[case] largest error {err.max():.1e}", flush=True)
     assert (err <= 4e-6).all()
+
+
+def test_fp32_indicators_of_large_fields(acx, torch_gpu):
+    """A field of 2e18, whose indicators are below the largest FP32 number, takes
+    the step of the field of order one, times its size, to the rounding of the
+    faces (relative L2 <= 1e-7, as for the flagged slabs of the FP32 stages)."""
+    torch = torch_gpu
+    grid = acx.Grid(n=(32, 28, 24), h=1.0 / 32, gamma_hi=0.85, gamma_lo=0.85)
+    U = torch.from_numpy(make_field(acx, grid, 31, "step") / 1.75).cuda()
+    amp = 2e18
+    print(f"[case] FP32 nonlinear weights of fields of {amp:g}", flush=True)
+    acx.nonfinite_clear()
+    try:
+        got = []
+        for a in (1.0, amp):
+            s = acx.CompensatedState(grid, U * a)
+            s.step(acx.cfl_dt(grid, 0.4))
+            got.append(s.value64() / a)
+        assert float((got[1] - got[0]).norm() / got[0].norm()) <= 1e-7
+    finally:
+        torch.cuda.synchronize()
+        acx.nonfinite_clear()
