@@ -568,12 +568,9 @@ k_ctcs_dma(const double *__restrict__ Pold, const double *__restrict__ P, double
 // The same update for 3D grids that live in the caches between steps (even x
 // extent, 16-byte aligned arrays): one thread per pair of x-neighbours, 13
 // 16-byte loads all in flight at once instead of a march along z.
-// Arithmetic as in k_ctcs, term by term.  Up to about 2.5e6 cells (four arrays
-// of 80 MB together) the march is bound by the latency of its planes, not by
-// bytes.  us per update, march and this kernel: 48^3 6.8 / 3.3, 64^3 7.1 /
-// 3.9, 100^3 11.7 / 7.8, 128^3 15.6 / 14.4, 160^3 24.2 / 26.2, 256^3 108 / 132.
+// Arithmetic as in k_ctcs, term by term.  At the sizes of ctcs_route the march
+// is bound by the latency of its planes, not by bytes.
 constexpr int CD_THREADS = 256;
-constexpr size_t CD_CELLS = 2500000;
 
 template <int ST>
 __global__ void __launch_bounds__(CD_THREADS)
@@ -644,15 +641,13 @@ static int launch_ctcs(const acx_ctcs *c, const double *POLD, const double *P, d
                        double *rcv, hipStream_t s)
 {
     const double src = ctcs_source_step(*c, it);
-    const bool vol = c->n[0] >= 5 && c->n[1] >= 5 && c->n[2] >= 5;
-    const bool pairs = vol && c->n[0] % 2 == 0 && (size_t)c->n[0] * c->n[1] < 0xffffffffu &&
-                       ((((uintptr_t)POLD) | ((uintptr_t)P) | ((uintptr_t)C) | ((uintptr_t)PNEW)) & 15) == 0;
-    if (pairs && (size_t)c->n[0] * c->n[1] * c->n[2] <= CD_CELLS) {
+    const int route = ctcs_route(c->n[0], c->n[1], c->n[2], (uintptr_t)POLD | (uintptr_t)P | (uintptr_t)C, (uintptr_t)PNEW);
+    if (route == CTCS_PAIRS) {
         const size_t bpp = ((size_t)c->n[0] / 2 * c->n[1] + CD_THREADS - 1) / CD_THREADS;
         dim3 blk(CD_THREADS), grd((unsigned)(bpp * c->n[2]));
         if (c->stencil == 1) hipLaunchKernelGGL(k_ctcs_pair<1>, grd, blk, 0, s, POLD, P, PNEW, C, *c, src, (int)bpp, rcv);
         else hipLaunchKernelGGL(k_ctcs_pair<2>, grd, blk, 0, s, POLD, P, PNEW, C, *c, src, (int)bpp, rcv);
-    } else if (pairs) {
+    } else if (route == CTCS_DMA) {
         // 3D, LDS-DMA march: z-chunk from the round model, two blocks per CU
         // (measured at 256^3: 144 -> 152 G cell-updates/s, bit-identical to
         // the register-queue march below)
@@ -662,7 +657,7 @@ static int launch_ctcs(const acx_ctcs *c, const double *POLD, const double *P, d
         dim3 blk(CtDma::BX, CtDma::BY), grd((unsigned)nb);
         if (c->stencil == 1) hipLaunchKernelGGL(k_ctcs_dma<1>, grd, blk, 0, s, POLD, P, PNEW, C, *c, src, zc, rcv);
         else hipLaunchKernelGGL(k_ctcs_dma<2>, grd, blk, 0, s, POLD, P, PNEW, C, *c, src, zc, rcv);
-    } else if (vol) {
+    } else if (route == CTCS_MARCH) {
         // 3D: z-march; 32 planes per block, halved (down to 4) below 1024 blocks
         const size_t cols = (size_t)((c->n[0] + CT_BX - 1) / CT_BX) * ((c->n[1] + CT_BY - 1) / CT_BY);
         int zc = 32;

@@ -34,4 +34,22 @@ constexpr bool plane_beyond_32_bits(int nx, int ny, int cell_bytes)
     return (uint64_t)nx * (uint64_t)ny * (uint64_t)cell_bytes > 0xffffffffu;
 }
 
+// Kernel of one leapfrog update.  2D and 1D programs (an axis of one cell): a
+// thread per cell.  3D: the LDS-DMA march where x is even and the arrays it
+// copies (POLD, P, C: `in`, their addresses or'ed) are 16-byte aligned, else the
+// register march.  Up to CTCS_PAIR_CELLS and with PNEW (`out`) aligned too, a
+// thread per pair of cells with its 16-byte store (four arrays of 80 MB together,
+// which stay in the caches between steps).  us per update, DMA march and pairs:
+// 48^3 6.8 / 3.3, 64^3 7.1 / 3.9, 100^3 11.7 / 7.8, 128^3 15.6 / 14.4, 160^3 24.2 /
+// 26.2, 256^3 108 / 132.
+enum { CTCS_CELLS, CTCS_MARCH, CTCS_DMA, CTCS_PAIRS };
+constexpr uint64_t CTCS_PAIR_CELLS = 2500000;
+
+constexpr int ctcs_route(int nx, int ny, int nz, uintptr_t in, uintptr_t out)
+{
+    if (nx < 5 || ny < 5 || nz < 5) return CTCS_CELLS;
+    if (nx % 2 != 0 || in % 16 != 0 || (uint64_t)nx * (uint64_t)ny >= 0xffffffffu) return CTCS_MARCH;
+    return (uint64_t)nx * (uint64_t)ny * (uint64_t)nz <= CTCS_PAIR_CELLS && out % 16 == 0 ? CTCS_PAIRS : CTCS_DMA;
+}
+
 } // namespace acx

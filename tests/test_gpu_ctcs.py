@@ -177,3 +177,22 @@ def test_steps_equal_single_updates(n, acx, torch_gpu):
     L = acx.lib()
     assert L.acx_ctcs_steps_f64(ctypes.byref(p), ptr(P[0]), ptr(P[0]), ptr(P[2]), ptr(C), 0, 1, None, acx._stream()) == 1
     assert L.acx_ctcs_steps_f64(ctypes.byref(p), ptr(P[0]), ptr(P[1]), ptr(P[2]), ptr(C), 0, -1, None, acx._stream()) == 1
+
+
+@pytest.mark.parametrize("n", [(8, 7, 6), (100, 21, 13), (176, 120, 120)])
+@pytest.mark.parametrize("stencil", [1, 2])
+def test_only_the_result_off_alignment(n, stencil, acx, torch_gpu):
+    torch = torch_gpu
+    import ctypes
+    N = n[0] * n[1] * n[2]
+    gen = torch.Generator("cuda").manual_seed(13)
+    old, cur, C = (torch.randn(N, dtype=torch.float64, device="cuda", generator=gen) for _ in range(3))
+    p = acx.Ctcs(n=n, dx=0.5, dy=0.4, dz=0.6, dt=1e-3, stencil=stencil, src=(1, 2, 3), rcv=(0, 0, 0)).c_struct()
+    print(f"[case] ctcs result off alignment n={n} stencil={stencil}", flush=True)
+    out = []
+    for off in (0, 1):
+        new = torch.empty(N + off, dtype=torch.float64, device="cuda")[off:]
+        ptr = [ctypes.c_void_p(t.data_ptr()) for t in (old, cur, new, C)]
+        acx._check(acx.lib().acx_ctcs_update_f64(ctypes.byref(p), *ptr, 3, None, acx._stream()))
+        out.append(new)
+    assert torch.equal(*out)

@@ -104,3 +104,20 @@ int main()
     CHECK(ens_wide({64, 64, 64, 16384, 16384, 4}) && !ens_wide({64, 64, 64, 16384, 16383, 4}), "any problem of a batch");
 }
 """)
+
+
+def test_leapfrog_routes(run_host):
+    """What each kernel form asks of sizes and alignment, and no more: the march
+    that copies POLD, P and C stores 8 bytes at a time."""
+    run_host("""
+int main()
+{
+    CHECK(ctcs_route(100, 100, 100, 0x1000, 0x2000) == CTCS_PAIRS, "small and aligned");
+    CHECK(ctcs_route(256, 256, 256, 0x1000, 0x2000) == CTCS_DMA, "large and aligned");
+    CHECK(ctcs_route(256, 256, 256, 0x1000, 0x2008) == CTCS_DMA, "PNEW off alignment, large");
+    CHECK(ctcs_route(100, 100, 100, 0x1000, 0x2008) == CTCS_DMA, "PNEW off alignment, small");
+    CHECK(ctcs_route(256, 256, 256, 0x1008, 0x2000) == CTCS_MARCH, "POLD, P or C off alignment");
+    CHECK(ctcs_route(255, 256, 256, 0, 0) == CTCS_MARCH && ctcs_route(101, 100, 100, 0, 0) == CTCS_MARCH, "odd rows");
+    CHECK(ctcs_route(256, 256, 1, 0, 0) == CTCS_CELLS && ctcs_route(256, 1, 1, 0, 0) == CTCS_CELLS, "2D, 1D");
+}
+""")
