@@ -363,8 +363,12 @@ class Ctcs:
 
 
 def ctcs_run(p, nt, stream=None):
-    """UpdatePressure loop of wave.c:109-121 on the GPU; returns the receiver trace."""
+    """UpdatePressure loop of wave.c:109-121 on the GPU; returns the receiver trace
+    (empty for nt <= 0)."""
     torch = _torch()
+    nt = len(range(nt))
+    if nt == 0:
+        return []
     n = (p.n[2], p.n[1], p.n[0])
     st = stream if stream is not None else torch.cuda.current_stream()
     with torch.cuda.stream(st):

@@ -196,3 +196,13 @@ def test_only_the_result_off_alignment(n, stencil, acx, torch_gpu):
         acx._check(acx.lib().acx_ctcs_update_f64(ctypes.byref(p), *ptr, 3, None, acx._stream()))
         out.append(new)
     assert torch.equal(*out)
+
+
+def test_run_of_no_steps(acx, torch_gpu):
+    print("[case] ctcs_run without steps", flush=True)
+    p = acx.Ctcs(n=(24, 20, 18), src=(12, 10, 9), rcv=(15, 13, 12), dt=0.0005)
+    assert acx.ctcs_run(p, 0) == [] and acx.ctcs_run(p, -3) == []
+    with pytest.raises(TypeError):
+        acx.ctcs_run(p, 2.5)
+    st = torch_gpu.cuda.Stream()
+    assert acx.ctcs_run(p, 40) == acx.ctcs_run(p, 40, stream=st) and len(acx.ctcs_run(p, 3)) == 3
