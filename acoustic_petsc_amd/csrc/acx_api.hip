@@ -29,42 +29,6 @@ int env_int(const char *name, int dflt)
     return (s && *s) ? atoi(s) : dflt;
 }
 
-// Automatic z-chunk of a 2.5D march.  A launch runs in ceil(workgroups /
-// slots) rounds (slots = CUs, or places for workgroups), each about as long
-// as one workgroup's march of zc planes plus a fixed start of `start` planes'
-// worth (z-halo planes, prologue); of the even divisions of the planes the one
-// that minimises rounds x (zc + start) is taken, the longer march on a tie.
-// Against a fixed list of 8 .. 128 planes: a walled FP64 step at 150 x 131 x
-// 90 225 -> 151 us (32 planes left 135 workgroups on 256 CUs, 18 planes 225),
-// a 32^3 WAVE2 step 34 -> 21 us (8 planes: 8 workgroups; 1 plane: 64), the
-// FP32 step at 384^3 2.57 -> 2.50 ms (77 planes instead of 128); the same
-// chunk as before at 256^3.
-// pair > 0: a slot holds two workgroups, which then take `pair` times as long
-// as one alone.
-int auto_zc(int ntx, int nty, int nz, int slots, int start, double *cost_out, double pair)
-{
-    int best = nz, prev = 0;
-    double best_cost = -1.0;
-    for (int k = 1; k <= nz; ++k) {
-        const int z = (nz + k - 1) / k;
-        if (z == prev) continue;
-        prev = z;
-        const long long wg = (long long)ntx * nty * ((nz + z - 1) / z);
-        double rounds = (double)((wg + slots - 1) / slots);
-        if (pair > 0.0) {
-            const long long full = wg / (2LL * slots), rest = wg - full * 2 * slots;
-            rounds = (double)full * pair + (rest == 0 ? 0.0 : rest <= slots ? 1.0 : pair);
-        }
-        const double cost = rounds * (z + start);
-        if (best_cost < 0 || cost < best_cost) {
-            best_cost = cost;
-            best = z;
-        }
-    }
-    if (cost_out) *cost_out = best_cost;
-    return best;
-}
-
 // CUs of the current device (cached per device).
 int device_cus()
 {

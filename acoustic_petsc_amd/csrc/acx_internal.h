@@ -65,9 +65,7 @@ constexpr size_t sel_buffer_bytes(size_t tiles) { return sel_list_offset(tiles) 
 int launch_cweno_tilemask(const CwArgs &a, const uint8_t *flags, uint8_t *mask, hipStream_t s);
 
 int set_error(int code, const char *fmt, ...);
-// z-chunk of a 2.5D march from the round model (acx_api.hip) and its cost in
-// planes; CUs of the current device
-int auto_zc(int ntx, int nty, int nz, int slots, int start, double *cost = nullptr, double pair = 0.0);
+// CUs of the current device
 int device_cus();
 // integer tuning knob from the environment (dflt when unset or empty)
 int env_int(const char *name, int dflt);

@@ -12,6 +12,7 @@ CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))),
 PROLOGUE = """
 #include <cstdio>
 #include <cstdlib>
+#include <initializer_list>
 #include "acx_plan.h"
 using namespace acx;
 #define CHECK(c, ...) do { if (!(c)) { std::printf(__VA_ARGS__); std::printf("\\n"); std::exit(1); } } while (0)
@@ -121,3 +122,46 @@ int main()
     CHECK(ctcs_route(256, 256, 1, 0, 0) == CTCS_CELLS && ctcs_route(256, 1, 1, 0, 0) == CTCS_CELLS, "2D, 1D");
 }
 """)
+
+
+def test_z_chunk_is_the_best_even_division(run_host):
+    """The chunk of the round model against all even divisions of the planes, and
+    its cost on an axis of two thousand million planes (a launch's host time)."""
+    run_host("""
+static int all_divisions(int ntx, int nty, int nz, int slots, int start, double *cost, double pair)
+{
+    int best = nz, prev = 0;
+    double best_cost = -1.0;
+    for (int k = 1; k <= nz; ++k) {
+        const int z = (nz + k - 1) / k;
+        if (z == prev) continue;
+        prev = z;
+        const long long wg = (long long)ntx * nty * ((nz + z - 1) / z);
+        double rounds = (double)((wg + slots - 1) / slots);
+        if (pair > 0.0) {
+            const long long full = wg / (2LL * slots), rest = wg - full * 2 * slots;
+            rounds = (double)full * pair + (rest == 0 ? 0.0 : rest <= slots ? 1.0 : pair);
+        }
+        const double c = rounds * (z + start);
+        if (best_cost < 0 || c < best_cost) best_cost = c, best = z;
+    }
+    *cost = best_cost;
+    return best;
+}
+
+int main()
+{
+    for (int nz = 1; nz <= 520; nz += nz < 130 ? 1 : 13)
+        for (int ntx : {1, 2, 5, 9, 12, 65})
+            for (int nty : {1, 3, 16, 26})
+                for (int slots : {256, 512, 1024})
+                    for (int start : {4, 10})
+                        for (double pair : {0.0, 1.5}) {
+                            double a, b;
+                            const int z = auto_zc(ntx, nty, nz, slots, start, &a, pair);
+                            const int w = all_divisions(ntx, nty, nz, slots, start, &b, pair);
+                            CHECK(z == w && a == b, "%d planes, %d x %d tiles, %d slots: %d (%g), best %d (%g)", nz, ntx, nty, slots, z, a, w, b);
+                        }
+    CHECK(auto_zc(1, 1, 2000000000, 256, 10) == 7812500, "a long axis");
+}
+""", timeout=10)
