@@ -226,16 +226,8 @@ static int ens_step(acx_ensemble *e, double dt, hipStream_t s)
     return ACX_OK;
 }
 
-extern "C" {
-
-int acx_ensemble_num_configs(void) { return ENS_NCONFIG; }
-
-int acx_ensemble_create(int nprob, const int32_t *n, double h, acx_ensemble **out)
+static int ens_make(acx_ensemble *e, int nprob, const int32_t *n, double h)
 {
-    if (nprob < 1 || nprob > ENS_MAXP || !n || !out || !(h > 0)) return set_error(ACX_EINVAL, "ensemble: bad arguments");
-    for (int i = 0; i < 3 * nprob; ++i)
-        if (n[i] < 4) return set_error(ACX_EINVAL, "ensemble: at least 4 cells per axis");
-    acx_ensemble *e = new acx_ensemble();
     e->nprob = nprob;
     e->h = h;
     e->dims.assign(n, n + 3 * nprob);
@@ -283,6 +275,26 @@ int acx_ensemble_create(int nprob, const int32_t *n, double h, acx_ensemble **ou
         rc = hip_check(hipMalloc(&e->d_tables, at), "ensemble alloc");
         e->config = ens_default_config(e);
         rc = rc ? rc : ens_layout(e, e->config);
+    }
+    return rc;
+}
+
+extern "C" {
+
+int acx_ensemble_num_configs(void) { return ENS_NCONFIG; }
+
+int acx_ensemble_create(int nprob, const int32_t *n, double h, acx_ensemble **out)
+{
+    if (nprob < 1 || nprob > ENS_MAXP || !n || !out || !(h > 0)) return set_error(ACX_EINVAL, "ensemble: bad arguments");
+    for (int i = 0; i < 3 * nprob; ++i)
+        if (n[i] < 4) return set_error(ACX_EINVAL, "ensemble: at least 4 cells per axis");
+    acx_ensemble *e = nullptr;
+    int rc;
+    try {
+        e = new acx_ensemble();
+        rc = ens_make(e, nprob, n, h);
+    } catch (const std::exception &x) {
+        rc = set_error(ACX_EHIP, "ensemble: %s", x.what());
     }
     if (rc) {
         acx_ensemble_destroy(e);
