@@ -74,3 +74,21 @@ def test_more_threads_than_scratch_slots(acx, torch_gpu):
     for t in ts:
         t.join()
     assert not bad, bad[:3]
+
+
+@pytest.mark.parametrize("nvar, comp", [(1, -1), (1, 0), (3, 1), (4, -1)])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_reductions_of_nothing(nvar, comp, offset, acx, torch_gpu):
+    """No cells, with a pointer to a buffer that has some: sums and maxima of 0."""
+    torch = torch_gpu
+    import ctypes
+    X = torch.full((64,), 7.0, dtype=torch.float64, device="cuda")[offset:]
+    out = (ctypes.c_double * 2)(3.0, 3.0)
+    ptr = lambda t: ctypes.c_void_p(t.data_ptr())  # noqa: E731
+    print(f"[case] norms of no cells nvar={nvar} comp={comp} offset={offset}", flush=True)
+    acx._check(acx.lib().acx_norms_f64(ptr(X), 0, nvar, comp, out, acx._stream()))
+    assert tuple(out) == (0.0, 0.0)
+    f = X.to(torch.float32)
+    out = (ctypes.c_double * 2)(3.0, 3.0)
+    acx._check(acx.lib().acx_diff_f32c_f64(ptr(f), None, ptr(X), 0, out, acx._stream()))
+    assert tuple(out) == (0.0, 0.0)
