@@ -68,3 +68,30 @@ def test_unflagged_component_ignores_diagonal_neighbours(acx, torch_gpu, clean):
     z, y, x = np.nonzero(bad)
     dist = np.abs(x - 16) + np.abs(y - 8) + np.minimum(np.abs(z - 4), 8 - np.abs(z - 4))
     assert bad.any() and dist.max() <= 12
+
+
+@pytest.mark.parametrize("bc", [(0, 0, 0), (0, 3, 0)])
+@pytest.mark.parametrize("n", [(96, 14, 8), (93, 15, 9), (90, 29, 17), (96, 13, 7)])
+def test_flagged_slab_is_not_the_linear_scheme(n, bc, acx, torch_gpu):
+    """A jump inside the compared part of the flagged slab and one inside the
+    unflagged part: the schemes differ there by far more than either tolerance,
+    and each part takes its own."""
+    torch = torch_gpu
+    grid = acx.Grid(n=n, h=1.0 / 96, bc=bc, gamma_hi=0.85, gamma_lo=0.85)
+    rng = np.random.default_rng(8)
+    x = np.arange(n[0])[None, None, :, None]
+    U = np.where((x // 24) % 2 == 0, 1.0, 0.1) + 0.01 * rng.standard_normal(grid.shape())
+    U = torch.from_numpy(U).cuda()
+    dt = acx.cfl_dt(grid, 0.4)
+    fl = torch.zeros((n[2], n[1], n[0]), dtype=torch.uint8, device="cuda")
+    fl[:, :, :48] = 15
+    print(f"[case] jumps in and out of the flagged slab n={n} bc={bc}", flush=True)
+    s = acx.CompensatedState(grid, U)
+    s.step(dt, flags=fl.reshape(-1))
+    got = s.value64().cpu().numpy()
+    cw = _step64(acx, torch, n, (0.85, 0.85), bc, U, dt)
+    lin = _step64(acx, torch, n, (1.0, 0.0), bc, U, dt)
+    for part, want, other in ((slice(12, 36), cw, lin), (slice(60, 76), lin, cw)):
+        assert rel_l2(other[:, :, part], want[:, :, part]) > 1e-4
+        assert rel_l2(got[:, :, part], want[:, :, part]) <= 1e-7
+        assert rel_l2(got[:, :, part], other[:, :, part]) > 1e-5
