@@ -16,10 +16,10 @@ template <typename T> struct Axis3 { T c1[3], c2[3], c3[3]; };
 // 1/t in FP64: hardware reciprocal estimate refined by one Newton step.
 // Measured on gfx950 over 2^20 seeded t in [1e-50, 2e50]: the estimate alone
 // has |r t - 1| up to 4.6e-8 (2^-24.4), one step brings it to 2.2e-15
-// (2^-48.7), which puts the nonlinear weights within about 20 units in the
-// last place: far inside the 1e-12 agreement with the FP64 reference
-// scheme.  A second step (full precision) cost 2 % of the FP64 nonlinear
-// step.
+// (2^-48.7), which puts the weights within about 20 units in the last place.
+// Enough for what cweno_weights serves in FP64, the training labels, which
+// compare the weights' deviation with a threshold; the stage kernels take
+// rcp64_full.
 __device__ __forceinline__ double rcp64(double t)
 {
     double r = __builtin_amdgcn_rcp(t);

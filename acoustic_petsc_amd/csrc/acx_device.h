@@ -50,8 +50,6 @@ __device__ __forceinline__ int xcd_logical_tile(int id, int nb)
     return xcd * base + (xcd < rem ? xcd : rem) + slot;
 }
 
-template <typename T> struct Vec2 { T a, b; };
-
 // AoS cell access (4 components: p,u,v,w; or 2 components: u,v)
 template <typename T, int NV> struct Cell { T v[NV]; };
 
@@ -201,11 +199,6 @@ template <typename T>
 __device__ __forceinline__ T stencil_B7(T m3, T m2, T m1, T q0, T p1, T p2, T p3)
 {
     return (p3 + m3) - T(6) * (p2 + m2) + T(15) * (p1 + m1) - T(20) * q0;
-}
-template <typename T>
-__device__ __forceinline__ T stencil_L7(T m3, T m2, T m1, T q0, T p1, T p2, T p3)
-{
-    return T(2) * (p2 + m2) - (p3 + m3) + T(49) * (p1 + m1) - T(100) * q0;
 }
 
 // Error-free sum of two floats (Knuth's TwoSum): s + e == a + b exactly.

@@ -137,6 +137,7 @@ __device__ __forceinline__ void linear_tile32(const LinArgs &p, int x0, int y0, 
     auto load = [](const float *plane_base, Off o) {
         return load_cell<float, NV>(reinterpret_cast<const float *>(reinterpret_cast<const char *>(plane_base) + o), 0);
     };
+    // (load_cell_nt: nontemporal for the 16-byte cells of ACOUSTIC4 alone)
     auto load_lo = [&](size_t cell) { return STREAM ? load_cell_nt<float, NV>(LO, cell) : load_cell<float, NV>(LO, cell); };
     // the plane loaded next, its offset and its ghost sign
     int zi = 0;
@@ -588,10 +589,11 @@ __device__ __forceinline__ void store_cell_buf(double *row, unsigned bytes, unsi
     }
 }
 
-// MEM_CACHED: results and base states may stay in the caches, for fields small
-// enough that the next stage finds them there; MEM_STREAM: nontemporal; MEM_WIDE:
-// the same for rows of 2 GB or longer (a store descriptor for each of the two
-// rows).
+// MEM_CACHED: results may stay in the caches, for fields small enough that the
+// next stage finds them there; MEM_STREAM: nontemporal results; MEM_WIDE: the
+// same for rows of 2 GB or longer (a store descriptor for each of the two rows).
+// Base states are read through the caches in every mode (streaming is for
+// WAVE2 only here, whose 16-byte cells load_cell_nt reads the same way).
 enum { MEM_CACHED = 0, MEM_STREAM = 1, MEM_WIDE = 2 };
 
 template <int SYS, int EPI, bool WALLS, int MEM, int ROWS>
@@ -646,8 +648,7 @@ __device__ __forceinline__ void linear_tile64(const LinArgs &p, int x0, int y0, 
         return load_cell<double, NV>(reinterpret_cast<const double *>(reinterpret_cast<const char *>(plane_base) + o), 0);
     };
     auto load_u0 = [&](int z) {
-        const double *u = reinterpret_cast<const double *>(reinterpret_cast<const char *>(U0 + (size_t)z * plane * NV) + colb);
-        return STREAM ? load_cell_nt<double, NV>(u, 0) : load_cell<double, NV>(u, 0);
+        return load(U0 + (size_t)z * plane * NV, colb);
     };
     // the plane loaded next, its offset and its ghost sign
     int zi = 0;
