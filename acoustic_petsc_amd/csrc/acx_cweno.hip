@@ -68,9 +68,9 @@ struct CwLds {
 // tile's march is what counts: one block per CU without spills (2 waves per
 // SIMD) beat two blocks per CU with 60 spilled registers (1.076 against 1.146
 // ms for a steep pulse's step at 256^3, 232 marked tiles, one round either
-// way).  A 256^3 patch is 55 (first stage) to 59 us (last), of which the vector
-// instructions of ten planes issue for about 43; it was 84 us with
-// cweno_weights + cweno_combine, a linear branch of its own and each epilogue
+// way).  A 256^3 patch is 56 (first stage) to 61 us (last; 54 and 58 before the
+// branch for the smooth side of a jump, when the vector instructions of ten
+// planes issued for about 43); it was 84 us with cweno_weights + cweno_combine, a linear branch of its own and each epilogue
 // load waited for at its place, and 57 to 61 with two barriers a plane.  The full-grid kernel keeps the registers too.
 template <bool SEL>
 struct CwWaves {
@@ -353,8 +353,8 @@ k_cweno(CwArgs p)
 // thread on 32 x 16 columns): the new arithmetic in the old kernel 5.38 ms (256
 // VGPRs, 2 waves per SIMD, 24 spilled); two components per thread on 32 x 16
 // columns 8.07 ms (128 VGPRs for 4 waves per SIMD, 35 spilled: the scratch
-// traffic leaves the L1); on 32 x 12 columns 4.64 ms (3 waves per SIMD, 167
-// VGPRs, no spills), although the smaller tile recomputes more of its ring
+// traffic leaves the L1); on 32 x 12 columns 4.64 ms (3 waves per SIMD, 150 to
+// 167 VGPRs, no spills), although the smaller tile recomputes more of its ring
 // (outputs are 78 % of the reconstructed columns instead of 82 %).  The WAVE2
 // RHS at 70 x 45 x 61 with walls: 31.8 -> 22.0 us.
 //

@@ -262,7 +262,7 @@ __device__ __forceinline__ T cweno_axes(const T (&s)[33], const CwArgs &p, Axis3
 //   2 c2 = C + w c + n1 a - ...,  2 c1 = 2 e2 + C + w c - n1 a + ...
 // (on the other side A - w a - n2 c and 2 e3 - A + w a - n2 c).  Above 1/1024 the
 // indicators are within a factor of 23 and the jump within 5 of the background.
-// The branch costs 2 % of a 256^3 ACOUSTIC4 step (4.36 -> 4.45 ms), where one
+// The branch costs 2 to 3 % of a 256^3 ACOUSTIC4 step (4.36 -> 4.46 ms), where one
 // wavefront in a hundred takes it, and 3 to 13 % of a 70 x 45 x 61 WAVE2 right-hand
 // side (12.3 -> 12.6 .. 13.8 us), whose odd walls are jumps in a third of the
 // wavefronts; these sums without a branch would add 7 % of the instructions
